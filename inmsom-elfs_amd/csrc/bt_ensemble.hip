@@ -434,6 +434,7 @@ FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase
     p.fry_in = mb.fry;
     p.hup_c = mb.hup_c;
     p.hvp_c = mb.hvp_c;
+    fast_constants(p);
     return p;
 }
 

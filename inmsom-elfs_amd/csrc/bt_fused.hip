@@ -535,6 +535,7 @@ static FusedParams make_params(inmsom_bt_ctx *c, FusedAlloc *a, int b, double ta
     p.nu = c->nu;
     p.ffs = (double)c->g.ffs;
     p.d = c->metric0;
+    fast_constants(p);
     return p;
 }
 

@@ -3,6 +3,8 @@
 // The algorithm and its modes are described at the top of bt_fused.hip.
 #pragma once
 
+#include <type_traits>
+
 #include "bt_internal.h"
 
 namespace ibt {
@@ -28,10 +30,20 @@ struct FusedParams {
     // sub-cycling: substep `sub` of `nsub` (tau = tau_inner = outer tau / nsub)
     int sub, nsub;
     double dn;             // dfloat(nstep)
+    double inv_d, g_d, nu_d, ffs_rho0;  // 1 / d, g / d, nu / d, ffs / rho0
     void *frx, *fry;       // forcing frozen over the substeps of one call (stencil type), written
     const void *frx_in, *fry_in;  // the same, read (a separate buffer when a launch forms new forcing)
     double *hup_c, *hvp_c; // filtered U/V depths carried between substeps (FP64_EXACT only)
 };
+
+// the quotients of the fast modes' constants, once on the host
+inline void fast_constants(FusedParams &p)
+{
+    p.inv_d = 1.0 / p.d;
+    p.g_d = p.g / p.d;
+    p.nu_d = p.nu / p.d;
+    p.ffs_rho0 = p.ffs / p.rho0;
+}
 
 // Lane shifts by DPP (no LDS traffic).  wave_shl:1 gives lane L the value
 // of lane L+1 (column m+1), wave_shr:1 the value of lane L-1 (column m-1);
@@ -515,6 +527,226 @@ struct Stage {
     }
 };
 
+// Explicit multiply-adds of the fast modes: the library is compiled without
+// contraction, so the march, the pair march, the pipeline and the tiles give
+// the same bits whatever the compiler does around them.
+__device__ __forceinline__ double fmad(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fmad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// a / b for a layer depth b (about 1 .. 10^4, far from the limits of the
+// format, so nothing is scaled): the hardware's reciprocal (FP32: 1 ulp;
+// FP64: about 2^-26, two Newton steps) and one correction of the quotient
+// by its exact remainder, within 0.51 ulp of the quotient.
+__device__ __forceinline__ float depth_div(float a, float b)
+{
+    const float r = __builtin_amdgcn_rcpf(b);
+    const float q = a * r;
+    return fmad(fmad(-b, q, a), r, q);
+}
+__device__ __forceinline__ double depth_div(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fmad(fmad(-b, r, 1.0), r, r);
+    r = fmad(fmad(-b, r, 1.0), r, r);
+    const double q = a * r;
+    return fmad(fmad(-b, q, a), r, q);
+}
+
+// Scalars of the fast modes' formulas.
+template <typename R>
+struct FastConst {
+    R id, two_tau, gid, nuid, ffr, cb, eb, two_tau_id;
+    double cts;
+    __device__ FastConst(const FusedParams &p)
+        : id(R(p.inv_d)), two_tau(R(2.0 * p.tau)), gid(R(p.g_d)), nuid(R(p.nu_d)), ffr(R(p.ffs_rho0)), cb(R(p.cb)),
+          eb(R(p.eb)), two_tau_id(R(2.0 * p.tau * p.inv_d)), cts(0.5 * p.ts / p.dn)
+    {
+    }
+};
+
+// The fast modes' formulas (FP64, FP32) on a uniform grid, point by point.
+// The reference's algebra with the metric factored out, every flux and
+// product formed once where its two neighbours share it: the fluxes u hu and
+// v hv, the advective fluxes, the viscous products nu hq str_t and nu hh
+// str_s (the mean viscosity of four wet cells is nu), the Coriolis products.
+namespace fast {
+// 1 / (number of wet T cells) of a U or V point: both wet (`both`) or one
+template <typename R>
+__device__ __forceinline__ R depth2(R wsum, bool any, bool both)
+{
+    return any ? (both ? R(0.5) * wsum : wsum) : R(0);
+}
+// the same on an H point with cnt wet T cells of 4
+template <typename R>
+__device__ __forceinline__ R depth4(R wsum, int cnt)
+{
+    const R rs = cnt == 4 ? R(0.25) : cnt == 3 ? R(1.0 / 3.0) : cnt == 2 ? R(0.5) : R(1);
+    return cnt > 0 ? rs * wsum : R(0);
+}
+// continuity (Function/vel_ssh.f90:487-499): the increment of the surface
+template <typename R>
+__device__ __forceinline__ double surface(const FastConst<R> &c, double sp, R wf, R fu, R ful, R fv, R fvs)
+{
+    const R div = (fu - ful) + (fv - fvs);
+    return sp + double(fmad(-c.two_tau_id, div, c.two_tau * (wf * c.ffr)));
+}
+// bottom drag rate (Function/fluxes.f90:226-250)
+template <typename R>
+__device__ __forceinline__ R drag(const FastConst<R> &c, R hq, R fu, R ful, R fv, R fvs)
+{
+    const R rh = depth_div(R(0.5), hq);
+    const R ut = (fu + ful) * rh, vt = (fv + fvs) * rh;
+    return c.cb * sqrt(fmad(ut, ut, fmad(vt, vt, c.eb)));
+}
+// new velocity of a U (V) point (Function/vel_ssh.f90:531-573): rhs the
+// frozen forcing, ds the surface difference, h, hp, hn the depth at levels
+// n, n-1, n+1, adv the sum of the four advective fluxes (times -4), dif the
+// viscous differences, rds the two Rayleigh coefficients, cor the signed sum
+// of the two Coriolis products, up the filtered velocity
+template <typename R>
+__device__ __forceinline__ R momentum(const FastConst<R> &c, R rhs, R ds, R h, R hp, R hn, R adv, R dif, R rds,
+                                      R cor, R up)
+{
+    R F = fmad(c.id, fmad(R(-0.25), adv, dif), rhs);
+    F = fmad(-c.gid * ds, h, F);
+    F = fmad(R(-0.5) * rds * up, h, F);
+    F = fmad(R(0.25), cor, F);
+    return depth_div(fmad(c.two_tau, F, up * hp), hn);
+}
+// Robert-Asselin filter (Function/vel_ssh.f90:588-612), in FP64
+__device__ __forceinline__ double filter(double cts, double now, double next, double prev)
+{
+    return fmad(cts, fmad(-2.0, now, next) + prev, now);
+}
+}  // namespace fast
+
+// One leap-frog substep marching down the rows of one strip in the fast
+// modes.  Cells outside the array enter with mask 0, and every use of a
+// neighbour is selected by a mask, so their values do not matter (they need
+// not be zeroed).  Lane shifts stand outside the selections: inside an arm
+// they would read lanes that the arm's branch has switched off.
+template <typename R, bool FORM>
+struct FastStage {
+    const FusedParams &p;
+    const FastConst<R> c;
+    const bool inx, inx1;
+
+    R u_0 = 0, v_0 = 0, s_0 = 0, s_p1 = 0, H_p1 = 0, rd_0 = 0;
+    double up_0 = 0, vp_0 = 0, sp_0 = 0;
+    int mb_0 = 0, mb_p1 = 0;
+    int lus_0 = 0;                         // wet T cells of (m, n), (m+1, n)
+    bool lv_0 = false;                     // (m, n) and (m, n+1) both wet
+    R w_p1 = 0, a_0 = 0;                   // wet depth of row n+1; sum over m, m+1 of row n
+    R wp_0 = 0, wn_0 = 0;                  // wet depth of the filtered and the new level
+    R hu_0 = 0, hup_0 = 0, hv_0 = 0, hun_0 = 0;
+    R fu_0 = 0, fv_0 = 0;                  // u hu, v hv
+    R fyU_m1 = 0, fyV_m1 = 0;              // advective fluxes through the south faces
+    R Q_m1 = 0, Fc_m1 = 0, P_0 = 0, bf_0 = 0;
+    double sn_0 = 0;
+
+    __device__ FastStage(const FusedParams &pp, int m)
+        : p(pp), c(pp), inx(m >= 3 && m <= pp.nx - 2), inx1(m >= 2 && m <= pp.nx - 1)
+    {
+    }
+
+    __device__ __forceinline__ void row(int n, const StageIn<R> &q, bool produce, StageOut<R> &o)
+    {
+        const int k1 = n + 1;
+        const bool tw = (mb_p1 & MB_LU) && inx && (k1 >= 3 && k1 <= p.ny - 2);
+        const bool hw = (mb_0 & MB_LUU) && inx && (n >= 3 && n <= p.ny - 2);
+        const int l1 = mb_p1 & MB_LU;
+        const int lus_p1 = l1 + dpp_from_right(l1);
+        const bool lu1 = l1 != 0, lv_p1 = (mb_p1 & q.mb2 & MB_LU) != 0;
+        const bool llu1 = mb_p1 & MB_LLU, lu2 = lus_p1 == 2;
+        const bool llv0 = mb_0 & MB_LLV, lcv0 = mb_0 & MB_LCV;
+        const R up1 = R(q.up1), vp1 = R(q.vp1), up0 = R(up_0), vp0 = R(vp_0);
+
+        // ---- depths (hh_init / hh_update, Function/depth.f90)
+        const R w_p2 = (q.mb2 & MB_LU) ? q.H2 + q.s2 : R(0);
+        const R a_p1 = w_p1 + xr(w_p1);
+        const R hu_p1 = fast::depth2(a_p1, llu1, lu2);
+        const R hv_p1 = fast::depth2(w_p1 + w_p2, bool(mb_p1 & MB_LLV), lv_p1);
+        const R hh_0 = fast::depth4(a_0 + a_p1, (mb_0 & MB_LUH) ? lus_0 + lus_p1 : 0);
+        const R wp_p1 = lu1 ? H_p1 + R(q.sp1) : R(0);
+        const R hup_p1 = fast::depth2(wp_p1 + xr(wp_p1), llu1, lu2);
+
+        // ---- T point of row n+1: continuity, new depths, tension, drag
+        const R fu_p1 = q.u1 * hu_p1, fv_p1 = q.v1 * hv_p1;
+        const R ful = xl(fu_p1);
+        const double sn_p1 = tw ? fast::surface(c, q.sp1, q.wf1, fu_p1, ful, fv_p1, fv_0) : 0.0;
+        const R wn_p1 = lu1 ? H_p1 + R(sn_p1) : R(0);
+        const R hun_p1 = fast::depth2(wn_p1 + xr(wn_p1), llu1, lu2);
+        const R tens = (up1 - xl(up1)) - (vp1 - vp0);
+        const R P_p1 = tw ? c.nuid * w_p1 * tens : R(0);
+        R bf_p1 = R(0);
+        if constexpr (FORM) bf_p1 = tw ? fast::drag(c, w_p1, fu_p1, ful, fv_p1, fv_0) : R(0);
+
+        // ---- H point of row n: shear, Coriolis (the metric vorticity is
+        // identically zero for uniform metrics, Function/vel_ssh.f90:35-37)
+        const R shear = (up1 - up0) + (xr(vp0) - vp0);
+        const R Q_0 = hw ? c.nuid * hh_0 * shear : R(0);
+        const R vsum = xr(v_0) + v_0, usum = q.u1 + u_0;
+        const R cor = q.f0 * hh_0;
+        const R Fc_0 = cor * vsum;
+        const R fvs = fv_0 + xr(fv_0);
+        const R fyU_0 = (mb_0 & MB_LUU) ? fvs * usum : R(0);
+        const R fyV_0 = (fv_0 + fv_p1) * (v_0 + q.v1);
+
+        // ---- outputs of row n
+        if (produce) {
+            R rhs_u = q.fx0, rhs_v = q.fy0;
+            if constexpr (FORM) {
+                // the RHS of Control/dyncall.f90:114-126, frozen over the call's substeps
+                rhs_u = fmad(R(-0.5) * (bf_0 + xr(bf_0)), up0, q.sx0);
+                rhs_v = fmad(R(-0.5) * (bf_0 + bf_p1), vp0, q.sy0);
+            }
+            o.rhs_u = rhs_u;
+            o.rhs_v = rhs_v;
+            const R hvp_0 = fast::depth2(wp_0 + wp_p1, llv0, lv_0);
+            const R hvn_0 = fast::depth2(wn_0 + wn_p1, llv0, lv_0);
+            const R fx = (fu_0 + xr(fu_0)) * (u_0 + xr(u_0));
+            const R gx = (fu_0 + fu_p1) * vsum;
+            const R Gc = cor * usum;
+            R un = fast::momentum(c, rhs_u, xr(s_0) - s_0, hu_0, hup_0, hun_0, (fx - xl(fx)) + (fyU_0 - fyU_m1),
+                                  (xr(P_0) - P_0) + (Q_0 - Q_m1), rd_0 + xr(rd_0), Fc_0 + Fc_m1, up0);
+            R vn = fast::momentum(c, rhs_v, s_p1 - s_0, hv_0, hvp_0, hvn_0, (gx - xl(gx)) + (fyV_0 - fyV_m1),
+                                  (P_0 - P_p1) + (Q_0 - xl(Q_0)), rd_0 + q.rd1, -(Gc + xl(Gc)), vp0);
+            const bool iny = (n >= 3 && n <= p.ny - 2);
+            un = ((mb_0 & MB_LCU) && inx && iny) ? un : R(0);
+            vn = (lcv0 && inx && iny) ? vn : R(0);
+
+            // time-level shift with the Robert-Asselin filter
+            const bool sh = inx1 && n >= 2 && n <= p.ny - 1;
+            const bool su = (mb_0 & MB_LCU) && sh, sv = lcv0 && sh, ss = (mb_0 & MB_LU) && sh;
+            o.s = ss ? R(sn_0) : s_0;
+            o.u = su ? un : u_0;
+            o.v = sv ? vn : v_0;
+            o.sp = ss ? fast::filter(c.cts, double(s_0), sn_0, sp_0) : sp_0;
+            o.up = su ? fast::filter(c.cts, double(u_0), double(un), up_0) : up_0;
+            o.vp = sv ? fast::filter(c.cts, double(v_0), double(vn), vp_0) : vp_0;
+        }
+
+        // ---- advance the window one row
+        u_0 = q.u1; v_0 = q.v1;
+        s_0 = s_p1; s_p1 = q.s2;
+        H_p1 = q.H2;
+        up_0 = q.up1; vp_0 = q.vp1; sp_0 = q.sp1; rd_0 = q.rd1;
+        mb_0 = mb_p1; mb_p1 = q.mb2;
+        lus_0 = lus_p1; lv_0 = lv_p1;
+        w_p1 = w_p2; a_0 = a_p1;
+        wp_0 = wp_p1; wn_0 = wn_p1;
+        hu_0 = hu_p1; hup_0 = hup_p1; hv_0 = hv_p1; hun_0 = hun_p1;
+        fu_0 = fu_p1; fv_0 = fv_p1;
+        fyU_m1 = fyU_0; fyV_m1 = fyV_0;
+        Q_m1 = Q_0; Fc_m1 = Fc_0; P_0 = P_p1; bf_0 = bf_p1;
+        sn_0 = sn_p1;
+    }
+};
+
+// the march of a mode
+template <typename R, bool EXACT, bool FORM>
+using MarchStage = std::conditional_t<EXACT, Stage<R, true, FORM>, FastStage<R, FORM>>;
+
 // Loads of one iteration n of a strip (issued one iteration ahead of their
 // use: measured on MI355X at 2048 x 1536, two iterations ahead runs 5 %
 // slower in FP32 and halves FP64's occupancy).
@@ -572,9 +804,28 @@ struct Loader {
         q.sy = tab(p.row_sy, n);
         q.wf = tab(p.row_wf, n + 1);
     }
-    // the prefetched values of iteration n, zeroed outside the array
+    // the prefetched values of iteration n, zeroed outside the array (in the
+    // fast modes the mask alone: FastStage selects by it)
     __device__ __forceinline__ void take(int n, StageIn<R> &in) const
     {
+        if constexpr (!EXACT) {
+            in.s2 = q.s;
+            in.H2 = q.H;
+            in.mb2 = rowok(n + 2) ? q.mb : 0;
+            in.u1 = q.u;
+            in.v1 = q.v;
+            in.up1 = q.up;
+            in.vp1 = q.vp;
+            in.sp1 = q.sp;
+            in.rd1 = q.rd;
+            in.fx0 = q.fx;
+            in.fy0 = q.fy;
+            in.f0 = R(q.f);
+            in.sx0 = R(q.sx);
+            in.sy0 = R(q.sy);
+            in.wf1 = R(q.wf);
+            return;
+        }
         const int k1 = n + 1;
         in.s2 = rowok(n + 2) ? q.s : R(0);
         in.H2 = rowok(n + 2) ? q.H : R(0);
@@ -623,7 +874,7 @@ __device__ __forceinline__ void fused_chunk(const FusedParams &p, int chunk_id, 
     const int r0 = chunk_id * p.chunk + 1;
     const int r1 = min(r0 + p.chunk, p.ny + 1);
 
-    Stage<R, EXACT, FORM> st(p, m);
+    MarchStage<R, EXACT, FORM> st(p, m);
     Loader<R, EXACT, !FORM> ld(p, m);
     StageIn<R> in;
     StageOut<R> o;
@@ -670,8 +921,8 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
     const int r1 = min(r0 + p.chunk, p.ny + 1);
     const int subB = p.sub + 1;
 
-    Stage<R, EXACT, AFORM> A(p, m);
-    Stage<R, EXACT, false> B(p, m);
+    MarchStage<R, EXACT, AFORM> A(p, m);
+    MarchStage<R, EXACT, false> B(p, m);
     Loader<R, EXACT, !AFORM> ld(p, m);
     StageIn<R> ia, ib;
     StageOut<R> oa, ob;
@@ -694,7 +945,7 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
         A.row(n, ia, keepA, oa);
         // A's row n as the 2-launch sequence would have stored it: zero
         // outside the array, as B's loads would read it
-        const bool okn = ld.rowok(n) && keepA;
+        const bool okn = !EXACT || (ld.rowok(n) && keepA);
         if (runB) {
             ib.s2 = okn ? oa.s : R(0);
             ib.H2 = H_d2;
@@ -734,8 +985,8 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
         H_d2 = H_d1; H_d1 = ia.H2;
         mb_d2 = mb_d1; mb_d1 = ia.mb2;
         rd_d2 = rd_d1; rd_d1 = ia.rd1;
-        fx_d2 = fx_d1; fx_d1 = keepA ? oa.rhs_u : R(0);
-        fy_d2 = fy_d1; fy_d1 = keepA ? oa.rhs_v : R(0);
+        fx_d2 = fx_d1; fx_d1 = (!EXACT || keepA) ? oa.rhs_u : R(0);
+        fy_d2 = fy_d1; fy_d1 = (!EXACT || keepA) ? oa.rhs_v : R(0);
         if constexpr (EXACT) {
             hu_d2 = hu_d1; hu_d1 = keepA ? oa.hu : 0.0;
             hv_d2 = hv_d1; hv_d1 = keepA ? oa.hv : 0.0;
@@ -805,7 +1056,7 @@ __device__ __forceinline__ void fused_pipe_stage(const FusedParams &p, int chunk
     const int valid_from = n0 + 3 + 2 * w;  // first row of valid results
     const bool last = (w == K - 1);
 
-    Stage<R, false, FORM> st(p, m);
+    FastStage<R, FORM> st(p, m);
     Loader<R, false, !FORM> ld(p, m);
     StageIn<R> in;
     StageOut<R> o;
@@ -837,26 +1088,25 @@ __device__ __forceinline__ void fused_pipe_stage(const FusedParams &p, int chunk
             in.fx0 = c.fx[lane];
             in.fy0 = c.fy[lane];
             in.hupc0 = in.hvpc0 = 0.0;
-            in.f0 = (r >= 1 && r <= p.ny) ? R(ld.tab(p.row_f, r)) : R(0);
+            in.f0 = R(ld.tab(p.row_f, r));
             in.sx0 = R(ld.tab(p.row_sx, r));
             in.sy0 = R(ld.tab(p.row_sy, r));
-            in.wf1 = (r + 1 >= 1 && r + 1 <= p.ny) ? R(ld.tab(p.row_wf, r + 1)) : R(0);
+            in.wf1 = R(ld.tab(p.row_wf, r + 1));
         }
         const bool keep = last ? (r >= r0) : (r >= valid_from);
         st.row(r, in, keep, o);
         if (!last) {
-            // row r for stage w + 1, zero outside the array or before the
-            // results are valid (what its loads would have read there)
+            // row r for stage w + 1 (outside the array its mask is 0; what is
+            // handed over before the results are valid reaches no output)
             PipeSlot<R> &q = ring[w][n & (PIPE_SLOTS - 1)];
-            const bool ok = ld.rowok(r) && keep;
-            q.s[lane] = ok ? o.s : R(0);
-            q.u[lane] = ok ? o.u : R(0);
-            q.v[lane] = ok ? o.v : R(0);
-            q.sp[lane] = ok ? o.sp : 0.0;
-            q.up[lane] = ok ? o.up : 0.0;
-            q.vp[lane] = ok ? o.vp : 0.0;
-            q.fx[lane] = keep ? o.rhs_u : R(0);
-            q.fy[lane] = keep ? o.rhs_v : R(0);
+            q.s[lane] = o.s;
+            q.u[lane] = o.u;
+            q.v[lane] = o.v;
+            q.sp[lane] = o.sp;
+            q.up[lane] = o.up;
+            q.vp[lane] = o.vp;
+            q.fx[lane] = o.rhs_u;
+            q.fy[lane] = o.rhs_v;
             q.H[lane] = H_d2;
             q.rd[lane] = rd_d1;
             q.mb[lane] = (uint8_t)mb_d2;
