@@ -93,6 +93,31 @@ __global__ void __launch_bounds__(2 * WAVE)
     }
 }
 
+// Substeps sub .. sub + ksub - 1 of every tile of an ensemble of small members
+// (fused_tile), one block per tile.
+template <typename R>
+__global__ void __launch_bounds__(WAVE * TILE_MAX_ROWS)
+    k_tile_batch(const FusedParams *__restrict__ table, const int *__restrict__ item_member,
+                 const int *__restrict__ item_local, int total, int per_xcd, int ksub, double tau_inner, int sub,
+                 int nsub)
+{
+    extern __shared__ __attribute__((aligned(16))) char tile_shared[];
+    const int b = blockIdx.x;
+    const int t = (b % NXCD) * per_xcd + (b / NXCD);
+    if (t >= total) return;  // the whole block
+    FusedParams p = table[item_member[t]];
+    p.tau = tau_inner;
+    p.sub = sub;
+    p.nsub = nsub;
+    p.dn = (double)nsub;
+    const int local = item_local[t];
+    const int ty = local / p.strips, tx = local - ty * p.strips;
+    // a call's first launch forms the forcing and saves it when the call
+    // goes on (no later launch writes it: no block reads what another writes)
+    const bool save = sub == 1 && ksub < nsub;
+    fused_tile<R>(p, ty, tx, ksub, sub == 1 ? 1 : 0, save, reinterpret_cast<R *>(tile_shared));
+}
+
 template <class R>
 __global__ void k_member_range(int nx, int ny, const uint8_t *mb, const R *ssh, const R *u, const R *v,
                                unsigned long long *bad)
@@ -162,7 +187,7 @@ struct inmsom_bt_ens {
     int subs = 0;           // substeps per launch: 0 = by mode, 1, 2
     int pipe = 0;           // substep pairs as a two-wave pipeline: 0 = by mode, 1 = off, 2 = on
     int built_chunk = -1;
-    bool built_two = false;
+    bool built_two = false, built_tile = false;
     unsigned table_gen = 0;  // bumped whenever build_tables replaces table[] / item_*
     int phase = 0;          // buffer set holding the current state
     // graph of one outer step for (tau, nstep, start phase)
@@ -209,22 +234,58 @@ int fail(const std::string &m, int code)
 
 size_t esz(int mode) { return mode == INMSOM_BT_FP32 ? 4 : 8; }
 
+long long all_cells(const inmsom_bt_ens *e)
+{
+    long long cells = 0;
+    for (const EnsMember &m : e->mem) cells += (long long)m.n;
+    return cells;
+}
+
+// the tiles: the fast modes below TWO_SUBSTEP_CELLS cells in all, unless the
+// caller chose a launch shape
+bool tile_path(const inmsom_bt_ens *e)
+{
+    return e->mode != INMSOM_BT_FP64_EXACT && e->subs == 0 && e->pipe == 0 && e->chunk == 0 && e->waves_per_xcd == 0 &&
+           all_cells(e) < TWO_SUBSTEP_CELLS;
+}
+
 // two substeps per launch: as set, or by mode and size as for one basin
 // (not in FP64_EXACT, whose IEEE divides make it compute-bound, nor below
-// TWO_SUBSTEP_CELLS cells in all, where the launches are latency-bound)
+// TWO_SUBSTEP_CELLS cells in all with a launch shape of the caller's)
 bool two_per_launch(const inmsom_bt_ens *e)
 {
     if (e->subs > 0) return e->subs == 2;
-    long long cells = 0;
-    for (const EnsMember &m : e->mem) cells += (long long)m.n;
-    return e->mode != INMSOM_BT_FP64_EXACT && cells >= TWO_SUBSTEP_CELLS;
+    return e->mode != INMSOM_BT_FP64_EXACT && (tile_path(e) || all_cells(e) >= TWO_SUBSTEP_CELLS);
 }
 
 // substep pairs as a two-wave pipeline (FP64 and FP32): as set, or by default
 bool pipe_pairs(const inmsom_bt_ens *e)
 {
-    if (e->mode == INMSOM_BT_FP64_EXACT || !two_per_launch(e)) return false;
+    if (e->mode == INMSOM_BT_FP64_EXACT || !two_per_launch(e) || tile_path(e)) return false;
     return e->pipe != 1;
+}
+
+const void *tile_kernel(const inmsom_bt_ens *e)
+{
+    return e->mode == INMSOM_BT_FP64 ? (const void *)&k_tile_batch<double> : (const void *)&k_tile_batch<float>;
+}
+
+size_t tile_lds_bytes(const inmsom_bt_ens *e, int nr)
+{
+    return e->mode == INMSOM_BT_FP64 ? tile_lds<double>(nr) : tile_lds<float>(nr);
+}
+
+// rows a tile writes, of the tile_rows rule over all members
+int tile_chunk(const inmsom_bt_ens *e)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device) != hipSuccess || cus < 1)
+        cus = 256;
+    return tile_out_rows(tile_rows(cus, [&](int rows) {
+        long long t = 0;
+        for (const EnsMember &m : e->mem) t += (long long)((m.nx + SW2 - 1) / SW2) * ((m.ny + rows - 1) / rows);
+        return t;
+    }));
 }
 
 // the batch kernel for (mode, two substeps, forming substep)
@@ -389,13 +450,13 @@ int build_member(inmsom_bt_ens *e, const inmsom_bt_grid *gr, const inmsom_bt_for
     return INMSOM_BT_OK;
 }
 
-FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase, int chunk, bool two)
+FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase, int chunk, bool two, bool tile)
 {
     FusedParams p{};
     p.nx = mb.nx;
     p.ny = mb.ny;
     const int sw = two ? SW2 : SW;
-    p.strips = (mb.nx + 2 + sw - 1) / sw;
+    p.strips = (mb.nx + (tile ? 0 : 2) + sw - 1) / sw;
     p.chunk = chunk;
     p.nchunks = (mb.ny + chunk - 1) / chunk;
     p.total = p.strips * p.nchunks;
@@ -441,11 +502,15 @@ FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase
 // (Re)builds the descriptor tables and the work list for a launch shape.
 int build_tables(inmsom_bt_ens *e, int chunk, bool two)
 {
-    if (e->built_chunk == chunk && e->built_two == two) return INMSOM_BT_OK;
+    const bool tile = tile_path(e);
+    if (e->built_chunk == chunk && e->built_two == two && e->built_tile == tile) return INMSOM_BT_OK;
+    if (tile)
+        EHC(hipFuncSetAttribute(tile_kernel(e), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)tile_lds_bytes(e, TILE_MAX_ROWS)));
     std::vector<FusedParams> t[2];
     std::vector<int> im, il;
     for (size_t k = 0; k < e->mem.size(); ++k) {
-        for (int ph = 0; ph < 2; ++ph) t[ph].push_back(member_params(e, e->mem[k], ph, chunk, two));
+        for (int ph = 0; ph < 2; ++ph) t[ph].push_back(member_params(e, e->mem[k], ph, chunk, two, tile));
         const int items = t[0].back().total;
         e->mem[k].items = items;
         for (int i = 0; i < items; ++i) {
@@ -467,6 +532,7 @@ int build_tables(inmsom_bt_ens *e, int chunk, bool two)
     e->total = (int)im.size();
     e->built_chunk = chunk;
     e->built_two = two;
+    e->built_tile = tile;
     ++e->table_gen;
     return INMSOM_BT_OK;
 }
@@ -484,6 +550,19 @@ void launch_batch(inmsom_bt_ens *e, int phase, double tau_inner, int sub, int ns
     hipLaunchKernel(k, grid, blk, args, 0, e->stream);
 }
 
+// Substeps sub .. sub + ksub - 1 on the tiles of the work list.
+void launch_tiles(inmsom_bt_ens *e, int phase, double tau_inner, int sub, int nsub, int ksub)
+{
+    int per_xcd = (e->total + NXCD - 1) / NXCD;
+    const int nr = e->built_chunk + 3 * TILE_K;
+    const FusedParams *tb = e->table[phase];
+    const int *im = e->item_member, *il = e->item_local;
+    int total = e->total;
+    void *args[] = {&tb, &im, &il, &total, &per_xcd, &ksub, &tau_inner, &sub, &nsub};
+    hipLaunchKernel(tile_kernel(e), dim3((unsigned)(per_xcd * NXCD)), dim3((unsigned)(WAVE * nr)), args,
+                    tile_lds_bytes(e, nr), e->stream);
+}
+
 // launches per outer step: substep pairs, and an odd last substep alone
 int launches_per_step(int nstep, bool two) { return two ? nstep / 2 + nstep % 2 : nstep; }
 
@@ -493,7 +572,10 @@ void outer_step(inmsom_bt_ens *e, int phase, double tau, int nstep, int wpx, boo
 {
     for (int sub = 1; sub <= nstep;) {
         const bool pair = two && sub + 1 <= nstep;
-        launch_batch(e, phase, tau / (double)nstep, sub, nstep, wpx, pair);
+        if (e->built_tile)
+            launch_tiles(e, phase, tau / (double)nstep, sub, nstep, pair ? 2 : 1);
+        else
+            launch_batch(e, phase, tau / (double)nstep, sub, nstep, wpx, pair);
         phase = 1 - phase;
         sub += pair ? 2 : 1;
     }
@@ -606,6 +688,11 @@ int ensure_graphs(inmsom_bt_ens *e, double tau, int nstep, int chunk, int wpx, b
 void launch_shape(const inmsom_bt_ens *e, bool *two, int *wpx, int *chunk)
 {
     *two = two_per_launch(e);
+    if (tile_path(e)) {
+        *wpx = 0;
+        *chunk = tile_chunk(e);
+        return;
+    }
     *wpx = e->waves_per_xcd > 0 ? e->waves_per_xcd : default_waves(e, *two);
     *chunk = e->chunk > 0 ? e->chunk : default_chunk(e, *two, *wpx);
 }

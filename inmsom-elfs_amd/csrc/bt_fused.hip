@@ -26,6 +26,7 @@
 //   FP32        FP64's algebra in FP32 for the level-n fields and all
 //               stencils; the filtered (n-1) level, the continuity
 //               accumulation and the Robert-Asselin filter stay FP64.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -70,6 +71,19 @@ __global__ void __launch_bounds__(WAVE * K) k_fused_pipe(FusedParams p, int form
     if (t >= p.total) return;  // the whole workgroup
     const int chunk_id = t / p.strips, strip = t - chunk_id * p.strips;
     fused_pipe<R, K>(p, chunk_id, strip, form_mask, save_forcing != 0, ring);
+}
+
+// ksub <= TILE_K substeps of a small grid per launch, one block per tile
+// (fused_tile).
+template <typename R>
+__global__ void __launch_bounds__(WAVE * TILE_MAX_ROWS) k_fused_tile(FusedParams p, int ksub, int form_mask, int save_forcing)
+{
+    extern __shared__ __attribute__((aligned(16))) char tile_shared[];
+    const int b = blockIdx.x;
+    const int t = (b % NXCD) * p.per_xcd + (b / NXCD);
+    if (t >= p.total) return;  // the whole block
+    const int ty = t / p.strips, tx = t - ty * p.strips;
+    fused_tile<R>(p, ty, tx, ksub, form_mask, save_forcing != 0, reinterpret_cast<R *>(tile_shared));
 }
 
 // -------------------------------------------------------------- helpers
@@ -417,6 +431,13 @@ int fused_flush(inmsom_bt_ctx *c)
     return INMSOM_BT_OK;
 }
 
+// Whether the next launches take the tiles: the fast modes on grids below
+// TWO_SUBSTEP_CELLS cells, unless the caller chose a launch shape.
+static bool tile_path(const inmsom_bt_ctx *c, int mode)
+{
+    return mode != INMSOM_BT_FP64_EXACT && c->n < TWO_SUBSTEP_CELLS && c->subs_per_launch == 0 && c->pipe_k == 0 && c->chunk == 0;
+}
+
 // Parameters of a launch that reads buffer set b and writes 1 - b: substep
 // `sub`, or substeps sub and sub + 1 when `two`.
 // Substeps per launch: as set, or automatically two in FP64 and FP32 on
@@ -428,6 +449,7 @@ int fused_flush(inmsom_bt_ctx *c)
 int subs_per_launch(const inmsom_bt_ctx *c, int mode)
 {
     if (c->subs_per_launch > 0) return c->subs_per_launch;
+    if (tile_path(c, mode)) return TILE_K;
     return mode != INMSOM_BT_FP64_EXACT && c->n >= TWO_SUBSTEP_CELLS ? 2 : 1;
 }
 
@@ -559,6 +581,41 @@ static void launch_pipe(inmsom_bt_ctx *c, const FusedParams &p, int mode, int K,
     (void)hipLaunchKernel(pipe_kernel(mode, K), grid, blk, args, 0, c->stream);
 }
 
+static const void *tile_kernel(int mode)
+{
+    return mode == INMSOM_BT_FP64 ? (const void *)&k_fused_tile<double> : (const void *)&k_fused_tile<float>;
+}
+
+static size_t tile_lds_bytes(int mode, int nr)
+{
+    return mode == INMSOM_BT_FP64 ? tile_lds<double>(nr) : tile_lds<float>(nr);
+}
+
+// rows per tile of a grid; the kernel's LDS limit raised to what they need
+static int tile_shape(inmsom_bt_ctx *c, int mode)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1)
+        cus = 256;
+    const long long strips = (c->nx + pipe_width(TILE_K) - 1) / pipe_width(TILE_K);
+    const int nr = tile_rows(cus, [&](int rows) { return strips * ((c->ny + rows - 1) / rows); });
+    (void)hipFuncSetAttribute(tile_kernel(mode), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)tile_lds_bytes(mode, nr));
+    return nr;
+}
+
+static void launch_tile(inmsom_bt_ctx *c, FusedParams &p, int mode, int nr, int ksub, int form_mask, int save_forcing)
+{
+    p.strips = (c->nx + pipe_width(TILE_K) - 1) / pipe_width(TILE_K);
+    p.chunk = tile_out_rows(nr);
+    p.nchunks = (c->ny + p.chunk - 1) / p.chunk;
+    p.total = p.strips * p.nchunks;
+    p.per_xcd = (p.total + NXCD - 1) / NXCD;
+    void *args[] = {&p, &ksub, &form_mask, &save_forcing};
+    (void)hipLaunchKernel(tile_kernel(mode), dim3((unsigned)(p.per_xcd * NXCD)), dim3((unsigned)(WAVE * nr)), args,
+                          tile_lds_bytes(mode, nr), c->stream);
+}
+
 static void launch(inmsom_bt_ctx *c, const FusedParams &p, int mode, bool two)
 {
     dim3 grid((unsigned)(p.per_xcd * NXCD)), blk(WAVE);
@@ -606,20 +663,22 @@ int fused_run(inmsom_bt_ctx *c, double tau, int nstep, int nsteps, int mode, dou
     // launch's first substep.  The K-wave pipeline may span outer steps;
     // one- and two-substep launches stay within one.
     const int K = pipe_stages(c, mode);
+    const bool tiles = tile_path(c, mode);
+    const int tile_nr = tiles ? tile_shape(c, mode) : 0;
     const long long total = (long long)nsteps * nstep;
     for (long long g = 0; g < total;) {
         const int sub = (int)(g % nstep) + 1;
-        if (K >= 2 && g + K <= total) {
+        if (tiles || (K >= 2 && g + K <= total)) {
+            const int ks = tiles ? (int)std::min<long long>(TILE_K, total - g) : K;  // substeps of this launch
             FusedParams p = make_params(c, a, c->fz_cur, tau, nstep, sub, mode, false);
-            pipe_shape(c, mode, K, p);
             int form_mask = 0;
-            for (int w = 0; w < K; ++w)
+            for (int w = 0; w < ks; ++w)
                 if ((g + w) % nstep == 0) form_mask |= 1 << w;
-            // the last stage's call continues after this launch: its forcing is
-            // saved, into the other set when a stage of this launch formed it
+            // the last substep's call continues after this launch: its forcing is
+            // saved, into the other set when a substep of this launch formed it
             // (the current set may still be read by other work items' first
-            // stage); a launch that forms none leaves the current set as it is
-            int save = (int)((g + K - 1) % nstep) != nstep - 1;
+            // substep); a launch that forms none leaves the current set as it is
+            int save = (int)((g + ks - 1) % nstep) != nstep - 1;
             if (save && form_mask) {
                 p.frx = a->frc_cur ? a->frx : a->frx2;
                 p.fry = a->frc_cur ? a->fry : a->fry2;
@@ -627,8 +686,13 @@ int fused_run(inmsom_bt_ctx *c, double tau, int nstep, int nsteps, int mode, dou
             } else {
                 save = 0;
             }
-            launch_pipe(c, p, mode, K, form_mask, save);
-            g += K;
+            if (tiles) {
+                launch_tile(c, p, mode, tile_nr, ks, form_mask, save);
+            } else {
+                pipe_shape(c, mode, K, p);
+                launch_pipe(c, p, mode, K, form_mask, save);
+            }
+            g += ks;
         } else {
             const bool two = subs_per_launch(c, mode) == 2 && sub + 1 <= nstep;
             FusedParams p = make_params(c, a, c->fz_cur, tau, nstep, sub, mode, two);

@@ -13,9 +13,13 @@ constexpr int WAVE = 64;
 constexpr int SW = 60;   // output columns per wave, one substep per launch
 constexpr int SW2 = 58;  // output columns per wave, two substeps per launch
 constexpr int NXCD = 8;
-// cells (summed over an ensemble's members) from which the fused step runs
-// two substeps per launch by default
-constexpr long long TWO_SUBSTEP_CELLS = 1LL << 20;
+// cells (summed over an ensemble's members) from which the fused step's fast
+// modes run substep pairs as a two-wave pipeline by default, and below which
+// they run them on tiles (fused_tile).  Measured on MI355X, us per substep,
+// tiles / pipeline: 512 x 384 FP64 7.9 / 8.2, FP32 6.4 / 8.4; 640 x 512 FP64
+// 11.4 / 10.8, FP32 9.1 / 9.8; 768 x 640 FP64 15.3 / 13.5, FP32 12.2 / 10.1;
+// 1021 x 763 FP64 22.3 / 17.0, FP32 17.5 / 13.0.
+constexpr long long TWO_SUBSTEP_CELLS = 300000;
 
 struct FusedParams {
     int nx, ny, strips, chunk, nchunks, total, per_xcd;
@@ -1150,6 +1154,183 @@ __device__ __forceinline__ void fused_pipe(const FusedParams &p, int chunk_id, i
             fused_pipe_stage<R, K, false, true>(p, chunk_id, strip, w, save_forcing, ring);
         else
             fused_pipe_stage<R, K, false, false>(p, chunk_id, strip, w, save_forcing, ring);
+    }
+}
+
+// ------------------------------------------------------------------
+// Small grids: TILE_K substeps per launch on tiles of 64 x nr points, one
+// point per lane and one row per wave.  The march above gives a small grid
+// too few waves, each of which then walks its rows one after the other
+// (2 rows and 3 of warm-up at 256 x 256: 7 us a substep, most of it waiting);
+// here every point is its own lane, a substep is four short phases with the
+// row neighbours' values exchanged through LDS between them (the column
+// neighbours come by lane shifts), and the intermediate level stays in
+// registers.  A tile writes its columns TILE_K .. 63 - 2 TILE_K and rows
+// TILE_K .. nr - 1 - 2 TILE_K (a substep reaches one point west and south, two
+// east and north; the rim is computed by the tiles on both sides).  The
+// formulas and their order are FastStage's: the same bits.  Measured on
+// MI355X, us per substep, one launch of the march each / tiles: FP64 64 x 64
+// 6.1 / 3.1, 256 x 256 6.6 / 3.8, 512 x 384 9.3 / 7.9; FP32 5.9 / 2.9,
+// 6.4 / 3.4, 7.5 / 6.4.  What is left is the launch and the loads' latency
+// (about 3 us of a launch) and, from 256 x 256 on, the issue of the rim's
+// redundant points (38 % at 16 rows).
+constexpr int TILE_K = 2;
+constexpr int TILE_MAX_ROWS = 16;
+constexpr int TILE_ARRAYS = 12;
+constexpr int tile_out_rows(int nr) { return nr - 3 * TILE_K; }
+template <typename R>
+constexpr size_t tile_lds(int nr) { return (size_t)TILE_ARRAYS * nr * WAVE * sizeof(R); }
+
+// Rows per tile (8, 12 or 16) for a grid or ensemble: `tiles(out_rows)` tiles
+// on a chip of `cus` CUs, the fewest rows that the busiest CU works through.
+// Measured (FP64, us per substep with 8 / 12 / 16 rows): 128 x 128 3.2 / 3.7 /
+// 4.1, 256 x 256 5.5 / 3.8 / 4.3, 512 x 384 10.8 / 9.5 / 7.9.
+template <typename F>
+inline int tile_rows(long long cus, F tiles)
+{
+    int best = TILE_MAX_ROWS;
+    long long best_cost = -1;
+    for (int nr = TILE_MAX_ROWS; nr >= 8; nr -= 4) {
+        const long long rounds = (tiles(tile_out_rows(nr)) + cus - 1) / cus;
+        const long long cost = rounds * (nr + 4);  // 4: the phases' latency in rows' issue time
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = nr;
+        }
+    }
+    return best;
+}
+
+// One tile: substeps p.sub .. p.sub + ksub - 1 (ksub <= TILE_K).  form_mask bit
+// j: substep j of the launch is the first of its call; save_forcing: the last
+// one's call goes on after this launch.  Every wave of the block calls it.
+template <typename R>
+__device__ __forceinline__ void fused_tile(const FusedParams &p, int ty, int tx, int ksub, int form_mask,
+                                           bool save_forcing, R *lds)
+{
+    const int lane = threadIdx.x % WAVE, nr = blockDim.x / WAVE;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int m = tx * pipe_width(TILE_K) + lane - (TILE_K - 1);
+    const int n = ty * tile_out_rows(nr) + w - (TILE_K - 1);
+    const FastConst<R> c(p);
+    // array a of row r, this lane's column
+    auto at = [&](int a, int r) -> R & { return lds[(a * nr + r) * WAVE + lane]; };
+    const int wn = min(w + 1, nr - 1), ws = max(w - 1, 0);  // (the rim rows' neighbours reach no output)
+
+    const RowAddr ra{p.nx, p.ny, min(max(m, 1), p.nx)};
+    const bool colok = m >= 1 && m <= p.nx;
+    const size_t i0 = ra.at(n), i1 = ra.at(n + 1);
+    R u = static_cast<const R *>(p.u)[i0], v = static_cast<const R *>(p.v)[i0], s = static_cast<const R *>(p.s)[i0];
+    double up = p.up[i0], vp = p.vp[i0], sp = p.sp[i0];
+    const R H = static_cast<const R *>(p.H)[i0];
+    const R rd = static_cast<const R *>(p.rd)[i0], rd1 = static_cast<const R *>(p.rd)[i1];
+    int mb = p.mb[i0], mb1 = p.mb[i1];
+    R rhs_u = R(0), rhs_v = R(0);
+    if (!(form_mask & 1)) {
+        rhs_u = static_cast<const R *>(p.frx_in)[i0];
+        rhs_v = static_cast<const R *>(p.fry_in)[i0];
+    }
+    const int rc = min(max(n, 1), p.ny) - 1;
+    const R f0 = R(p.row_f[rc]), sx = R(p.row_sx[rc]), sy = R(p.row_sy[rc]), wf = R(p.row_wf[rc]);
+    if (!(colok && n >= 1 && n <= p.ny)) mb = 0;
+    if (!(colok && n + 1 >= 1 && n + 1 <= p.ny)) mb1 = 0;
+
+    const bool in = m >= 3 && m <= p.nx - 2 && n >= 3 && n <= p.ny - 2;
+    const bool sh = m >= 2 && m <= p.nx - 1 && n >= 2 && n <= p.ny - 1;
+    const int l0 = mb & MB_LU, l1 = mb1 & MB_LU;
+    const int lus0 = l0 + dpp_from_right(l0), lus1 = l1 + dpp_from_right(l1);
+    const bool lu = l0 != 0, lu2 = lus0 == 2, lv = (l0 & l1) != 0, llu = mb & MB_LLU, llv = mb & MB_LLV;
+    const bool tw = lu && in, luu = mb & MB_LUU, hw = luu && in, lcu = mb & MB_LCU, lcv = mb & MB_LCV;
+    const int cnt = (mb & MB_LUH) ? lus0 + lus1 : 0;
+    const R rdu = rd + xr(rd), rdv = rd + rd1;
+
+    for (int j = 0; j < ksub; ++j) {
+        const bool form = (form_mask >> j) & 1;
+        const R upr = R(up), vpr = R(vp);
+        const R w0 = lu ? H + s : R(0);
+        const R wp = lu ? H + R(sp) : R(0);
+        at(0, w) = w0;
+        at(1, w) = wp;
+        at(2, w) = s;
+        at(3, w) = u;
+        at(4, w) = v;
+        at(5, w) = upr;
+        at(6, w) = vpr;
+        __syncthreads();
+        // depths, fluxes, shear and Coriolis products
+        const R w1 = at(0, wn);
+        const R a0 = w0 + xr(w0), a1 = w1 + xr(w1);
+        const R hu = fast::depth2(a0, llu, lu2), hv = fast::depth2(w0 + w1, llv, lv);
+        const R hh = fast::depth4(a0 + a1, cnt);
+        const R hup = fast::depth2(wp + xr(wp), llu, lu2), hvp = fast::depth2(wp + at(1, wn), llv, lv);
+        const R ds_v = at(2, wn) - s, u1 = at(3, wn), v1 = at(4, wn), vs = at(4, ws), up1 = at(5, wn), vps = at(6, ws);
+        const R fu = u * hu, fv = v * hv;
+        const R shear = (up1 - upr) + (xr(vpr) - vpr);
+        const R Q = hw ? c.nuid * hh * shear : R(0);
+        const R vsum = xr(v) + v, usum = u1 + u;
+        const R cor = f0 * hh;
+        const R Fc = cor * vsum, Gc = cor * usum;
+        const R fvs = fv + xr(fv);
+        const R fyU = luu ? fvs * usum : R(0);
+        at(7, w) = fv;
+        at(8, w) = fu;
+        at(9, w) = Q;
+        at(10, w) = Fc;
+        at(11, w) = fyU;
+        __syncthreads();
+        // T point: continuity, new depth, tension, drag
+        const R fv_s = at(7, ws), fv_n = at(7, wn), ful = xl(fu);
+        const R Qs = at(9, ws), Fcs = at(10, ws), fyUs = at(11, ws);
+        const R fu1 = at(8, wn);
+        const double sn = tw ? fast::surface(c, sp, wf, fu, ful, fv, fv_s) : 0.0;
+        const R wnew = lu ? H + R(sn) : R(0);
+        const R tens = (upr - xl(upr)) - (vpr - vps);
+        const R P = tw ? c.nuid * w0 * tens : R(0);
+        R bf = R(0);
+        if (form) bf = tw ? fast::drag(c, w0, fu, ful, fv, fv_s) : R(0);
+        at(0, w) = wnew;
+        at(1, w) = P;
+        at(2, w) = bf;
+        __syncthreads();
+        // momentum and the time-level shift
+        const R bf1 = at(2, wn), P1 = at(1, wn);
+        if (form) {
+            rhs_u = fmad(R(-0.5) * (bf + xr(bf)), upr, sx);
+            rhs_v = fmad(R(-0.5) * (bf + bf1), vpr, sy);
+        }
+        const R hun = fast::depth2(wnew + xr(wnew), llu, lu2), hvn = fast::depth2(wnew + at(0, wn), llv, lv);
+        const R fx = (fu + xr(fu)) * (u + xr(u));
+        const R gx = (fu + fu1) * vsum;
+        const R fyV = (fv + fv_n) * (v + v1), fyVs = (fv_s + fv) * (vs + v);
+        R un = fast::momentum(c, rhs_u, xr(s) - s, hu, hup, hun, (fx - xl(fx)) + (fyU - fyUs), (xr(P) - P) + (Q - Qs),
+                              rdu, Fc + Fcs, upr);
+        R vn = fast::momentum(c, rhs_v, ds_v, hv, hvp, hvn, (gx - xl(gx)) + (fyV - fyVs), (P - P1) + (Q - xl(Q)), rdv,
+                              -(Gc + xl(Gc)), vpr);
+        un = (lcu && in) ? un : R(0);
+        vn = (lcv && in) ? vn : R(0);
+        const bool ss = lu && sh, su = lcu && sh, sv = lcv && sh;
+        sp = ss ? fast::filter(c.cts, double(s), sn, sp) : sp;
+        up = su ? fast::filter(c.cts, double(u), double(un), up) : up;
+        vp = sv ? fast::filter(c.cts, double(v), double(vn), vp) : vp;
+        s = ss ? R(sn) : s;
+        u = su ? un : u;
+        v = sv ? vn : v;
+        if (j + 1 < ksub) __syncthreads();  // the last reads of the arrays the next substep writes
+    }
+    if (colok && n >= 1 && n <= p.ny && lane >= TILE_K && lane <= WAVE - 1 - 2 * TILE_K && w >= TILE_K &&
+        w <= nr - 1 - 2 * TILE_K) {
+        const size_t io = (size_t)(n - 1) * p.nx + (m - 1);
+        if (save_forcing) {
+            static_cast<R *>(p.frx)[io] = rhs_u;
+            static_cast<R *>(p.fry)[io] = rhs_v;
+        }
+        // (cached: the grid is small and the next launch reads it)
+        static_cast<R *>(p.so)[io] = s;
+        static_cast<R *>(p.uo)[io] = u;
+        static_cast<R *>(p.vo)[io] = v;
+        p.spo[io] = sp;
+        p.upo[io] = up;
+        p.vpo[io] = vp;
     }
 }
 

@@ -1,0 +1,48 @@
+"""The tiles of the fast modes on small grids: bit for bit what the march
+gives (a launch shape of the caller's, here one row chunk, selects the march),
+over tile edges in both directions, odd substep counts and calls that span
+launches, for one basin and for an ensemble."""
+import pytest
+
+from _util import STATE, assert_bitwise
+from inmsom_bt import BarotropicModel, make_basin, randomize_state
+from inmsom_bt.ensemble import Ensemble
+
+pytestmark = pytest.mark.gpu
+
+
+def _basin(nxi, nyi, seed=3):
+    return randomize_state(make_basin(nxi, nyi, seed=seed, sigma=min(4.0, 0.2 * min(nxi, nyi))), seed + 1)
+
+
+# array sizes around the 58-column tiles and the 2-, 6- and 10-row ones; the
+# smallest; one just below the size at which the pipeline takes over
+@pytest.mark.parametrize("mode", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape,nstep,steps", [((8, 6), 2, 3), ((54, 30), 2, 3), ((55, 31), 3, 3), ((113, 37), 1, 5),
+                                               ((200, 91), 4, 2), ((271, 240), 5, 3), ((560, 520), 2, 2)])
+def test_tiles_equal_march(mode, shape, nstep, steps):
+    b = _basin(*shape)
+    print(f"tiles {mode} {shape} nstep={nstep}", flush=True)
+    out = []
+    for chunk in (0, 5):
+        with BarotropicModel(b) as m:
+            m.set_launch(chunk)
+            m.run(steps, mode, nstep=nstep, tau=5.0 * nstep)
+            m.run(1, mode, nstep=nstep, tau=5.0 * nstep)
+            out.append(m.get_state())
+    assert_bitwise(out[0], out[1], STATE, f"tiles vs march {mode} {shape} nstep={nstep}")
+
+
+@pytest.mark.parametrize("mode,nstep", [("fp32", 2), ("fp64", 3), ("fp32", 1)])
+def test_ensemble_tiles_equal_march(mode, nstep):
+    basins = [_basin(x, y, seed=9 + k) for k, (x, y) in enumerate(((40, 90), (130, 33), (61, 62), (9, 7)))]
+    print(f"ensemble tiles {mode} nstep={nstep}", flush=True)
+    out = []
+    for rows, graph in ((0, True), (0, False), (7, False)):
+        with Ensemble(basins, mode=mode) as ens:
+            ens.set_launch(rows, 0)
+            ens.run(9, nstep=nstep, tau=5.0 * nstep, graph=graph)
+            out.append([ens.get_state(k) for k in range(len(basins))])
+    for o in out[1:]:
+        for k in range(len(basins)):
+            assert_bitwise(o[k], out[0][k], STATE, f"member {k} {mode} nstep={nstep}")
