@@ -97,8 +97,8 @@ int inmsom_bt_finalize(inmsom_bt_ctx *ctx);
  * inmsom_bt_get_depths.
  * Path: one fused kernel launch per substep (bit for bit the reference)
  * when full_free_surface = 1, the grid is not periodic and the two halo
- * cells of every side are land (with ksw4 > 0 the biharmonic term of each
- * substep comes from two reference-order sweeps before its launch);
+ * cells of every side are land (with ksw4 > 0 the same launch forms the
+ * substep's biharmonic term);
  * otherwise one kernel per reference sweep (also bit for bit).
  * inmsom_bt_set_dropin_path chooses. */
 int inmsom_bt_barotropic_dynamics(inmsom_bt_ctx *ctx, double tau, int nstep, int ksw4,

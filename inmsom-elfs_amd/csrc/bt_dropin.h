@@ -8,9 +8,7 @@
 namespace ibt {
 
 // Whether the fused path can take a call with this ksw4 on this context's
-// grid (see bt_dropin.hip); *why says why not.  ksw4 > 0 is covered: the
-// biharmonic term comes from a pre-pass of reference-order kernels per
-// substep (lit_diff4_terms).
+// grid (see bt_dropin.hip); *why says why not.  ksw4 > 0 is covered.
 bool dropin_eligible(inmsom_bt_ctx *c, int ksw4, std::string *why);
 // One call of barotropic_dynamics (Function/vel_ssh.f90:379-679) on device
 // arrays: the state (u, up, v, vp, ssh, sshp) is replaced by the state

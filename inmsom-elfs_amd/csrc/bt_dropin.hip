@@ -27,12 +27,10 @@
 //
 // Eligible calls: full_free_surface = 1, no periodicity, and land on the
 // two halo cells of every side (the reference's loop bounds then coincide
-// with its masks).  Other calls take the stage-by-stage path.  With ksw4 >
-// 0 the biharmonic term uv_diff4 (vel_ssh.f90:187-317) of each substep is
-// formed before its launch by the reference-order kernels of the
-// stage-by-stage path from the substep's entering state (its two terms per
-// component, lit_diff4_terms) and added by the kernel to its uv_diff2 result
-// in the reference's order.
+// with its masks).  Other calls take the stage-by-stage path.
+// Two kernels: the march of k_dropin, and one point per lane on tiles
+// (k_dropin_tile) for small grids and for the biharmonic term uv_diff4
+// (ksw4 > 0, vel_ssh.f90:187-317), which it forms in the same launch.
 // Metrics: per cell (any grid), or per row when every metric and the
 // Coriolis parameter are uniform along x (Cartesian and longitude-latitude
 // grids): then they are read from row tables instead of 8 + 1 arrays.
@@ -52,19 +50,22 @@ struct DropinParams {
     const uint8_t *mb;
     const double *H, *rd, *mu, *wf, *rx, *ry;
     // dx, dy, dxt, dyt, dxh, dyh, dxb, dyb and rlh_s: per cell, or (ROWMET)
-    // per row, row n at [n - 1]
-    const double *met[9];
+    // per row, row n at [n - 1]; rows only: dy/dx, dx/dy, dxb/dyb, dyb/dxb
+    const double *met[13];
     const double *u, *v, *s, *up, *vp, *sp;  // state entering the substep
     double *uo, *vo, *so, *upo, *vpo, *spo;  // state after it (uo null: not written)
     double *cu, *cv, *cs, *cup, *cvp, *csp;  // copy of the entering state (cu null: none)
     double *hupc, *hvpc;                     // filtered U/V depths carried in place (substeps > 1 read)
     bool carry_out;                          // write the filtered U/V depths for the next substep
     double *acc[4];                          // ubrtr_i, vbrtr_i, ssh4gradx, ssh4grady, in place
-    const double *d4[4];                     // ksw4 > 0: uv_diff4's terms px, qx, py, qy of the substep
+    const double *mu4;                       // the biharmonic viscosity (ksw4 > 0)
     double g, rho0, ts, tau, ffs, dn, d4n;
 };
 
-// What iteration n consumes (zeroed outside the array): row n+2 of the
+// What iteration n consumes (outside the array the mask is 0 and the rest
+// whatever the clamped loads give: every use is selected by a mask, or
+// multiplied by a depth that is 0 there; zeroing the row metrics by lane would
+// hold them in vector registers): row n+2 of the
 // surface height, depth at rest, masks, dx, dy; row n+1 of the level-n and
 // filtered velocities and height, Rayleigh coefficient, viscosity, water
 // flux, dxt, dyh, dxh, dyt; row n of the Coriolis parameter, the caller's
@@ -74,7 +75,6 @@ struct DIn {
     int mb2;
     double u1, v1, up1, vp1, sp1, rd1, mu1, wf1, dxt1, dyh1, dxh1, dyt1;
     double f0, rx0, ry0, dxb0, dyb0, hupc0, hvpc0, a0, a1, a2, a3;
-    double d4[4];  // uv_diff4's terms of row n (D4)
 };
 
 // What one substep produces for row n.
@@ -86,10 +86,8 @@ struct DOut {
 
 // One substep marching down the rows of one strip.  Suffixes: m1 = row
 // n-1, 0 = row n, p1 = row n+1, p2 = row n+2.  FIRST: the call's first
-// substep (filtered depths from hh_init, accumulators start at zero).  D4:
-// the biharmonic viscosity is on (ksw4 > 0); its terms come precomputed
-// per cell and are added to the uv_diff2 result in the reference's order.
-template <bool FIRST, bool D4>
+// substep (filtered depths from hh_init, accumulators start at zero).
+template <bool FIRST>
 struct DStage {
     const DropinParams &p;
     const bool inx, inx1;
@@ -248,10 +246,8 @@ struct DStage {
             const double fx_m = xl(fx_p);
             const double radv = -(fx_p - fx_m + fyU_0 - fyU_m1) + (Cc_0 + Cc_m1) / 4.0;
             const double muh_m = (mu_0 + xr(mu_0) + mu_m1 + xr(mu_m1)) / 4.0;
-            double rdfx = (xr(P_0) - P_0) / dyh_0 +
-                          (dxb_0 * dxb_0 * muh_p * hh_0 * sts_0 - dxb_m1 * dxb_m1 * muh_m * hh_m1 * sts_m1) / dxt_0;
-            // uv_diff4 adds to uv_diff2's result (vel_ssh.f90:292-295)
-            if constexpr (D4) rdfx = rdfx + q.d4[0] + q.d4[1];
+            const double rdfx = (xr(P_0) - P_0) / dyh_0 +
+                                (dxb_0 * dxb_0 * muh_p * hh_0 * sts_0 - dxb_m1 * dxb_m1 * muh_m * hh_m1 * sts_m1) / dxt_0;
             const double bp = hun_0 * dxt_0 * dyh_0 / 2.0 / tau;
             const double bp0 = hupc * dxt_0 * dyh_0 / 2.0 / tau;
             const double slx = -G * (xr(s_0) - s_0) * dyh_0 * hu_0;
@@ -267,10 +263,8 @@ struct DStage {
             const double rady = -(fxV_p - fxV_m + fyV_0 - fyV_m1) - (D + xl(D)) / 4.0;
             const double muhv_m = (mu_0 + xl(mu_0) + mu_p1 + xl(mu_p1)) / 4.0;
             const double dybl = xl(dyb_0), hhl = xl(hh_0), stsl = xl(sts_0);
-            double rdfy = -(Px_p1 - Px_0) / dxh_0 +
-                          (dyb_0 * dyb_0 * muh_p * hh_0 * sts_0 - dybl * dybl * muhv_m * hhl * stsl) / dyt_0;
-            // (vel_ssh.f90:306-309)
-            if constexpr (D4) rdfy = rdfy - q.d4[2] + q.d4[3];
+            const double rdfy = -(Px_p1 - Px_0) / dxh_0 +
+                                (dyb_0 * dyb_0 * muh_p * hh_0 * sts_0 - dybl * dybl * muhv_m * hhl * stsl) / dyt_0;
             const double bq = hvn_0 * dyt_0 * dxh_0 / 2.0 / tau;
             const double bq0 = hvpc * dyt_0 * dxh_0 / 2.0 / tau;
             const double sly = -G * (s_p1 - s_0) * dxh_0 * hv_0;
@@ -373,7 +367,7 @@ struct DStage {
 };
 
 // Loads of one iteration, issued one iteration ahead of their use.
-template <bool FIRST, bool ROWMET, bool D4>
+template <bool FIRST, bool ROWMET>
 struct DLoader {
     const DropinParams &p;
     const RowAddr ra;
@@ -381,7 +375,6 @@ struct DLoader {
     struct Pre {
         double s, H, dx, dy, u, v, up, vp, sp, rd, mu, wf, dxt, dyh, dxh, dyt, f, rx, ry, dxb, dyb, hupc, hvpc;
         double a[4];
-        double d4[D4 ? 4 : 1];
         int mb;
     } q;
 
@@ -394,7 +387,7 @@ struct DLoader {
     __device__ __forceinline__ double met(int k, int row, size_t i) const
     {
         if constexpr (ROWMET)
-            return p.met[k][min(max(row, 1), p.ny) - 1];
+            return scalar_load(p.met[k] + min(max(row, 1), p.ny) - 1);
         else
             return p.met[k][i];
     }
@@ -423,8 +416,6 @@ struct DLoader {
         q.f = met(8, n, i0);
         q.rx = p.rx[i0];
         q.ry = p.ry[i0];
-        if constexpr (D4)
-            for (int k = 0; k < 4; ++k) q.d4[k] = p.d4[k][i0];
         if constexpr (!FIRST) {
             q.hupc = p.hupc[i0];
             q.hvpc = p.hvpc[i0];
@@ -433,31 +424,28 @@ struct DLoader {
     }
     __device__ __forceinline__ void take(int n, DIn &in) const
     {
-        const bool r2 = rowok(n + 2), r1 = rowok(n + 1), r0 = rowok(n);
-        in.s2 = r2 ? q.s : 0.0;
-        in.H2 = r2 ? q.H : 0.0;
-        in.mb2 = r2 ? q.mb : 0;
-        in.dx2 = r2 ? q.dx : 0.0;
-        in.dy2 = r2 ? q.dy : 0.0;
-        in.u1 = r1 ? q.u : 0.0;
-        in.v1 = r1 ? q.v : 0.0;
-        in.up1 = r1 ? q.up : 0.0;
-        in.vp1 = r1 ? q.vp : 0.0;
-        in.sp1 = r1 ? q.sp : 0.0;
-        in.rd1 = r1 ? q.rd : 0.0;
-        in.mu1 = r1 ? q.mu : 0.0;
-        in.wf1 = r1 ? q.wf : 0.0;
-        in.dxt1 = r1 ? q.dxt : 0.0;
-        in.dyh1 = r1 ? q.dyh : 0.0;
-        in.dxh1 = r1 ? q.dxh : 0.0;
-        in.dyt1 = r1 ? q.dyt : 0.0;
-        in.f0 = r0 ? q.f : 0.0;
-        in.rx0 = r0 ? q.rx : 0.0;
-        in.ry0 = r0 ? q.ry : 0.0;
-        in.dxb0 = r0 ? q.dxb : 0.0;
-        in.dyb0 = r0 ? q.dyb : 0.0;
-        if constexpr (D4)
-            for (int k = 0; k < 4; ++k) in.d4[k] = q.d4[k];
+        in.s2 = q.s;
+        in.H2 = q.H;
+        in.mb2 = rowok(n + 2) ? q.mb : 0;
+        in.dx2 = q.dx;
+        in.dy2 = q.dy;
+        in.u1 = q.u;
+        in.v1 = q.v;
+        in.up1 = q.up;
+        in.vp1 = q.vp;
+        in.sp1 = q.sp;
+        in.rd1 = q.rd;
+        in.mu1 = q.mu;
+        in.wf1 = q.wf;
+        in.dxt1 = q.dxt;
+        in.dyh1 = q.dyh;
+        in.dxh1 = q.dxh;
+        in.dyt1 = q.dyt;
+        in.f0 = q.f;
+        in.rx0 = q.rx;
+        in.ry0 = q.ry;
+        in.dxb0 = q.dxb;
+        in.dyb0 = q.dyb;
         if constexpr (!FIRST) {
             in.hupc0 = q.hupc;
             in.hvpc0 = q.hvpc;
@@ -471,13 +459,12 @@ struct DLoader {
     }
 };
 
-// Two waves per SIMD (the later substeps would take 256 VGPRs + 4 AGPRs,
-// one wave; bounded they spill 12 bytes per lane): at 2048 x 1536 on
-// MI355X a call of 4 launches takes 0.782 ms instead of 0.867.  With the
-// biharmonic terms (D4) one wave, whose registers hold what two waves
-// would spill.
-template <bool FIRST, bool ROWMET, bool D4>
-__global__ void __launch_bounds__(WAVE, D4 ? 1 : 2) k_dropin(DropinParams p)
+// Two waves per SIMD (with the row metrics by the scalar unit 211 VGPRs; from
+// vector loads, and zeroed by lane outside the array, they took 256 and spilled
+// 12 bytes per lane).  At 2048 x 1536 on MI355X a call of 4 launches takes
+// 0.768 ms (0.782); bound by FP64 issue, 44 IEEE divisions a point.
+template <bool FIRST, bool ROWMET>
+__global__ void __launch_bounds__(WAVE, 2) k_dropin(DropinParams p)
 {
     const int w = blockIdx.x;
     const int t = (w % NXCD) * p.per_xcd + (w / NXCD);
@@ -490,8 +477,8 @@ __global__ void __launch_bounds__(WAVE, D4 ? 1 : 2) k_dropin(DropinParams p)
     const int r0 = chunk_id * p.chunk + 1;
     const int r1 = min(r0 + p.chunk, p.ny + 1);
 
-    DStage<FIRST, D4> st(p, m);
-    DLoader<FIRST, ROWMET, D4> ld(p, m);
+    DStage<FIRST> st(p, m);
+    DLoader<FIRST, ROWMET> ld(p, m);
     DIn in;
     DOut o;
     ld.issue(r0 - 3);
@@ -533,19 +520,285 @@ __global__ void __launch_bounds__(WAVE, D4 ? 1 : 2) k_dropin(DropinParams p)
     }
 }
 
+// Small grids: one substep per launch on tiles of 64 x nr points, one point
+// per lane and one row per wave (the scheme of the fast modes' fused_tile).
+// A march gives a 289 x 163 grid 400 waves of 5 dependent rows, and the
+// biharmonic term two more launches; here a substep is four phases (six with
+// the biharmonic term, whose terms are formed in the same launch) with the
+// row neighbours' values exchanged through LDS, the column neighbours' by
+// lane shifts.  A substep reaches two points at most in every direction, so a
+// tile writes lanes 2..61 of rows 2..nr-3.  The expressions are DStage's and
+// the stage-by-stage path's (uv_diff4), operand for operand: the same bits.
+// FIRST of DStage is the launch argument here (it is uniform).
+// Measured on MI355X, us per substep on a longitude-latitude grid, march /
+// tiles: 285 x 159 14.5 / 7.7, 512 x 384 24.3 / 19.1, 640 x 512 31.3 / 29.4,
+// 900 x 700 48.7 / 54; with the biharmonic term (its march took two more
+// launches) 285 x 159 42 / 10.3, 2048 x 1536 408 / 369, and with metrics per
+// cell 657 / 434.  Bound by FP64 issue (about 30 IEEE divisions a point, 50
+// with the term) and, below 300 x 200, by the launch and the phases' latency.
+constexpr int DT_MAX_ROWS = 12;
+constexpr int DT_RIM = 4;  // rows of a tile that it does not write
+constexpr int DT_ARRAYS = 18;
+constexpr size_t dropin_tile_lds(int nr) { return (size_t)DT_ARRAYS * nr * WAVE * sizeof(double); }
+
+template <bool ROWMET, bool D4>
+__global__ void __launch_bounds__(WAVE * DT_MAX_ROWS) k_dropin_tile(DropinParams p, int first)
+{
+    extern __shared__ __attribute__((aligned(16))) double dt_shared[];
+    const int t = (blockIdx.x % NXCD) * p.per_xcd + (blockIdx.x / NXCD);
+    if (t >= p.total) return;  // the whole block
+    const int ty = t / p.strips, tx = t - ty * p.strips;
+    const int lane = threadIdx.x % WAVE, nr = blockDim.x / WAVE;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int m = tx * SW + lane - 1, n = ty * (nr - DT_RIM) + w - 1;
+    auto at = [&](int a, int r) -> double & { return dt_shared[(a * nr + r) * WAVE + lane]; };
+    const int rn = min(w + 1, nr - 1), rs = max(w - 1, 0);  // (the rim rows' neighbours reach no output)
+
+    const RowAddr ra{p.nx, p.ny, min(max(m, 1), p.nx)};
+    const bool colok = m >= 1 && m <= p.nx;
+    const size_t i0 = ra.at(n), i1 = ra.at(n + 1), is = ra.at(n - 1);
+    const double u = p.u[i0], v = p.v[i0], s = p.s[i0], up = p.up[i0], vp = p.vp[i0], sp = p.sp[i0];
+    const double H = p.H[i0], rd = p.rd[i0], rd1 = p.rd[i1], mu = p.mu[i0], mu1 = p.mu[i1], mus = p.mu[is];
+    const double wf = p.wf[i0], rx = p.rx[i0], ry = p.ry[i0];
+    double mu4 = 0.0, mu41 = 0.0, mu4s = 0.0;
+    if constexpr (D4) {
+        mu4 = p.mu4[i0];
+        mu41 = p.mu4[i1];
+        mu4s = p.mu4[is];
+    }
+    int mb = p.mb[i0], mb1 = p.mb[i1];
+    auto met = [&](int k, int row, size_t i) -> double {
+        if constexpr (ROWMET)
+            return p.met[k][min(max(row, 1), p.ny) - 1];
+        else
+            return p.met[k][i];
+    };
+    const double dx = met(0, n, i0), dy = met(1, n, i0), dxt = met(2, n, i0), dyt = met(3, n, i0);
+    const double dxh = met(4, n, i0), dyh = met(5, n, i0), dxb = met(6, n, i0), dyb = met(7, n, i0);
+    const double f = met(8, n, i0), dxbs = met(6, n - 1, is);
+    if (!(colok && n >= 1 && n <= p.ny)) mb = 0;
+    if (!(colok && n + 1 >= 1 && n + 1 <= p.ny)) mb1 = 0;
+    const bool writer = colok && n >= 1 && n <= p.ny && lane >= 2 && lane <= SW + 1 && w >= 2 && w <= nr - 3;
+    const size_t io = i0;  // a writer's point is in the array
+    double hupc = 0.0, hvpc = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    if (!first && writer) {
+        hupc = p.hupc[io];
+        hvpc = p.hvpc[io];
+        a0 = p.acc[0][io];
+        a1 = p.acc[1][io];
+        a2 = p.acc[2][io];
+        a3 = p.acc[3][io];
+    }
+
+    const bool in = m >= 3 && m <= p.nx - 2 && n >= 3 && n <= p.ny - 2;
+    const double lu0 = bitf<double>(mb, MB_LU), lu1 = bitf<double>(mb1, MB_LU);
+    const double lu0r = xr(lu0), lu1r = xr(lu1);
+    const bool tw = (mb & MB_LU) && in, hw = (mb & MB_LUU) && in;
+    const double G = p.g, tau = p.tau;
+
+    // ---- phase 1: depths' area weights and the stresses' quotients
+    const double hq = H + s;
+    const double w0 = hq * dx * dy * lu0;
+    const double wp0 = (H + sp) * dx * dy * lu0;
+    const double qa = up / dyh, qb = vp / dxh, qc = up / dxt, qe = vp / dyt;
+    const double hh_ = u * dxt, gg = v * dyt;
+    at(0, w) = w0;
+    at(1, w) = wp0;
+    at(2, w) = qb;
+    at(3, w) = qc;
+    at(4, w) = hh_;
+    at(5, w) = u;
+    at(6, w) = s;
+    at(7, w) = v;
+    __syncthreads();
+    // ---- phase 2: depths, fluxes, stresses, vorticity and Coriolis products
+    auto avg = [](double wsum, double slu, double m1, double m2) { return wsum / slu / m1 / m2; };
+    const double w1 = at(0, rn), w0r = xr(w0), w1r = xr(w1);
+    double hu = avg(w0 + w0r, lu0 + lu0r, dxt, dyh), hv = avg(w0 + w1, lu0 + lu1, dxh, dyt);
+    double hh = avg(w0 + w0r + w1 + w1r, lu0 + lu0r + lu1 + lu1r, dxb, dyb);
+    hu = (mb & MB_LLU) ? hu : 0.0;
+    hv = (mb & MB_LLV) ? hv : 0.0;
+    hh = (mb & MB_LUH) ? hh : 0.0;
+    if (first) {
+        const double wp1 = at(1, rn), wp0r = xr(wp0);
+        hupc = (mb & MB_LLU) ? avg(wp0 + wp0r, lu0 + lu0r, dxt, dyh) : 0.0;
+        hvpc = (mb & MB_LLV) ? avg(wp0 + wp1, lu0 + lu1, dxh, dyt) : 0.0;
+    }
+    const double qbs = at(2, rs), qc1 = at(3, rn), hh1_ = at(4, rn), u1 = at(5, rn), s1 = at(6, rn), v1 = at(7, rn);
+    const double vs = at(7, rs);
+    const double fu = u * hu * dyh, fv = v * hv * dxh;
+    const double A = u * dyh * hu, Bv = v * dxh * hv;
+    double yx, xy, bxy, byx;
+    if constexpr (ROWMET) {
+        yx = met(9, n, i0);
+        xy = met(10, n, i0);
+        bxy = met(11, n, i0);
+        byx = met(12, n, i0);
+    } else {
+        yx = dy / dx;
+        xy = dx / dy;
+        bxy = dxb / dyb;
+        byx = dyb / dxb;
+    }
+    const double st = yx * (qa - xl(qa)) - xy * (qb - qbs);
+    const double stt = tw ? st : 0.0;
+    const double P = dy * dy * mu * hq * stt, Px = dx * dx * mu * hq * stt;
+    const double ss = bxy * (qc1 - qc) + byx * (xr(qe) - qe);
+    const double v0r = xr(v);
+    const double vo_ = (xr(gg) - gg) - (hh1_ - hh_) - ((v0r - v) * dyb - (u1 - u) * dxb);
+    const double sts = hw ? ss : 0.0, vo = hw ? vo_ : 0.0;
+    const double fyU = (Bv + xr(Bv)) / 2.0 * (u1 + u) / 2.0 * bitf<double>(mb, MB_LUU);
+    const double vh = vo * hh;
+    const double Cc = vh * (v0r + v);
+    const double fhdd = f * hh * dxb * dyb;
+    const double Fc = fhdd * (v0r + v);
+    double P4 = 0.0, Px4 = 0.0;
+    at(8, w) = fv;
+    at(9, w) = Bv;
+    at(10, w) = A;
+    at(11, w) = Px;
+    at(12, w) = hh;
+    at(13, w) = sts;
+    at(14, w) = fyU;
+    at(15, w) = Cc;
+    at(16, w) = Fc;
+    if constexpr (D4) {
+        P4 = dy * dy * mu4 * hq * stt;
+        Px4 = dx * dx * mu4 * hq * stt;
+        at(17, w) = Px4;
+    }
+    __syncthreads();
+    // ---- phase 3: continuity and the new depths; uv_diff4's first pass
+    const double fvs = at(8, rs), Bvs = at(9, rs), Bv1 = at(9, rn), A1 = at(10, rn), Px1 = at(11, rn);
+    const double hhs = at(12, rs), stss = at(13, rs), fyUs = at(14, rs), Ccs = at(15, rs), Fcs = at(16, rs);
+    const double sn_ = sp + 2.0 * tau * (wf / p.rho0 * p.ffs - (fu - xl(fu) + fv - fvs) / (dx * dy));
+    const double sn = tw ? sn_ : 0.0;
+    const double wn0 = (H + sn) * dx * dy * lu0;
+    at(0, w) = wn0;
+    at(1, w) = sn;
+    const double dybl = xl(dyb), hhl = xl(hh), stsl = xl(sts);
+    double qa4 = 0.0, qb4 = 0.0, qc4 = 0.0, qe4 = 0.0, mu4p = 0.0, mu4m = 0.0, mu4v = 0.0;
+    if constexpr (D4) {
+        const double mu4r = xr(mu4), mu41r = xr(mu41);
+        mu4p = (mu4 + mu4r + mu41 + mu41r) / 4.0;
+        mu4m = (mu4 + mu4r + mu4s + xr(mu4s)) / 4.0;
+        mu4v = (mu4 + xl(mu4) + mu41 + xl(mu41)) / 4.0;
+        const double pu = (xr(P4) - P4) / dyh;
+        const double qu = (dxb * dxb * mu4p * hh * sts - dxbs * dxbs * mu4m * hhs * stss) / dxt;
+        const double pv = (at(17, rn) - Px4) / dxh;
+        const double qv = (dyb * dyb * mu4p * hh * sts - dybl * dybl * mu4v * hhl * stsl) / dyt;
+        const double fu4 = pu + qu, fv4 = -pv + qv;
+        const double vx = -fu4 / hu / dxt / dyh, vy = -fv4 / hv / dxh / dyt;
+        const double fx = ((mb & MB_LCU) && in) ? vx : 0.0, fy = ((mb & MB_LCV) && in) ? vy : 0.0;
+        qa4 = fx / dyh;
+        qb4 = fy / dxh;
+        qc4 = fx / dxt;
+        qe4 = fy / dyt;
+        at(2, w) = qb4;
+        at(3, w) = qc4;
+    }
+    __syncthreads();
+    const double wn1 = at(0, rn), sn1 = at(1, rn);
+    double px = 0.0, qx = 0.0, py = 0.0, qy = 0.0;
+    if constexpr (D4) {
+        // uv_diff4's second pass: the stress of (fx, fy) and its two terms
+        const double tt = yx * (qa4 - xl(qa4)) - xy * (qb4 - at(2, rs));
+        const double sh = bxy * (at(3, rn) - qc4) + byx * (xr(qe4) - qe4);
+        const double stt4 = tw ? tt : 0.0, sts4 = hw ? sh : 0.0;
+        const double R4 = dy * dy * mu4 * hq * stt4, Rx4 = dx * dx * mu4 * hq * stt4;
+        at(4, w) = Rx4;
+        at(5, w) = sts4;
+        __syncthreads();
+        const double sts4l = xl(sts4);
+        px = (xr(R4) - R4) / dyh;
+        qx = (dxb * dxb * mu4p * hh * sts4 - dxbs * dxbs * mu4m * hhs * at(5, rs)) / dxt;
+        py = (at(4, rn) - Rx4) / dxh;
+        qy = (dyb * dyb * mu4p * hh * sts4 - dybl * dybl * mu4v * hhl * sts4l) / dyt;
+    }
+    // ---- last phase: momentum, averages, time-level shift (DStage::row)
+    double hun = avg(wn0 + xr(wn0), lu0 + lu0r, dxt, dyh), hvn = avg(wn0 + wn1, lu0 + lu1, dxh, dyt);
+    hun = (mb & MB_LLU) ? hun : 0.0;
+    hvn = (mb & MB_LLV) ? hvn : 0.0;
+    const double mur = xr(mu), mu1r = xr(mu1);
+    const double muh_p = (mu + mur + mu1 + mu1r) / 4.0;
+    const double fx_p = (A + xr(A)) / 2.0 * (u + xr(u)) / 2.0;
+    const double fx_m = xl(fx_p);
+    const double radv = -(fx_p - fx_m + fyU - fyUs) + (Cc + Ccs) / 4.0;
+    const double muh_m = (mu + mur + mus + xr(mus)) / 4.0;
+    double rdfx = (xr(P) - P) / dyh + (dxb * dxb * muh_p * hh * sts - dxbs * dxbs * muh_m * hhs * stss) / dxt;
+    if constexpr (D4) rdfx = rdfx + px + qx;
+    const double bp = hun * dxt * dyh / 2.0 / tau;
+    const double bp0 = hupc * dxt * dyh / 2.0 / tau;
+    const double slx = -G * (xr(s) - s) * dyh * hu;
+    const double slxn = -G * (xr(sn) - sn) * dyh * hun;
+    const double grx = rx + slx + rdfx + radv - (rd + xr(rd)) / 2.0 * up * dxt * dyh * hu + (Fc + Fcs) / 4.0;
+    double un = (up * bp0 + grx) / bp;
+
+    const double fxV_p = (A + A1) / 2.0 * (v0r + v) / 2.0;
+    const double fxV_m = xl(fxV_p);
+    const double fyV = (Bv + Bv1) / 2.0 * (v + v1) / 2.0, fyVs = (Bvs + Bv) / 2.0 * (vs + v) / 2.0;
+    const double D = vh * (u1 + u);
+    const double rady = -(fxV_p - fxV_m + fyV - fyVs) - (D + xl(D)) / 4.0;
+    const double muhv_m = (mu + xl(mu) + mu1 + xl(mu1)) / 4.0;
+    double rdfy = -(Px1 - Px) / dxh + (dyb * dyb * muh_p * hh * sts - dybl * dybl * muhv_m * hhl * stsl) / dyt;
+    if constexpr (D4) rdfy = rdfy - py + qy;
+    const double bq = hvn * dyt * dxh / 2.0 / tau;
+    const double bq0 = hvpc * dyt * dxh / 2.0 / tau;
+    const double sly = -G * (s1 - s) * dxh * hv;
+    const double slyn = -G * (sn1 - sn) * dxh * hvn;
+    const double Gc = fhdd * (u1 + u);
+    const double gry = ry + sly + rdfy + rady - (rd + rd1) / 2.0 * vp * dxh * dyt * hv - (Gc + xl(Gc)) / 4.0;
+    double vn = (vp * bq0 + gry) / bq;
+    const bool uw = (mb & MB_LCU) && in, vw = (mb & MB_LCV) && in;
+    un = uw ? un : 0.0;
+    vn = vw ? vn : 0.0;
+    if (!writer) return;
+    if (p.cu) {
+        // the state entering this substep: the call's result when this is
+        // substep nstep + 1 (vel_ssh.f90:638-648)
+        p.cu[io] = u;
+        p.cv[io] = v;
+        p.cs[io] = s;
+        p.cup[io] = up;
+        p.cvp[io] = vp;
+        p.csp[io] = sp;
+    }
+    p.acc[0][io] = uw ? a0 + (u * hu + un * hun) / p.d4n : a0;
+    p.acc[2][io] = uw ? a2 + (slx + slxn) / p.d4n : a2;
+    p.acc[1][io] = vw ? a1 + (v * hv + vn * hvn) / p.d4n : a1;
+    p.acc[3][io] = vw ? a3 + (sly + slyn) / p.d4n : a3;
+    if (!p.uo) return;
+    const double ts = p.ts;
+    const bool sh_ = m >= 2 && m <= p.nx - 1 && n >= 2 && n <= p.ny - 1;
+    const double spn = s + ts * (sn - 2.0 * s + sp) / 2.0 / p.dn;
+    const double upn = u + ts * (un - 2.0 * u + up) / 2.0 / p.dn;
+    const double vpn = v + ts * (vn - 2.0 * v + vp) / 2.0 / p.dn;
+    const double hupn = hu + ts * (hun - 2.0 * hu + hupc) / 2.0 / p.dn;
+    const double hvpn = hv + ts * (hvn - 2.0 * hv + hvpc) / 2.0 / p.dn;
+    const bool bs = sh_ && (mb & MB_LU), bu = sh_ && (mb & MB_LCU), bv = sh_ && (mb & MB_LCV);
+    p.so[io] = bs ? sn : s;
+    p.spo[io] = bs ? spn : sp;
+    p.uo[io] = bu ? un : u;
+    p.upo[io] = bu ? upn : up;
+    p.vo[io] = bv ? vn : v;
+    p.vpo[io] = bv ? vpn : vp;
+    p.hupc[io] = sh_ && (mb & MB_LLU) ? hupn : hupc;
+    p.hvpc[io] = sh_ && (mb & MB_LLV) ? hvpn : hvpc;
+}
+
 // ------------------------------------------------------------------ host
 
 struct DropinAlloc {
     double *S[2][6] = {};  // ping-pong state of the substeps: u, up, v, vp, ssh, sshp
     double *hupc = nullptr, *hvpc = nullptr;
-    double *rowmet = nullptr;  // 9 x ny: the metrics and rlh_s per row (when uniform along x)
+    double *rowmet = nullptr;  // 13 x ny: the metrics, rlh_s and four quotients per row (uniform along x)
     uint8_t *mb = nullptr;
     int eligible = -1;  // grid part of the eligibility: -1 not checked, 0 no, 1 yes
     std::string why;
     bool rowmet_ok = false;
     int chunk = 0;
     long long slots = 0;
-    double *b4[6] = {};  // fx, fy, px, qx, py, qy of the biharmonic pre-pass (ksw4 > 0)
+    int tile_nr[2] = {};  // rows per tile without and with the biharmonic term (0: the march)
 };
 
 namespace {
@@ -576,6 +829,37 @@ __global__ void k_dropin_masks(size_t n, const float *lu, const float *luu, cons
     if (llu[i] > 0.5f) b |= MB_LLU;
     if (llv[i] > 0.5f) b |= MB_LLV;
     mb[i] = b;
+}
+
+const void *tile_kernel(bool rowmet, bool d4)
+{
+    return rowmet ? (d4 ? (const void *)k_dropin_tile<true, true> : (const void *)k_dropin_tile<true, false>)
+                  : (d4 ? (const void *)k_dropin_tile<false, true> : (const void *)k_dropin_tile<false, false>);
+}
+
+// Whether this grid's calls run on tiles (below DT_CELLS cells, where they
+// are measured faster than the march; with the biharmonic term always), and
+// their rows: 8 or 12, which give the busiest CU the fewest to work through.
+constexpr size_t DT_CELLS = 400000;
+int choose_tiles(inmsom_bt_ctx *c, DropinAlloc *a, int cus)
+{
+    const long long strips = (c->nx + SW - 1) / SW;
+    for (int d4 = 0; d4 < 2; ++d4) {
+        a->tile_nr[d4] = 0;
+        if (!d4 && c->n >= DT_CELLS) continue;
+        long long best = -1;
+        for (int nr : {12, 8}) {
+            const int rows = nr - DT_RIM;
+            const long long cost = (strips * ((c->ny + rows - 1) / rows) + cus - 1) / cus * (nr + 4);
+            if (best < 0 || cost < best) {
+                best = cost;
+                a->tile_nr[d4] = nr;
+            }
+        }
+        DHC(hipFuncSetAttribute(tile_kernel(a->rowmet_ok, d4), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)dropin_tile_lds(DT_MAX_ROWS)));
+    }
+    return INMSOM_BT_OK;
 }
 
 // The grid part of the eligibility and the row tables, checked once per
@@ -612,7 +896,7 @@ int check_grid(inmsom_bt_ctx *c, DropinAlloc *a)
     // land on the halo the outputs never depend on columns 1 and nx (the
     // reference's own grid set-up leaves its metrics zero there and rlh_s
     // unscaled, Service/basin_parameters.f90:250-300).
-    std::vector<double> f(n), tab((size_t)9 * ny);
+    std::vector<double> f(n), tab((size_t)13 * ny);
     bool rows = true;
     for (int k = 0; k < 9 && rows; ++k) {
         DHC(hipMemcpy(f.data(), k < 8 ? c->metric[k] : c->rlh_s, n * 8, hipMemcpyDeviceToHost));
@@ -627,6 +911,13 @@ int check_grid(inmsom_bt_ctx *c, DropinAlloc *a)
         }
     }
     a->rowmet_ok = rows;
+    for (int r = 0; r < ny && rows; ++r) {
+        const double dx = tab[r], dy = tab[ny + r], dxb = tab[(size_t)6 * ny + r], dyb = tab[(size_t)7 * ny + r];
+        tab[(size_t)9 * ny + r] = dy / dx;
+        tab[(size_t)10 * ny + r] = dx / dy;
+        tab[(size_t)11 * ny + r] = dxb / dyb;
+        tab[(size_t)12 * ny + r] = dyb / dxb;
+    }
     if (rows) {
         DHC(hipMalloc(&a->rowmet, tab.size() * 8));
         DHC(hipMemcpy(a->rowmet, tab.data(), tab.size() * 8, hipMemcpyHostToDevice));
@@ -639,11 +930,12 @@ int check_grid(inmsom_bt_ctx *c, DropinAlloc *a)
     int dev = 0, cus = 0, per_cu = 0;
     DHC(hipGetDevice(&dev));
     DHC(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const void *kf = rows ? (const void *)k_dropin<false, true, false> : (const void *)k_dropin<false, false, false>;
+    const void *kf = rows ? (const void *)k_dropin<false, true> : (const void *)k_dropin<false, false>;
     DHC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kf, WAVE, 0));
     a->slots = (long long)cus * (per_cu > 0 ? per_cu : 1);
     const int strips = (nx + SW - 1) / SW;
     a->chunk = fit_chunk(ny, strips, a->slots, 3, 2);
+    if (const int rc = choose_tiles(c, a, cus)) return rc;
     DHC(hipStreamSynchronize(c->stream));
     a->eligible = 1;
     return INMSOM_BT_OK;
@@ -662,24 +954,11 @@ int ensure_buffers(inmsom_bt_ctx *c, DropinAlloc *a)
     return INMSOM_BT_OK;
 }
 
-// the work planes of the biharmonic pre-pass (lit_diff4_terms), zeroed once
-int ensure_diff4(inmsom_bt_ctx *c, DropinAlloc *a)
-{
-    for (double *&q : a->b4)
-        if (!q) {
-            DHC(hipMalloc(&q, c->n * 8));
-            DHC(hipMemsetAsync(q, 0, c->n * 8, c->stream));
-        }
-    return INMSOM_BT_OK;
-}
-
 template <bool FIRST>
 void launch_dropin(inmsom_bt_ctx *c, const DropinParams &p, bool rowmet)
 {
     dim3 grid((unsigned)(p.per_xcd * NXCD)), blk(WAVE);
-    const bool d4 = p.d4[0] != nullptr;
-    const void *k = rowmet ? (d4 ? (const void *)k_dropin<FIRST, true, true> : (const void *)k_dropin<FIRST, true, false>)
-                           : (d4 ? (const void *)k_dropin<FIRST, false, true> : (const void *)k_dropin<FIRST, false, false>);
+    const void *k = rowmet ? (const void *)k_dropin<FIRST, true> : (const void *)k_dropin<FIRST, false>;
     void *args[] = {const_cast<DropinParams *>(&p)};
     (void)hipLaunchKernel(k, grid, blk, args, 0, c->stream);
 }
@@ -703,7 +982,7 @@ bool dropin_eligible(inmsom_bt_ctx *c, int ksw4, std::string *why)
         if (why) *why = a->why;
         return false;
     }
-    (void)ksw4;  // the biharmonic term is covered by a pre-pass per substep
+    (void)ksw4;  // the biharmonic term runs on the tiles
     return true;
 }
 
@@ -737,6 +1016,7 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
         hupc = a->hupc;
         hvpc = a->hvpc;
     }
+    const int tile_nr = a->tile_nr[ksw4 > 0];
     DropinParams p{};
     p.nx = c->nx;
     p.ny = c->ny;
@@ -752,8 +1032,8 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
     p.wf = wflux;
     p.rx = rhsx;
     p.ry = rhsy;
-    for (int k = 0; k < 9; ++k)
-        p.met[k] = a->rowmet_ok ? a->rowmet + (size_t)k * c->ny : (k < 8 ? c->metric[k] : c->rlh_s);
+    for (int k = 0; k < 13; ++k)
+        p.met[k] = a->rowmet_ok ? a->rowmet + (size_t)k * c->ny : k < 8 ? c->metric[k] : k == 8 ? c->rlh_s : nullptr;
     p.hupc = hupc;
     p.hvpc = hvpc;
     for (int k = 0; k < 4; ++k) p.acc[k] = acc[k];
@@ -769,7 +1049,13 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
             set_error("mu4 is required when ksw4 > 0");
             return INMSOM_BT_EINVAL;
         }
-        if ((rc = ensure_diff4(c, a))) return rc;
+    }
+    if (tile_nr) {
+        p.mu4 = mu4;
+        p.chunk = tile_nr - DT_RIM;
+        p.nchunks = (c->ny + p.chunk - 1) / p.chunk;
+        p.total = p.strips * p.nchunks;
+        p.per_xcd = (p.total + NXCD - 1) / NXCD;
     }
     const int last = 2 * nstep;
     for (int k = 1; k <= last; ++k) {
@@ -792,12 +1078,6 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
         p.spo = wr ? out[5] : nullptr;
         // substep nstep + 1 enters with the state after substep nstep: the
         // call's result (vel_ssh.f90:638-648)
-        // uv_diff4 of this substep from its entering state (level-n surface,
-        // filtered velocities), added by the kernel to its uv_diff2 result
-        if (ksw4 > 0) {
-            lit_diff4_terms(c, in[1], in[3], in[4], mu4, a->b4, a->rowmet_ok ? a->rowmet : nullptr, a->mb);
-            for (int q = 0; q < 4; ++q) p.d4[q] = a->b4[2 + q];
-        }
         const bool snap = k == nstep + 1;
         p.cu = snap ? st[0] : nullptr;
         p.cup = snap ? st[1] : nullptr;
@@ -806,7 +1086,12 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
         p.cs = snap ? st[4] : nullptr;
         p.csp = snap ? st[5] : nullptr;
         p.carry_out = k < last;
-        if (k == 1)
+        if (tile_nr) {
+            int first = k == 1;
+            void *args[] = {&p, &first};
+            (void)hipLaunchKernel(tile_kernel(a->rowmet_ok, ksw4 > 0), dim3((unsigned)(p.per_xcd * NXCD)),
+                                  dim3((unsigned)(WAVE * tile_nr)), args, dropin_tile_lds(tile_nr), c->stream);
+        } else if (k == 1)
             launch_dropin<true>(c, p, a->rowmet_ok);
         else
             launch_dropin<false>(c, p, a->rowmet_ok);
@@ -864,8 +1149,6 @@ void dropin_release(inmsom_bt_ctx *c)
         for (double *q : b)
             if (q) (void)hipFree(q);
     for (void *q : {(void *)a->hupc, (void *)a->hvpc, (void *)a->rowmet, (void *)a->mb})
-        if (q) (void)hipFree(q);
-    for (double *q : a->b4)
         if (q) (void)hipFree(q);
     delete a;
     c->da = nullptr;

@@ -49,6 +49,16 @@ inline void fast_constants(FusedParams &p)
     p.ffs_rho0 = p.ffs / p.rho0;
 }
 
+// A wave-uniform value of a table that no kernel writes, by the scalar unit:
+// into scalar registers (the compiler cannot tell by itself that the kernel's
+// stores leave the table alone).
+template <class T>
+__device__ __forceinline__ T scalar_load(const T *p)
+{
+    typedef const T __attribute__((address_space(4))) * ConstPtr;
+    return *(ConstPtr)(uintptr_t)p;
+}
+
 // Lane shifts by DPP (no LDS traffic).  wave_shl:1 gives lane L the value
 // of lane L+1 (column m+1), wave_shr:1 the value of lane L-1 (column m-1);
 // the lanes at the wave's ends receive 0 and only ever feed halo lanes.

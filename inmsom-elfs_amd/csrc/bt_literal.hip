@@ -64,11 +64,8 @@ __global__ void k_cyclize_y(DevGrid g, double *f)
     f[I(m, g.ny - 1)] = b;
 }
 
-// Metrics and masks of the grid at (a, b), for the stencil helpers below.
-// CellView reads the grid's per-cell planes; RowView (for grids whose
-// metrics are uniform along x on columns 2..nx-1) reads a table of nine
-// rows-long metric vectors (dx dy dxt dyt dxh dyh dxb dyb rlh_s) and packed
-// mask bits (MB_*) for the same values.
+// Metrics and masks of the grid at (a, b), for the stencil helpers below,
+// from the grid's per-cell planes.
 struct CellView {
     const DevGrid *g;
     __device__ size_t at(int a, int b) const { return IDX(*g, a, b); }
@@ -89,30 +86,6 @@ struct CellView {
     __device__ bool is_llv(int a, int b) const { return is(g->llv, a, b); }
     __device__ bool is_lcu(int a, int b) const { return is(g->lcu, a, b); }
     __device__ bool is_lcv(int a, int b) const { return is(g->lcv, a, b); }
-};
-
-struct RowView {
-    const DevGrid *g;
-    const double *__restrict__ rm;
-    const uint8_t *__restrict__ mb;
-    __device__ size_t at(int a, int b) const { return IDX(*g, a, b); }
-    __device__ double met(int k, int b) const { return rm[(size_t)k * (size_t)g->ny + (size_t)(b - 1)]; }
-    __device__ double dx(int, int b) const { return met(0, b); }
-    __device__ double dy(int, int b) const { return met(1, b); }
-    __device__ double dxt(int, int b) const { return met(2, b); }
-    __device__ double dyt(int, int b) const { return met(3, b); }
-    __device__ double dxh(int, int b) const { return met(4, b); }
-    __device__ double dyh(int, int b) const { return met(5, b); }
-    __device__ double dxb(int, int b) const { return met(6, b); }
-    __device__ double dyb(int, int b) const { return met(7, b); }
-    __device__ float lu(int a, int b) const { return (mb[at(a, b)] & MB_LU) ? 1.0f : 0.0f; }
-    __device__ bool is_lu(int a, int b) const { return mb[at(a, b)] & MB_LU; }
-    __device__ bool is_luu(int a, int b) const { return mb[at(a, b)] & MB_LUU; }
-    __device__ bool is_luh(int a, int b) const { return mb[at(a, b)] & MB_LUH; }
-    __device__ bool is_llu(int a, int b) const { return mb[at(a, b)] & MB_LLU; }
-    __device__ bool is_llv(int a, int b) const { return mb[at(a, b)] & MB_LLV; }
-    __device__ bool is_lcu(int a, int b) const { return mb[at(a, b)] & MB_LCU; }
-    __device__ bool is_lcv(int a, int b) const { return mb[at(a, b)] & MB_LCV; }
 };
 
 // Depth on U, V and H points from T-point depths hq(m, n) given by Q,
@@ -449,214 +422,6 @@ __global__ void k_diff4_add(DevGrid g, const double *__restrict__ mu, const doub
     }
 }
 
-// uv_diff4 (Function/vel_ssh.f90:203-312) in two sweeps for a caller that
-// adds its terms itself in the reference's order (RHSx_dif + px + qx and
-// RHSy_dif - py + qy), on a grid that is not periodic.  Each sweep forms
-// what the stage-by-stage path keeps in planes (level-n depths of hh_update,
-// Function/depth.f90:108-170; the stresses of stress_components) at the
-// points its stencil reads, with the same expressions, and the value 0 where
-// the reference does not compute them (outside their index range or mask),
-// as the zero-initialised planes hold there.
-// A view whose reads are moved into the array ([1, nx] x [1, ny]): the
-// stencil of a point outside the interior can then be formed without a
-// branch and discarded; at interior points nothing moves.
-template <class V>
-struct ClampView {
-    V w;
-    const DevGrid *g;
-    __device__ int cx(int a) const { return min(max(a, 1), g->nx); }
-    __device__ int cy(int b) const { return min(max(b, 1), g->ny); }
-    __device__ size_t at(int a, int b) const { return w.at(cx(a), cy(b)); }
-    __device__ double dx(int a, int b) const { return w.dx(cx(a), cy(b)); }
-    __device__ double dy(int a, int b) const { return w.dy(cx(a), cy(b)); }
-    __device__ double dxt(int a, int b) const { return w.dxt(cx(a), cy(b)); }
-    __device__ double dyt(int a, int b) const { return w.dyt(cx(a), cy(b)); }
-    __device__ double dxh(int a, int b) const { return w.dxh(cx(a), cy(b)); }
-    __device__ double dyh(int a, int b) const { return w.dyh(cx(a), cy(b)); }
-    __device__ double dxb(int a, int b) const { return w.dxb(cx(a), cy(b)); }
-    __device__ double dyb(int a, int b) const { return w.dyb(cx(a), cy(b)); }
-};
-
-template <class V>
-struct D4Depth {
-    const V w;
-    const double *sh;
-    // hq = H + ssh at a T point
-    __device__ double hq(int a, int b) const
-    {
-        const size_t j = w.at(a, b);
-        return w.g->hr[j] + sh[j];
-    }
-    __device__ bool in_range(int a, int b) const
-    {
-        return a >= 2 && a <= w.g->nx - 2 && b >= 2 && b <= w.g->ny - 2;
-    }
-    __device__ double hu(int a, int b) const
-    {
-        if (!in_range(a, b) || !w.is_llu(a, b)) return 0.0;
-        return avg_u_w(w, [this](int x, int y) { return hq(x, y); }, a, b);
-    }
-    __device__ double hv(int a, int b) const
-    {
-        if (!in_range(a, b) || !w.is_llv(a, b)) return 0.0;
-        return avg_v_w(w, [this](int x, int y) { return hq(x, y); }, a, b);
-    }
-    __device__ double hh(int a, int b) const
-    {
-        if (!in_range(a, b) || !w.is_luh(a, b)) return 0.0;
-        return avg_h_w(w, [this](int x, int y) { return hq(x, y); }, a, b);
-    }
-    __device__ double hu_nb(int a, int b) const
-    {
-        const int ac = min(max(a, 1), w.g->nx - 1), bc = min(max(b, 1), w.g->ny - 1);
-        const double h = avg_u_w(w, [this](int x, int y) { return hq(x, y); }, ac, bc);
-        return in_range(a, b) && w.is_llu(ac, bc) ? h : 0.0;
-    }
-    __device__ double hv_nb(int a, int b) const
-    {
-        const int ac = min(max(a, 1), w.g->nx - 1), bc = min(max(b, 1), w.g->ny - 1);
-        const double h = avg_v_w(w, [this](int x, int y) { return hq(x, y); }, ac, bc);
-        return in_range(a, b) && w.is_llv(ac, bc) ? h : 0.0;
-    }
-    // the same values without a branch: the average is formed at (a, b)
-    // moved into [1, nx-1] x [1, ny-1] (every point it reads in the array;
-    // unchanged where the value is used) and selected
-    __device__ double hh_nb(int a, int b) const
-    {
-        const int ac = min(max(a, 1), w.g->nx - 1), bc = min(max(b, 1), w.g->ny - 1);
-        const double h = avg_h_w(w, [this](int x, int y) { return hq(x, y); }, ac, bc);
-        return in_range(a, b) && w.is_luh(ac, bc) ? h : 0.0;
-    }
-};
-
-template <class V>
-struct D4Stress {
-    const V w;
-    Plane u, v;
-    __device__ bool interior(int a, int b) const
-    {
-        return a >= 3 && a <= w.g->nx - 2 && b >= 3 && b <= w.g->ny - 2;
-    }
-    __device__ double t(int a, int b) const
-    {
-        if (!interior(a, b) || !w.is_lu(a, b)) return 0.0;
-        return tension_at(w, u, v, a, b);
-    }
-    __device__ double s(int a, int b) const
-    {
-        if (!interior(a, b) || !w.is_luu(a, b)) return 0.0;
-        return shear_at(w, u, v, a, b);
-    }
-    // t and s without a branch, as D4Depth::hh_nb: tension reads (a-1..a,
-    // b-1..b), shear (a..a+1, b..b+1)
-    __device__ double t_nb(int a, int b) const
-    {
-        const int ac = min(max(a, 2), w.g->nx - 1), bc = min(max(b, 2), w.g->ny - 1);
-        const double t = tension_at(w, u, v, ac, bc);
-        return interior(a, b) && w.is_lu(ac, bc) ? t : 0.0;
-    }
-    __device__ double s_nb(int a, int b) const
-    {
-        const int ac = min(max(a, 1), w.g->nx - 1), bc = min(max(b, 1), w.g->ny - 1);
-        const double sv = shear_at(w, u, v, ac, bc);
-        return interior(a, b) && w.is_luu(ac, bc) ? sv : 0.0;
-    }
-};
-
-// One sweep per launch over tiles of D4_TX x D4_TY points (one thread per
-// column, D4_ROWS rows of threads, a wave per row of threads): the tile
-// first forms, once per point, the tension on [m0, m0 + D4_TX] x
-// [n0, n0 + D4_TY] and the shear and H-point depths on
-// [m0 - 1, m0 + D4_TX - 1] x [n0 - 1, n0 + D4_TY - 1] in LDS, which is every
-// point the viscous stencil of its own points reads.
-// FIRST: the sweep of :216-257 from the stress of (a, b) = (up, vp), giving
-// o0, o1 = fx, fy; else the sweep of :259-312 from the stress of
-// (a, b) = (fx, fy), giving o0..o3 = px, qx, py, qy.  Every point of the
-// array is written, 0 off lcu / lcv and outside the interior.  A wave's
-// points share their row, so with RowView its metric reads are uniform.
-constexpr int D4_TX = 64, D4_TY = 15, D4_ROWS = 4;
-constexpr int D4_W = D4_TX + 1, D4_H = D4_TY + 1;
-
-template <bool FIRST, class V>
-__device__ __forceinline__ void d4_sweep(const V &w, const double *__restrict__ mu, const double *__restrict__ a,
-                                         const double *__restrict__ b, const double *__restrict__ sh,
-                                         double *__restrict__ o0, double *__restrict__ o1, double *__restrict__ o2,
-                                         double *__restrict__ o3)
-{
-    __shared__ double Ts[D4_H][D4_W], Ss[D4_H][D4_W], Hs[D4_H][D4_W];
-    const DevGrid &g = *w.g;
-    int bx, by;
-    xcd_tile((int)gridDim.x, (int)gridDim.y, (int)(blockIdx.y * gridDim.x + blockIdx.x), bx, by);
-    const int m0 = 1 + bx * D4_TX, n0 = 1 + by * D4_TY;
-    const int tx = (int)threadIdx.x, tid = (int)(threadIdx.y * D4_TX + threadIdx.x);
-    const D4Depth<V> d{w, sh};
-    const D4Stress<V> st{w, Plane{&g, a}, Plane{&g, b}};
-    for (int r = (int)threadIdx.y; r < D4_H; r += D4_ROWS) {
-        const int ru = __builtin_amdgcn_readfirstlane(r);  // one row per wave
-        Ts[ru][tx] = st.t_nb(m0 + tx, n0 + ru);
-        Ss[ru][tx] = st.s_nb(m0 - 1 + tx, n0 - 1 + ru);
-        Hs[ru][tx] = d.hh_nb(m0 - 1 + tx, n0 - 1 + ru);
-    }
-    if (tid < D4_H) {  // the tile's last column
-        Ts[tid][D4_TX] = st.t(m0 + D4_TX, n0 + tid);
-        Ss[tid][D4_TX] = st.s(m0 - 1 + D4_TX, n0 - 1 + tid);
-        Hs[tid][D4_TX] = d.hh(m0 - 1 + D4_TX, n0 - 1 + tid);
-    }
-    __syncthreads();
-    auto tt = [&](int x, int y) { return Ts[y - n0][x - m0]; };
-    auto ss = [&](int x, int y) { return Ss[y - n0 + 1][x - m0 + 1]; };
-    auto hh = [&](int x, int y) { return Hs[y - n0 + 1][x - m0 + 1]; };
-    // phase 2 forms both stencils at every point of the tile without a
-    // branch (LDS reads stay in the tile; array reads go through cw) and
-    // keeps them on lcu / lcv points of the interior
-    const ClampView<V> cw{w, &g};
-    auto hq = [&](int x, int y) { return d.hq(cw.cx(x), cw.cy(y)); };
-    const int m = m0 + tx;
-    if (m > g.nx) return;
-    for (int j = (int)threadIdx.y; j < D4_TY; j += D4_ROWS) {
-        const int n = __builtin_amdgcn_readfirstlane(n0 + j);  // one row per wave
-        if (n > g.ny) return;
-        const size_t i = w.at(m, n);
-        double pu, qu, pv, qv;
-        const bool in = IN_INTERIOR(g);
-        const bool cu = in && w.is_lcu(m, n), cv = in && w.is_lcv(m, n);
-        visc_u_at(cw, mu, tt, ss, hq, hh, m, n, pu, qu);
-        visc_v_at(cw, mu, tt, ss, hq, hh, m, n, pv, qv);
-        if constexpr (FIRST) {
-            const double fu = pu + qu;
-            const double vx = -fu / d.hu_nb(m, n) / cw.dxt(m, n) / cw.dyh(m, n);
-            const double fv = -pv + qv;
-            const double vy = -fv / d.hv_nb(m, n) / cw.dxh(m, n) / cw.dyt(m, n);
-            o0[i] = cu ? vx : 0.0;
-            o1[i] = cv ? vy : 0.0;
-        } else {
-            o0[i] = cu ? pu : 0.0;
-            o1[i] = cu ? qu : 0.0;
-            o2[i] = cv ? pv : 0.0;
-            o3[i] = cv ? qv : 0.0;
-        }
-    }
-}
-
-// ROW: metrics from rm, the row table (9 x ny) of a grid whose metrics are
-// uniform along x, and masks from mb, the packed mask bits; else the grid's
-// per-cell planes
-template <bool FIRST, bool ROW>
-__global__ __launch_bounds__(D4_TX *D4_ROWS) void k_d4_sweep(DevGrid g, const double *__restrict__ rm,
-                                                             const uint8_t *__restrict__ mb,
-                                                             const double *__restrict__ mu,
-                                                             const double *__restrict__ a,
-                                                             const double *__restrict__ b,
-                                                             const double *__restrict__ sh, double *__restrict__ o0,
-                                                             double *__restrict__ o1, double *__restrict__ o2,
-                                                             double *__restrict__ o3)
-{
-    if constexpr (ROW)
-        d4_sweep<FIRST>(RowView{&g, rm, mb}, mu, a, b, sh, o0, o1, o2, o3);
-    else
-        d4_sweep<FIRST>(CellView{&g}, mu, a, b, sh, o0, o1, o2, o3);
-}
-
 // momentum with Coriolis, pressure gradient, Rayleigh friction and the
 // time-mean accumulators (Function/vel_ssh.f90:531-573)
 struct MomArgs {
@@ -799,25 +564,6 @@ void lit_hh_update(inmsom_bt_ctx *c, const double *sh, double *hqn, double *hun,
     cyclize(c, hun);
     cyclize(c, hvn);
     cyclize(c, hhn);
-}
-
-void lit_diff4_terms(inmsom_bt_ctx *c, const double *up, const double *vp, const double *sh, const double *mu4,
-                     double *const t[6], const double *rowmet, const uint8_t *mb)
-{
-    const DevGrid &g = c->g;
-    const dim3 grid((unsigned)((g.nx + D4_TX - 1) / D4_TX), (unsigned)((g.ny + D4_TY - 1) / D4_TY));
-    const dim3 blk(D4_TX, D4_ROWS);
-    if (rowmet && mb) {
-        hipLaunchKernelGGL((k_d4_sweep<true, true>), grid, blk, 0, c->stream, g, rowmet, mb, mu4, up, vp, sh, t[0],
-                           t[1], nullptr, nullptr);
-        hipLaunchKernelGGL((k_d4_sweep<false, true>), grid, blk, 0, c->stream, g, rowmet, mb, mu4, t[0], t[1], sh,
-                           t[2], t[3], t[4], t[5]);
-    } else {
-        hipLaunchKernelGGL((k_d4_sweep<true, false>), grid, blk, 0, c->stream, g, nullptr, nullptr, mu4, up, vp, sh,
-                           t[0], t[1], nullptr, nullptr);
-        hipLaunchKernelGGL((k_d4_sweep<false, false>), grid, blk, 0, c->stream, g, nullptr, nullptr, mu4, t[0], t[1],
-                           sh, t[2], t[3], t[4], t[5]);
-    }
 }
 
 // Device array of the 12 depth pointers (k_hh_init and k_shift index
