@@ -482,3 +482,43 @@ def test_fused_inference_equals_layer_by_layer(mode):
                 assert np.array_equal(st[k][f].view(np.uint64), ref_st[k][f].view(np.uint64)), (fused, ratio, graph,
                                                                                                k, f)
     assert (out[("never", 3.0, True)][2][:, 0] > 0).all()              # every member had a closure tendency
+
+
+@pytest.mark.parametrize("kind", ["uv", "psi"])
+@pytest.mark.parametrize("b,h,w", [(1, 8, 32), (3, 17, 65), (2, 5, 97)])
+def test_training_batch_in_place(kind, b, h, w):
+    """A training step on samples of the device's training set gives the loss
+    and gradient of the same batch set from the host, bit for bit (the same
+    kernels on the same values; samples repeated and out of order), and the
+    batch keeps its values when the training set changes under it."""
+    n = b + 2
+    x, tgt, mask = _batch(41, n, h, w)
+    x2, tgt2, mask2 = _batch(43, 1, h, w)
+    idx = [n - 1] + [1] * (b - 1)
+    print(f"training batch in place {kind} {b}x{h}x{w} idx {idx}", flush=True)
+    with ClosureNet(b, h, w) as net, ClosureNet(b, h, w) as ref:
+        for m in (net, ref):
+            m.set_output(kind)
+            m.set_params(_params(7))
+        net.dataset_alloc(n)
+        for i in range(n):
+            net.dataset_set(i, x[i], tgt[i], mask[i])
+        ref.set_batch(x[idx], tgt[idx], mask[idx])
+        loss, want = net.eval(idx), ref.loss_grad()
+        assert loss == want, (loss, want)
+        assert net.train_step(idx, lr=1e-3) == want
+        assert np.array_equal(net.grad(), ref.grad())
+        ref.set_params(net.params())
+        # the set changes: the batch is still what it was
+        net.dataset_set(idx[0], x2[0], tgt2[0], mask2[0])
+        assert np.array_equal(net.forward(), ref.forward())
+        assert net.loss_grad() == ref.loss_grad()
+        assert np.array_equal(net.grad(), ref.grad())
+        # new inputs without targets: the training set's stay the batch's
+        net.eval(idx)
+        y, ty, my = x[idx].copy(), tgt[idx].copy(), mask[idx].copy()
+        ty[0], my[0] = tgt2[0], mask2[0]
+        net.set_batch(y)
+        ref.set_batch(y, ty, my)
+        assert net.loss_grad() == ref.loss_grad()
+        assert np.array_equal(net.grad(), ref.grad())
