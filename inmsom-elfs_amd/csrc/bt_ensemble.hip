@@ -35,6 +35,7 @@ __global__ void __launch_bounds__(WAVE)
         p.sub = sub;
         p.nsub = nsub;
         p.dn = (double)nsub;
+        if constexpr (EXACT) time_constants(p);
         const int local = item_local[t];
         const int chunk_id = local / p.strips, strip = local - chunk_id * p.strips;
         fused_chunk<R, EXACT, FORM>(p, chunk_id, strip);
@@ -57,6 +58,7 @@ __global__ void __launch_bounds__(WAVE)
         p.sub = sub;
         p.nsub = nsub;
         p.dn = (double)nsub;
+        if constexpr (EXACT) time_constants(p);
         const int local = item_local[t];
         const int chunk_id = local / p.strips, strip = local - chunk_id * p.strips;
         fused_chunk2<R, EXACT, AFORM>(p, chunk_id, strip);
@@ -250,7 +252,7 @@ bool tile_path(const inmsom_bt_ens *e)
 }
 
 // two substeps per launch: as set, or by mode and size as for one basin
-// (not in FP64_EXACT, whose IEEE divides make it compute-bound, nor below
+// (not in FP64_EXACT, where two windows leave one wave per SIMD, nor below
 // TWO_SUBSTEP_CELLS cells in all with a launch shape of the caller's)
 bool two_per_launch(const inmsom_bt_ens *e)
 {
@@ -495,7 +497,7 @@ FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase
     p.fry_in = mb.fry;
     p.hup_c = mb.hup_c;
     p.hvp_c = mb.hvp_c;
-    fast_constants(p);
+    step_constants(p);
     return p;
 }
 

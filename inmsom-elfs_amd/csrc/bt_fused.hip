@@ -443,8 +443,8 @@ static bool tile_path(const inmsom_bt_ctx *c, int mode)
 // Substeps per launch: as set, or automatically two in FP64 and FP32 on
 // grids large enough to be bandwidth-bound and one otherwise.  Measured on
 // MI355X (us per substep, one / two per launch): 2048 x 1536 FP64 91.3 /
-// 81.5, FP32 66.1 / 53.9, FP64_EXACT 153.8 / 183.1 (its IEEE divides make
-// it compute-bound); 512 x 384 (latency-bound, rows per wave 2) FP32
+// 81.5, FP32 66.1 / 53.9, FP64_EXACT 118 / 138 (two windows in one wave's
+// registers leave one wave per SIMD); 512 x 384 (latency-bound, rows per wave 2) FP32
 // 8.7 / 9.5 per substep.
 int subs_per_launch(const inmsom_bt_ctx *c, int mode)
 {
@@ -557,7 +557,8 @@ static FusedParams make_params(inmsom_bt_ctx *c, FusedAlloc *a, int b, double ta
     p.nu = c->nu;
     p.ffs = (double)c->g.ffs;
     p.d = c->metric0;
-    fast_constants(p);
+    step_constants(p);
+    time_constants(p);
     return p;
 }
 

@@ -5,6 +5,7 @@
 
 #include <type_traits>
 
+#include "bt_exactdiv.h"
 #include "bt_internal.h"
 
 namespace ibt {
@@ -35,18 +36,34 @@ struct FusedParams {
     int sub, nsub;
     double dn;             // dfloat(nstep)
     double inv_d, g_d, nu_d, ffs_rho0;  // 1 / d, g / d, nu / d, ffs / rho0
+    Den q_d, q_dd, q_tau, q_dn, q_rho0;    // FP64_EXACT: divisors d, d * d, tau, dn, rho0
+    int exp_lim;                           // and the limit of ExpCheck
     void *frx, *fry;       // forcing frozen over the substeps of one call (stencil type), written
     const void *frx_in, *fry_in;  // the same, read (a separate buffer when a launch forms new forcing)
     double *hup_c, *hvp_c; // filtered U/V depths carried between substeps (FP64_EXACT only)
 };
 
-// the quotients of the fast modes' constants, once on the host
-inline void fast_constants(FusedParams &p)
+// the constants' quotients of the fast modes and FP64_EXACT's divisors, once on
+// the host, and the divisors that go with a call's time step
+constexpr double DEN_MIN = 0x1p-60, DEN_MAX = 0x1p60;  // divisors' range (ExpCheck)
+inline void step_constants(FusedParams &p)
 {
     p.inv_d = 1.0 / p.d;
     p.g_d = p.g / p.d;
     p.nu_d = p.nu / p.d;
     p.ffs_rho0 = p.ffs / p.rho0;
+    p.q_d = make_den(p.d);
+    p.q_dd = make_den(p.d * p.d);
+    p.q_rho0 = make_den(p.rho0);
+    const bool ok = p.d > DEN_MIN && p.d < DEN_MAX && p.rho0 > DEN_MIN && p.rho0 < DEN_MAX;
+    p.exp_lim = ok ? ExpCheck::LIMIT : -1;  // -1: IEEE divisions throughout
+}
+__host__ __device__ inline void time_constants(FusedParams &p)
+{
+    p.q_tau = make_den(p.tau);
+    p.q_dn = make_den(p.dn);
+    const bool ok = p.tau > DEN_MIN && p.tau < DEN_MAX && p.dn > DEN_MIN && p.dn < DEN_MAX;
+    p.exp_lim = ok ? p.exp_lim : -1;
 }
 
 // A wave-uniform value of a table that no kernel writes, by the scalar unit:
@@ -79,6 +96,7 @@ __device__ __forceinline__ double xl(double x)  // value of column m-1
     return __hiloint2double(dpp_from_left(__double2hiint(x)), dpp_from_left(__double2loint(x)));
 }
 __device__ __forceinline__ float xr(float x) { return __int_as_float(dpp_from_right(__float_as_int(x))); }
+__device__ __forceinline__ int xr(int x) { return dpp_from_right(x); }
 __device__ __forceinline__ float xl(float x) { return __int_as_float(dpp_from_left(__float_as_int(x))); }
 
 // Stores of the step's outputs.  Measured on MI355X at 2048 x 1536 (us per
@@ -102,39 +120,6 @@ __device__ __forceinline__ R bitf(int mb, int bit)
 {
     return (mb & bit) ? R(1) : R(0);
 }
-
-template <typename R, bool EXACT>
-struct Ops {
-    const FusedParams &p;
-    R d, inv_d;
-    __device__ Ops(const FusedParams &pp) : p(pp), d(R(pp.d)), inv_d(R(1.0 / pp.d)) {}
-
-    // depth on a U or V point from its two T points (Function/depth.f90:29-49)
-    __device__ R avg2(R qa, R qb, R la, R lb) const
-    {
-        R slu = la + lb;
-        if constexpr (EXACT) {
-            return (((qa * d) * d) * la + ((qb * d) * d) * lb) / slu / d / d;
-        } else {
-#pragma clang fp contract(fast)
-            return (la * qa + lb * qb) * (slu > R(1.5) ? R(0.5) : R(1));
-        }
-    }
-    // depth on an H point from its four T points (:51-66)
-    __device__ R avg4(R q1, R q2, R q3, R q4, R l1, R l2, R l3, R l4) const
-    {
-        R slu = l1 + l2 + l3 + l4;
-        if constexpr (EXACT) {
-            return (((q1 * d) * d) * l1 + ((q2 * d) * d) * l2 + ((q3 * d) * d) * l3 +
-                    ((q4 * d) * d) * l4) /
-                   slu / d / d;
-        } else {
-#pragma clang fp contract(fast)
-            R rs = slu > R(3.5) ? R(0.25) : slu > R(2.5) ? R(1.0 / 3.0) : slu > R(1.5) ? R(0.5) : R(1);
-            return (l1 * q1 + l2 * q2 + l3 * q3 + l4 * q4) * rs;
-        }
-    }
-};
 
 // Loads are branch-free: the address is clamped into the array and the
 // value is zeroed afterwards when the cell lies outside it.  Straight-line
@@ -188,7 +173,7 @@ inline int auto_chunk(bool fp32, long long strip_rows)
     return (int)(c < 4 ? 4 : c > big ? big : c);
 }
 
-// What one substep consumes at iteration n of its march (already zeroed
+// What one substep consumes at iteration n of its march (the mask bits zeroed
 // outside the array): surface height, depth at rest and mask bits of row
 // n+2; level-n velocity, filtered level and Rayleigh coefficient of row
 // n+1; the frozen forcing and carried U/V depths of row n; the row tables.
@@ -215,44 +200,68 @@ struct StageOut {
     double hu, hv;
 };
 
-// One leap-frog substep marching down the rows of one strip: the rolling
-// register window (suffix m1 = row n-1, 0 = row n, p1 = n+1, p2 = n+2) of
-// input rows and of the T- and H-point intermediates.  row(n) takes the
-// inputs of iteration n and, when asked, computes the outputs of row n.
-// FORM: the call's first substep, which forms the wind + drag forcing;
-// the later substeps take it frozen (StageIn::fx0, fy0).
-template <typename R, bool EXACT, bool FORM>
-struct Stage {
-    static constexpr bool frozen = !FORM;
+// One leap-frog substep of FP64_EXACT marching down the rows of one strip: the
+// rolling register window (suffix m1 = row n-1, 0 = row n, p1 = n+1, p2 = n+2)
+// of input rows and of T-, U-, V- and H-point terms.  row(n) takes the inputs
+// of iteration n and, when asked, computes the outputs of row n.  FORM: the
+// call's first substep, which forms the wind + drag forcing; the later
+// substeps take it frozen (StageIn::fx0, fy0).
+//
+// The results are the reference's expressions operation by operation.  Bound
+// by its FP64 operations, of which IEEE divisions were two thirds, so:
+//  - terms that neighbours use (the cell volumes w of the depth averages, the
+//    fluxes, the stress terms, a velocity's quotient by d) are formed once and
+//    shifted; a sum of two is the same in either order;
+//  - d / d is 1, and a quotient by 1, 2 or 4 a product, exactly;
+//  - the quotients by d, d * d, tau, dn and rho0 take quots (bt_exactdiv.h),
+//    groups of them after one look at their numerators' exponents;
+//  - the quotient by 3 of a depth average of three cells is formed where a
+//    lane of the wave has one;
+//  - un and vn, by a depth, stay IEEE divisions.
+// Measured on MI355X, us per substep before / after: 1021 x 763 43.5 / 34.6,
+// 2048 x 1536 154 / 118, where its traffic (about 160 bytes a cell: 103 us at
+// the copy rate of 4.9 TB/s) bounds it instead.
+template <bool FORM>
+struct ExactStage {
     const FusedParams &p;
-    const Ops<R, EXACT> op;
     const bool inx, inx1;
 
-    R u_m1 = 0, u_0 = 0, u_p1 = 0, v_m1 = 0, v_0 = 0, v_p1 = 0;
-    R s_0 = 0, s_p1 = 0, s_p2 = 0, H_p1 = 0, H_p2 = 0;
+    double u_0 = 0, u_p1 = 0, v_0 = 0, v_p1 = 0;
+    double s_0 = 0, s_p1 = 0, s_p2 = 0, H_p1 = 0, H_p2 = 0;
     double up_0 = 0, up_p1 = 0, vp_0 = 0, vp_p1 = 0, sp_0 = 0, sp_p1 = 0;
-    R rd_0 = 0, rd_p1 = 0;
-    int mb_m1 = 0, mb_0 = 0, mb_p1 = 0, mb_p2 = 0;
-    R hq_0 = 0, hq_p1 = 0, hq_p2 = 0, hqp_0 = 0, hqp_p1 = 0, hqn_0 = 0, hqn_p1 = 0;
-    R hu_0 = 0, hu_p1 = 0, hup_0 = 0, hup_p1 = 0;
-    R hv_m1 = 0, hv_0 = 0, hv_p1 = 0, hvp_0 = 0, hvn_0 = 0;
-    R hh_m1 = 0, hh_0 = 0;
-    double sn_0 = 0, sn_p1 = 0;
-    R hun_0 = 0, hun_p1 = 0, stt_0 = 0, stt_p1 = 0, bf_0 = 0, bf_p1 = 0;
-    R sts_m1 = 0, sts_0 = 0, vo_m1 = 0, vo_0 = 0;
-    R f_m1 = 0, f_0 = 0;
+    double rd_0 = 0, rd_p1 = 0;
+    int mb_0 = 0, mb_p1 = 0, mb_p2 = 0;
+    // cell volumes ((q * d) * d) * lu of the levels n, n-1 and n+1, and w + its
+    // right neighbour's
+    double w_p1 = 0, w_p2 = 0, su_0 = 0, su_p1 = 0, wp_0 = 0, wn_0 = 0;
+    int lus_0 = 0, lus_p1 = 0, lu_p1 = 0, lu_p2 = 0;  // lu, lu + its right neighbour's
+    double hq_p1 = 0, hq_p2 = 0;
+    double hu_0 = 0, hu_p1 = 0, hup_0 = 0, hv_0 = 0, hv_p1 = 0;
+    double sn_0 = 0, hun_0 = 0;
+    double qu_0 = 0, qv_0 = 0;            // up / d, vp / d
+    double V_0 = 0, Q_0 = 0;              // v hv d, v d d hv
+    double A_0 = 0, B_0 = 0;              // u d hu, v d hv
+    double T_0 = 0, S_m1 = 0;             // d d mu hq stt, d d muh hh sts
+    double fy_m1 = 0, gy_m1 = 0;          // momentum fluxes through the row's south faces
+    double C_m1 = 0, E_m1 = 0;            // vorticity and Coriolis terms of the H point south
+    double bf_0 = 0;
+    int slow = 0;                         // rows for which the depths take IEEE divisions
 
-    __device__ Stage(const FusedParams &pp, int m)
-        : p(pp), op(pp), inx(m >= 3 && m <= pp.nx - 2), inx1(m >= 2 && m <= pp.nx - 1)
+    __device__ ExactStage(const FusedParams &pp, int m)
+        : p(pp), inx(m >= 3 && m <= pp.nx - 2), inx1(m >= 2 && m <= pp.nx - 1)
     {
     }
 
-    __device__ __forceinline__ void row(int n, const StageIn<R> &q, bool produce, StageOut<R> &o)
+    // 1 / n of a depth average over n = 1, 2 or 4 cells (n = 3: the quotient,
+    // n = 0: not a number, as 0 / 0)
+    static __device__ __forceinline__ double inv_cells(int n)
     {
-        const R d = op.d;
-        const R tau = R(p.tau);
-        const R G = R(p.g);
-        const R nu = R(p.nu);
+        return n == 4 ? 0.25 : n == 2 ? 0.5 : n == 0 ? __builtin_inf() : 1.0;
+    }
+
+    __device__ __forceinline__ void row(int n, const StageIn<double> &q, bool produce, StageOut<double> &o)
+    {
+        const double d = p.d, tau = p.tau, nu = p.nu;
         const int k1 = n + 1;
         s_p2 = q.s2;
         H_p2 = q.H2;
@@ -263,281 +272,199 @@ struct Stage {
         vp_p1 = q.vp1;
         sp_p1 = q.sp1;
         rd_p1 = q.rd1;
-        f_m1 = f_0;
-        f_0 = q.f0;
-        const R sx_0 = q.sx0, sy_0 = q.sy0, wf_p1 = q.wf1;
-
-        const R lu_0 = bitf<R>(mb_0, MB_LU), lu_p1 = bitf<R>(mb_p1, MB_LU), lu_p2 = bitf<R>(mb_p2, MB_LU);
-        const R lu_0r = xr(lu_0), lu_p1r = xr(lu_p1);
+        const double f_0 = q.f0;
         const bool iny1 = (k1 >= 3 && k1 <= p.ny - 2);
+        const bool tw = (mb_p1 & MB_LU) && inx && iny1;
 
         // ---- depths (hh_init / hh_update, Function/depth.f90)
+        lu_p2 = mb_p2 & MB_LU ? 1 : 0;
+        lus_p1 = lu_p1 + xr(lu_p1);
+        const int lu_0 = mb_0 & MB_LU ? 1 : 0;
+        const double lf_p1 = lu_p1, lf_p2 = lu_p2;
         hq_p2 = H_p2 + s_p2;
-        hqp_p1 = H_p1 + R(sp_p1);
+        w_p2 = ((hq_p2 * d) * d) * lf_p2;
+        su_p1 = w_p1 + xr(w_p1);
+        const double wp_p1 = (((H_p1 + sp_p1) * d) * d) * lf_p1;
+        double hup_p1 = 0.0, hvp_0 = 0.0, hh_0;
         {
-            const R hq1r = xr(hq_p1), hqp1r = xr(hqp_p1), hqp0 = hqp_0;
-            hu_p1 = (mb_p1 & MB_LLU) ? op.avg2(hq_p1, hq1r, lu_p1, lu_p1r) : R(0);
-            hup_p1 = (mb_p1 & MB_LLU) ? op.avg2(hqp_p1, hqp1r, lu_p1, lu_p1r) : R(0);
-            hv_p1 = (mb_p1 & MB_LLV) ? op.avg2(hq_p1, hq_p2, lu_p1, lu_p2) : R(0);
-            hvp_0 = (mb_0 & MB_LLV) ? op.avg2(hqp0, hqp_p1, lu_0, lu_p1) : R(0);
-            const R hq0r = xr(hq_0);
-            hh_0 = (mb_0 & MB_LUH) ? op.avg4(hq_0, hq0r, hq_p1, hq1r, lu_0, lu_0r, lu_p1, lu_p1r) : R(0);
+            ExpCheck ck;
+            ck.add(w_p2);
+            if (FORM) ck.add(wp_p1);
+            slow = ck.any(p.exp_lim) ? 4 : slow - 1;
+            const int nh = lus_0 + lus_p1;
+            const double sum4 = (su_0 + w_p1) + xr(w_p1);
+            double mean4 = sum4 * inv_cells(nh);
+            if (__any(nh == 3)) mean4 = nh == 3 ? sum4 / 3.0 : mean4;
+            double a[3] = {su_p1 * inv_cells(lus_p1), (w_p1 + w_p2) * inv_cells(lu_p1 + lu_p2), mean4};
+            quots2(a, p.q_d, slow > 0);
+            hu_p1 = (mb_p1 & MB_LLU) ? a[0] : 0.0;
+            hv_p1 = (mb_p1 & MB_LLV) ? a[1] : 0.0;
+            hh_0 = (mb_0 & MB_LUH) ? a[2] : 0.0;
+            if constexpr (FORM) {
+                double b[2] = {(wp_p1 + xr(wp_p1)) * inv_cells(lus_p1), (wp_0 + wp_p1) * inv_cells(lu_0 + lu_p1)};
+                quots2(b, p.q_d, slow > 0);
+                hup_p1 = (mb_p1 & MB_LLU) ? b[0] : 0.0;
+                hvp_0 = (mb_0 & MB_LLV) ? b[1] : 0.0;
+            }
         }
 
         // ---- T-point stage of row n+1: continuity, new depths, tension, drag
-        const R u1l = xl(u_p1), hu1l = xl(hu_p1), up1l = xl(R(up_p1));
+        const double U_p1 = u_p1 * hu_p1 * d, V_p1 = v_p1 * hv_p1 * d;
+        const double div = U_p1 - xl(U_p1) + V_p1 - V_0;
+        double qc[1] = {div}, qw[1] = {q.wf1}, quv[2] = {up_p1, vp_p1};
         {
-            const bool tw = (mb_p1 & MB_LU) && inx && iny1;
-            const R wf = wf_p1;
-            double sn;
-            if constexpr (EXACT) {
-                sn = sp_p1 + 2.0 * p.tau *
-                                 (wf / p.rho0 * p.ffs -
-                                  (u_p1 * hu_p1 * d - u1l * hu1l * d + v_p1 * hv_p1 * d -
-                                   v_0 * hv_0 * d) /
-                                      (d * d));
-            } else {
-#pragma clang fp contract(fast)
-                const R inc = R(2.0 * p.tau) * (wf * R(p.ffs / p.rho0) -
-                                                (u_p1 * hu_p1 - u1l * hu1l + v_p1 * hv_p1 - v_0 * hv_0) *
-                                                    op.inv_d);
-                sn = sp_p1 + double(inc);
-            }
-            sn_p1 = tw ? sn : 0.0;
+            ExpCheck ck;
+            ck.add(div);
+            ck.add(q.wf1);
+            ck.add(up_p1);
+            ck.add(vp_p1);
+            const bool ieee = ck.any(p.exp_lim);
+            quots(qc, p.q_dd, ieee);
+            quots(qw, p.q_rho0, ieee);
+            quots(quv, p.q_d, ieee);
         }
-        hqn_p1 = H_p1 + R(sn_p1);
+        const double sn = sp_p1 + 2.0 * tau * (qw[0] * p.ffs - qc[0]);
+        const double sn_p1 = tw ? sn : 0.0;
+        const double wn_p1 = (((H_p1 + sn_p1) * d) * d) * lf_p1;
+        double hun_p1, hvn_0;
         {
-            const R hqn1r = xr(hqn_p1);
-            hun_p1 = (mb_p1 & MB_LLU) ? op.avg2(hqn_p1, hqn1r, lu_p1, lu_p1r) : R(0);
-            hvn_0 = (mb_0 & MB_LLV) ? op.avg2(hqn_0, hqn_p1, lu_0, lu_p1) : R(0);
+            ExpCheck ck;
+            ck.add(wn_p1);
+            if (ck.any(p.exp_lim)) slow = 4;
+            double a[2] = {(wn_p1 + xr(wn_p1)) * inv_cells(lus_p1), (wn_0 + wn_p1) * inv_cells(lu_0 + lu_p1)};
+            quots2(a, p.q_d, slow > 0);
+            hun_p1 = (mb_p1 & MB_LLU) ? a[0] : 0.0;
+            hvn_0 = (mb_0 & MB_LLV) ? a[1] : 0.0;
         }
-        {
-            const bool tw = (mb_p1 & MB_LU) && inx && iny1;
-            R st, bf;
-            const R upr = R(up_p1), vpr = R(vp_p1), vp0r = R(vp_0);
-            bf = R(0);
-            if constexpr (EXACT) {
-                st = d / d * (upr / d - up1l / d) - d / d * (vpr / d - vp0r / d);
-                if constexpr (FORM) {
-                    R ut = (u_p1 * d * d * hu_p1 + u1l * d * d * hu1l) / 2.0 / d / d / hq_p1;
-                    R vt = (v_p1 * d * d * hv_p1 + v_0 * d * d * hv_0) / 2.0 / d / d / hq_p1;
-                    bf = R(p.cb) * sqrt(ut * ut + vt * vt + R(p.eb));
-                }
-            } else {
-#pragma clang fp contract(fast)
-                st = op.inv_d * ((upr - up1l) - (vpr - vp0r));
-                if constexpr (FORM) {
-                    const R rh = R(0.5) / hq_p1;
-                    R ut = (u_p1 * hu_p1 + u1l * hu1l) * rh;
-                    R vt = (v_p1 * hv_p1 + v_0 * hv_0) * rh;
-                    bf = R(p.cb) * sqrt(ut * ut + vt * vt + R(p.eb));
-                }
-            }
-            stt_p1 = tw ? st : R(0);
-            bf_p1 = (tw && FORM) ? bf : R(0);
+        const double qu_p1 = quv[0], qv_p1 = quv[1];
+        const double qu1l = xl(qu_p1), qv0r = xr(qv_0);  // lane shifts, outside any branch
+        const double stt_p1 = tw ? (qu_p1 - qu1l) - (qv_p1 - qv_0) : 0.0;
+        double bf_p1 = 0.0, Q_p1 = 0.0;
+        if constexpr (FORM) {
+            const double P_p1 = u_p1 * d * d * hu_p1;
+            Q_p1 = v_p1 * d * d * hv_p1;
+            double a[2] = {(P_p1 + xl(P_p1)) / 2.0, (Q_p1 + Q_0) / 2.0};
+            ExpCheck ck;
+            ck.add(a[0]);
+            ck.add(a[1]);
+            quots2(a, p.q_d, ck.any(p.exp_lim));
+            const double ut = a[0] / hq_p1, vt = a[1] / hq_p1;
+            const double bf = p.cb * sqrt(ut * ut + vt * vt + p.eb);
+            bf_p1 = tw ? bf : 0.0;
         }
 
-        // ---- H-point stage of row n: shear and metric vorticity
-        {
-            const bool hw = (mb_0 & MB_LUU) && inx && (n >= 3 && n <= p.ny - 2);
-            const R vp0 = R(vp_0), vp0r = xr(vp0);
-            const R v0r = xr(v_0);
-            R ss, vo;
-            if constexpr (EXACT) {
-                ss = d / d * (R(up_p1) / d - R(up_0) / d) + d / d * (vp0r / d - vp0 / d);
-                vo = (v0r * d - v_0 * d) - (u_p1 * d - u_0 * d) - ((v0r - v_0) * d - (u_p1 - u_0) * d);
-            } else {
-#pragma clang fp contract(fast)
-                ss = op.inv_d * ((R(up_p1) - R(up_0)) + (vp0r - vp0));
-                vo = R(0);  // identically zero for uniform metrics (vel_ssh.f90:35-37)
-            }
-            sts_0 = hw ? ss : R(0);
-            vo_0 = hw ? vo : R(0);
-        }
+        // ---- H-point stage of row n: shear, metric vorticity, Coriolis
+        const double v0r = xr(v_0);
+        const bool hw = (mb_0 & MB_LUU) && inx && (n >= 3 && n <= p.ny - 2);
+        const double sts_0 = hw ? (qu_p1 - qu_0) + (qv0r - qv_0) : 0.0;
+        const double vo = (v0r * d - v_0 * d) - (u_p1 * d - u_0 * d) - ((v0r - v_0) * d - (u_p1 - u_0) * d);
+        const double vh = (hw ? vo : 0.0) * hh_0;
+        const double fh = f_0 * hh_0 * d * d;
+        const double C_0 = vh * (v0r + v_0), D_0 = vh * (u_p1 + u_0);
+        const double E_0 = fh * (v0r + v_0), F_0 = fh * (u_p1 + u_0);
+        // viscosity: mu at T points, its mean at the H point
+        const double mu_0 = lu_0 * nu, mu_p1 = lf_p1 * nu;
+        const double muh = (mu_0 + xr(mu_0) + mu_p1 + xr(mu_p1)) / 4.0;
+        const double T_p1 = d * d * mu_p1 * hq_p1 * stt_p1, S_0 = d * d * muh * hh_0 * sts_0;
+        // momentum fluxes (uv_trans, vel_ssh.f90:59-105)
+        const double A_p1 = u_p1 * d * hu_p1, B_p1 = v_p1 * d * hv_p1;
+        const double B0r = xr(B_0), luu0 = mb_0 & MB_LUU ? 1.0 : 0.0;
+        const double fy_0 = (B_0 + B0r) / 2.0 * (u_p1 + u_0) / 2.0 * luu0;
+        const double gy_0 = (B_0 + B_p1) / 2.0 * (v_0 + v_p1) / 2.0;
 
         // ---- outputs of row n
         if (produce) {
             const bool iny = (n >= 3 && n <= p.ny - 2);
-            const R lu_m1 = bitf<R>(mb_m1, MB_LU);
-            const R mu_m1 = lu_m1 * nu, mu_0 = lu_0 * nu, mu_p1 = lu_p1 * nu;
-            const R mu_m1r = xr(mu_m1), mu_0r = xr(mu_0), mu_p1r = xr(mu_p1);
-            const R mu_0l = xl(mu_0), mu_p1l = xl(mu_p1);
-            const R u0r = xr(u_0), u0l = xl(u_0), hu0r = xr(hu_0), hu0l = xl(hu_0);
-            const R v0r = xr(v_0), v0l = xl(v_0), hv0r = xr(hv_0);
-            const R vm1r = xr(v_m1), hvm1r = xr(hv_m1);
-            const R up1l_ = xl(u_p1), hup1l = xl(hu_p1);
-            const R s0r = xr(s_0), rd0r = xr(rd_0), bf0r = xr(bf_0);
-            const R hq0r = xr(hq_0), stt0r = xr(stt_0);
-            const R hh0l = xl(hh_0), sts0l = xl(sts_0), vo0l = xl(vo_0);
-            const R up0 = R(up_0), vp0 = R(vp_0);
-            const R luu0 = bitf<R>(mb_0, MB_LUU), luum1 = bitf<R>(mb_m1, MB_LUU);
-            const R sx = sx_0, sy = sy_0;
+            const double bf0r = xr(bf_0), s0r = xr(s_0), rd0r = xr(rd_0);
             // the RHS of Control/dyncall.f90:114-126 is formed once per call
             // (first substep) and frozen over the call's substeps
-            R rhs_u = q.fx0, rhs_v = q.fy0;
+            double rhs_u = q.fx0, rhs_v = q.fy0;
             if constexpr (FORM) {
-                if constexpr (EXACT) {
-                    rhs_u = 0.0 + (sx + (-(bf_0 + bf0r) / 2.0 * up0)) * d * d;
-                    rhs_v = 0.0 + (sy + (-(bf_0 + bf_p1) / 2.0 * vp0)) * d * d;
-                } else {
-#pragma clang fp contract(fast)
-                    rhs_u = sx - R(0.5) * (bf_0 + bf0r) * up0;
-                    rhs_v = sy - R(0.5) * (bf_0 + bf_p1) * vp0;
-                }
+                rhs_u = 0.0 + (q.sx0 + (-(bf_0 + bf0r) / 2.0 * up_0)) * d * d;
+                rhs_v = 0.0 + (q.sy0 + (-(bf_0 + bf_p1) / 2.0 * vp_0)) * d * d;
             }
             o.rhs_u = rhs_u;
             o.rhs_v = rhs_v;
             // level n-1 U/V depths: hh_init values at the first substep,
             // the hh_shift-filtered carry afterwards (depth.f90:195-203)
-            R hupc = hup_0, hvpc = hvp_0;
-            if constexpr (EXACT && frozen) {
-                hupc = R(q.hupc0);
-                hvpc = R(q.hvpc0);
+            const double hupc = FORM ? hup_0 : q.hupc0, hvpc = FORM ? hvp_0 : q.hvpc0;
+            const double T0r = xr(T_0), S0l = xl(S_0), F0l = xl(F_0), D0l = xl(D_0);
+            double a[4] = {T0r - T_0, S_0 - S_m1, T_p1 - T_0, S_0 - S0l};
+            double b[4] = {hun_0 * d * d / 2.0, hupc * d * d / 2.0, hvn_0 * d * d / 2.0, hvpc * d * d / 2.0};
+            {
+                ExpCheck ck;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    ck.add(a[k]);
+                    ck.add(b[k]);
+                }
+                const bool ieee = ck.any(p.exp_lim);
+                quots(a, p.q_d, ieee);
+                quots(b, p.q_tau, ieee);
             }
-            R un, vn;
-            if constexpr (EXACT) {
-                // zonal momentum (vel_ssh.f90:536-551) with uv_trans (:59-81) and uv_diff2 (:146-159)
-                R rhsx = rhs_u;
-                R fx_p = (u_0 * d * hu_0 + u0r * d * hu0r) / 2.0 * (u_0 + u0r) / 2.0;
-                R fx_m = (u_0 * d * hu_0 + u0l * d * hu0l) / 2.0 * (u_0 + u0l) / 2.0;
-                R fy_p = (v_0 * d * hv_0 + v0r * d * hv0r) / 2.0 * (u_p1 + u_0) / 2.0 * luu0;
-                R fy_m = (v_m1 * d * hv_m1 + vm1r * d * hvm1r) / 2.0 * (u_m1 + u_0) / 2.0 * luum1;
-                R radv = -(fx_p - fx_m + fy_p - fy_m) +
-                         (vo_0 * hh_0 * (v0r + v_0) + vo_m1 * hh_m1 * (vm1r + v_m1)) / 4.0;
-                R muh_p = (mu_0 + mu_0r + mu_p1 + mu_p1r) / 4.0;
-                R muh_m = (mu_0 + mu_0r + mu_m1 + mu_m1r) / 4.0;
-                R pp = (d * d * mu_0r * hq0r * stt0r - d * d * mu_0 * hq_0 * stt_0) / d;
-                R qq = (d * d * muh_p * hh_0 * sts_0 - d * d * muh_m * hh_m1 * sts_m1) / d;
-                R rdfx = pp + qq;
-                R bp = hun_0 * d * d / 2.0 / tau;
-                R bp0 = hupc * d * d / 2.0 / tau;
-                R slx = -G * (s0r - s_0) * d * hu_0;
-                R grx = rhsx + slx + rdfx + radv - (rd_0 + rd0r) / 2.0 * up0 * d * d * hu_0 +
-                        (f_0 * hh_0 * d * d * (v0r + v_0) + f_m1 * hh_m1 * d * d * (vm1r + v_m1)) / 4.0;
-                un = (up0 * bp0 + grx) / bp;
+            // zonal momentum (vel_ssh.f90:536-551) with uv_trans (:59-81) and uv_diff2 (:146-159)
+            double un, vn;
+            {
+                const double fx_p = (A_0 + xr(A_0)) / 2.0 * (u_0 + xr(u_0)) / 2.0, fx_m = xl(fx_p);
+                const double radv = -(fx_p - fx_m + fy_0 - fy_m1) + (C_0 + C_m1) / 4.0;
+                const double rdfx = a[0] + a[1];
+                const double slx = -p.g * (s0r - s_0) * d * hu_0;
+                const double grx =
+                    rhs_u + slx + rdfx + radv - (rd_0 + rd0r) / 2.0 * up_0 * d * d * hu_0 + (E_0 + E_m1) / 4.0;
+                un = (up_0 * b[1] + grx) / b[0];
+            }
+            // meridional momentum (vel_ssh.f90:554-569) with uv_trans (:84-105) and uv_diff2 (:162-175)
+            {
+                const double gx_p = (A_0 + A_p1) / 2.0 * (v0r + v_0) / 2.0, gx_m = xl(gx_p);
+                const double rady = -(gx_p - gx_m + gy_0 - gy_m1) - (D_0 + D0l) / 4.0;
+                const double rdfy = -a[2] + a[3];
+                const double sly = -p.g * (s_p1 - s_0) * d * hv_0;
+                const double gry =
+                    rhs_v + sly + rdfy + rady - (rd_0 + rd_p1) / 2.0 * vp_0 * d * d * hv_0 - (F_0 + F0l) / 4.0;
+                vn = (vp_0 * b[3] + gry) / b[2];
+            }
+            un = ((mb_0 & MB_LCU) && inx && iny) ? un : 0.0;
+            vn = ((mb_0 & MB_LCV) && inx && iny) ? vn : 0.0;
 
-                // meridional momentum (vel_ssh.f90:554-569) with uv_trans (:84-105) and uv_diff2 (:162-175)
-                R rhsy = rhs_v;
-                R gy_p = (v_0 * d * hv_0 + v_p1 * d * hv_p1) / 2.0 * (v_0 + v_p1) / 2.0;
-                R gy_m = (v_0 * d * hv_0 + v_m1 * d * hv_m1) / 2.0 * (v_0 + v_m1) / 2.0;
-                R gx_p = (u_0 * d * hu_0 + u_p1 * d * hu_p1) / 2.0 * (v0r + v_0) / 2.0;
-                R gx_m = (u0l * d * hu0l + up1l_ * d * hup1l) / 2.0 * (v0l + v_0) / 2.0;
-                R rady = -(gx_p - gx_m + gy_p - gy_m) -
-                         (vo_0 * hh_0 * (u_p1 + u_0) + vo0l * hh0l * (up1l_ + u0l)) / 4.0;
-                R nuh_p = (mu_0 + mu_0r + mu_p1 + mu_p1r) / 4.0;
-                R nuh_m = (mu_0 + mu_0l + mu_p1 + mu_p1l) / 4.0;
-                R py = (d * d * mu_p1 * hq_p1 * stt_p1 - d * d * mu_0 * hq_0 * stt_0) / d;
-                R qy = (d * d * nuh_p * hh_0 * sts_0 - d * d * nuh_m * hh0l * sts0l) / d;
-                R rdfy = -py + qy;
-                R bq = hvn_0 * d * d / 2.0 / tau;
-                R bq0 = hvpc * d * d / 2.0 / tau;
-                R sly = -G * (s_p1 - s_0) * d * hv_0;
-                R gry = rhsy + sly + rdfy + rady - (rd_0 + rd_p1) / 2.0 * vp0 * d * d * hv_0 -
-                        (f_0 * hh_0 * d * d * (u_p1 + u_0) + f_0 * hh0l * d * d * (up1l_ + u0l)) / 4.0;
-                vn = (vp0 * bq0 + gry) / bq;
-            } else {
-#pragma clang fp contract(fast)
-                const R id = op.inv_d;
-                const R two_tau = R(2.0) * tau;
-                // forces per unit area (the reference's terms divided by dxt*dyh)
-                R adv = R(-0.25) * ((u_0 * hu_0 + u0r * hu0r) * (u_0 + u0r) -
-                                    (u_0 * hu_0 + u0l * hu0l) * (u_0 + u0l) +
-                                    luu0 * (v_0 * hv_0 + v0r * hv0r) * (u_p1 + u_0) -
-                                    luum1 * (v_m1 * hv_m1 + vm1r * hvm1r) * (u_m1 + u_0));
-                R muh_p = R(0.25) * (mu_0 + mu_0r + mu_p1 + mu_p1r);
-                R muh_m = R(0.25) * (mu_0 + mu_0r + mu_m1 + mu_m1r);
-                R dif = (mu_0r * hq0r * stt0r - mu_0 * hq_0 * stt_0) +
-                        (muh_p * hh_0 * sts_0 - muh_m * hh_m1 * sts_m1);
-                R F = rhs_u - G * id * (s0r - s_0) * hu_0 +
-                      id * (adv + dif) - R(0.5) * (rd_0 + rd0r) * up0 * hu_0 +
-                      R(0.25) * (f_0 * hh_0 * (v0r + v_0) + f_m1 * hh_m1 * (vm1r + v_m1));
-                un = (up0 * hupc + two_tau * F) / hun_0;
-
-                R advy = R(-0.25) * ((u_0 * hu_0 + u_p1 * hu_p1) * (v0r + v_0) -
-                                     (u0l * hu0l + up1l_ * hup1l) * (v0l + v_0) +
-                                     (v_0 * hv_0 + v_p1 * hv_p1) * (v_0 + v_p1) -
-                                     (v_0 * hv_0 + v_m1 * hv_m1) * (v_0 + v_m1));
-                R nuh_p = R(0.25) * (mu_0 + mu_0r + mu_p1 + mu_p1r);
-                R nuh_m = R(0.25) * (mu_0 + mu_0l + mu_p1 + mu_p1l);
-                R dify = -(mu_p1 * hq_p1 * stt_p1 - mu_0 * hq_0 * stt_0) +
-                         (nuh_p * hh_0 * sts_0 - nuh_m * hh0l * sts0l);
-                R Fy = rhs_v - G * id * (s_p1 - s_0) * hv_0 +
-                       id * (advy + dify) - R(0.5) * (rd_0 + rd_p1) * vp0 * hv_0 -
-                       R(0.25) * f_0 * (hh_0 * (u_p1 + u_0) + hh0l * (up1l_ + u0l));
-                vn = (vp0 * hvpc + two_tau * Fy) / hvn_0;
+            // time-level shift with the Robert-Asselin filter (vel_ssh.f90:588-612),
+            // and hh_shift of the U/V depths for the next substep (depth.f90:195-203)
+            const double ts = p.ts;
+            double e[5] = {ts * (sn_0 - 2.0 * s_0 + sp_0) / 2.0, ts * (un - 2.0 * u_0 + up_0) / 2.0,
+                           ts * (vn - 2.0 * v_0 + vp_0) / 2.0, ts * (hun_0 - 2.0 * hu_0 + hupc) / 2.0,
+                           ts * (hvn_0 - 2.0 * hv_0 + hvpc) / 2.0};
+            {
+                ExpCheck ck;
+#pragma unroll
+                for (int k = 0; k < 5; ++k) ck.add(e[k]);
+                quots(e, p.q_dn, ck.any(p.exp_lim));
             }
-            const bool uw = (mb_0 & MB_LCU) && inx && iny;
-            const bool vw = (mb_0 & MB_LCV) && inx && iny;
-            un = uw ? un : R(0);
-            vn = vw ? vn : R(0);
-
-            // time-level shift with the Robert-Asselin filter (vel_ssh.f90:588-612)
-            R s_new = s_0, u_new = u_0, v_new = v_0;
-            double sp_new = sp_0, up_new = up_0, vp_new = vp_0;
-            if (inx1 && n >= 2 && n <= p.ny - 1) {
-                const double ts = p.ts, cts = 0.5 * p.ts / p.dn;
-                if (mb_0 & MB_LU) {
-                    if constexpr (EXACT) {
-                        sp_new = s_0 + ts * (sn_0 - 2.0 * s_0 + sp_0) / 2.0 / p.dn;
-                    } else {
-#pragma clang fp contract(fast)
-                        sp_new = double(s_0) + cts * (sn_0 - 2.0 * double(s_0) + sp_0);
-                    }
-                    s_new = R(sn_0);
-                }
-                if (mb_0 & MB_LCU) {
-                    if constexpr (EXACT) {
-                        up_new = u_0 + ts * (un - 2.0 * u_0 + up_0) / 2.0 / p.dn;
-                    } else {
-#pragma clang fp contract(fast)
-                        up_new = double(u_0) + cts * (double(un) - 2.0 * double(u_0) + up_0);
-                    }
-                    u_new = un;
-                }
-                if (mb_0 & MB_LCV) {
-                    if constexpr (EXACT) {
-                        vp_new = v_0 + ts * (vn - 2.0 * v_0 + vp_0) / 2.0 / p.dn;
-                    } else {
-#pragma clang fp contract(fast)
-                        vp_new = double(v_0) + cts * (double(vn) - 2.0 * double(v_0) + vp_0);
-                    }
-                    v_new = vn;
-                }
-            }
-            o.s = s_new;
-            o.u = u_new;
-            o.v = v_new;
-            o.sp = sp_new;
-            o.up = up_new;
-            o.vp = vp_new;
-            if constexpr (EXACT) {
-                // hh_shift of the U/V depths for the next substep (depth.f90:195-203)
-                const double ts = p.ts;
-                double hu_new = hupc, hv_new = hvpc;
-                if (inx1 && n >= 2 && n <= p.ny - 1) {
-                    if (mb_0 & MB_LLU) hu_new = hu_0 + ts * (hun_0 - 2.0 * hu_0 + hupc) / 2.0 / p.dn;
-                    if (mb_0 & MB_LLV) hv_new = hv_0 + ts * (hvn_0 - 2.0 * hv_0 + hvpc) / 2.0 / p.dn;
-                }
-                o.hu = hu_new;
-                o.hv = hv_new;
-            }
+            const bool sh = inx1 && n >= 2 && n <= p.ny - 1;
+            const bool su = sh && (mb_0 & MB_LU), uu = sh && (mb_0 & MB_LCU), vv = sh && (mb_0 & MB_LCV);
+            o.s = su ? sn_0 : s_0;
+            o.u = uu ? un : u_0;
+            o.v = vv ? vn : v_0;
+            o.sp = su ? s_0 + e[0] : sp_0;
+            o.up = uu ? u_0 + e[1] : up_0;
+            o.vp = vv ? v_0 + e[2] : vp_0;
+            o.hu = sh && (mb_0 & MB_LLU) ? hu_0 + e[3] : hupc;
+            o.hv = sh && (mb_0 & MB_LLV) ? hv_0 + e[4] : hvpc;
         }
 
         // ---- advance the window one row
-        u_m1 = u_0; u_0 = u_p1;
-        v_m1 = v_0; v_0 = v_p1;
+        u_0 = u_p1; v_0 = v_p1;
         s_0 = s_p1; s_p1 = s_p2;
         H_p1 = H_p2;
         up_0 = up_p1; vp_0 = vp_p1; sp_0 = sp_p1; rd_0 = rd_p1;
-        mb_m1 = mb_0; mb_0 = mb_p1; mb_p1 = mb_p2;
-        hq_0 = hq_p1; hq_p1 = hq_p2;
-        hqp_0 = hqp_p1; hqn_0 = hqn_p1;
-        hu_0 = hu_p1; hup_0 = hup_p1;
-        hv_m1 = hv_0; hv_0 = hv_p1;
-        hh_m1 = hh_0;
+        mb_0 = mb_p1; mb_p1 = mb_p2;
+        lu_p1 = lu_p2; lus_0 = lus_p1;
+        w_p1 = w_p2; su_0 = su_p1; wp_0 = wp_p1; wn_0 = wn_p1;
+        hq_p1 = hq_p2;
+        hu_0 = hu_p1; hup_0 = hup_p1; hv_0 = hv_p1;
         sn_0 = sn_p1; hun_0 = hun_p1;
-        stt_0 = stt_p1; bf_0 = bf_p1;
-        sts_m1 = sts_0; vo_m1 = vo_0;
+        qu_0 = qu_p1; qv_0 = qv_p1;
+        V_0 = V_p1; Q_0 = Q_p1; A_0 = A_p1; B_0 = B_p1;
+        T_0 = T_p1; S_m1 = S_0; fy_m1 = fy_0; gy_m1 = gy_0; C_m1 = C_0; E_m1 = E_0;
+        bf_0 = bf_p1;
     }
 };
 
@@ -759,15 +686,21 @@ struct FastStage {
 
 // the march of a mode
 template <typename R, bool EXACT, bool FORM>
-using MarchStage = std::conditional_t<EXACT, Stage<R, true, FORM>, FastStage<R, FORM>>;
+using MarchStage = std::conditional_t<EXACT, ExactStage<FORM>, FastStage<R, FORM>>;
 
 // Loads of one iteration n of a strip (issued one iteration ahead of their
 // use: measured on MI355X at 2048 x 1536, two iterations ahead runs 5 %
 // slower in FP32 and halves FP64's occupancy).
+// A row is the same for the whole wave, so its address is formed by the scalar
+// unit and a lane adds its constant column (the loads of an iteration took 47
+// vector operations for their addresses, now none; 2048 x 1536, us per substep:
+// FP32 35.2 -> 33.4, FP64 48.0 -> 47.7, FP64_EXACT 122 -> 118).  Rows and columns
+// outside the array are clamped into it and their mask bits zeroed: the stages
+// select by them, and no value outside the array reaches an output.
 template <typename R, bool EXACT, bool FROZEN>
 struct Loader {
     const FusedParams &p;
-    const RowAddr ra;
+    const uint32_t col;  // the lane's column, clamped, from 0
     const bool colok;
     struct Pre {
         R s, H, u, v, rd, fx, fy;
@@ -776,13 +709,18 @@ struct Loader {
     } q;
 
     __device__ Loader(const FusedParams &pp, int m)
-        : p(pp), ra{pp.nx, pp.ny, min(max(m, 1), pp.nx)}, colok(m >= 1 && m <= pp.nx)
+        : p(pp), col(min(max(m, 1), pp.nx) - 1), colok(m >= 1 && m <= pp.nx)
     {
     }
-    __device__ __forceinline__ bool rowok(int row) const { return colok && row >= 1 && row <= p.ny; }
     __device__ __forceinline__ double tab(const double *t, int row) const
     {
-        return t[min(max(row, 1), p.ny) - 1];
+        return scalar_load(t + (min(max(row, 1), p.ny) - 1));
+    }
+    // the lane's element of the row that starts at element `row` of the array
+    template <class T>
+    __device__ __forceinline__ T at(const T *base, size_t row) const
+    {
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base + row) + (uint32_t)(col * sizeof(T)));
     }
     __device__ __forceinline__ void issue(int n)  // the loads iteration n consumes
     {
@@ -790,26 +728,27 @@ struct Loader {
         const R *U = static_cast<const R *>(p.u), *V = static_cast<const R *>(p.v);
         const R *RD = static_cast<const R *>(p.rd);
         const R *FX = static_cast<const R *>(p.frx_in), *FY = static_cast<const R *>(p.fry_in);
-        const size_t i2 = ra.at(n + 2), i1 = ra.at(n + 1), i0 = ra.at(n);
-        q.s = S[i2];
-        q.H = Hh[i2];
-        q.mb = p.mb[i2];
-        q.u = U[i1];
-        q.v = V[i1];
-        q.up = p.up[i1];
-        q.vp = p.vp[i1];
-        q.sp = p.sp[i1];
-        q.rd = RD[i1];
+        auto row = [&](int r) { return (size_t)(min(max(r, 1), p.ny) - 1) * (size_t)p.nx; };
+        const size_t r2 = row(n + 2), r1 = row(n + 1), r0 = row(n);
+        q.s = at(S, r2);
+        q.H = at(Hh, r2);
+        q.mb = at(p.mb, r2);
+        q.u = at(U, r1);
+        q.v = at(V, r1);
+        q.up = at(p.up, r1);
+        q.vp = at(p.vp, r1);
+        q.sp = at(p.sp, r1);
+        q.rd = at(RD, r1);
         // per-cell frozen forcing and carried depths of the output row n
         if constexpr (FROZEN) {
-            q.fx = FX[i0];
-            q.fy = FY[i0];
+            q.fx = at(FX, r0);
+            q.fy = at(FY, r0);
         } else {
             q.fx = q.fy = R(0);
         }
         if constexpr (EXACT && FROZEN) {
-            q.hupc = p.hup_c[i0];
-            q.hvpc = p.hvp_c[i0];
+            q.hupc = at(p.hup_c, r0);
+            q.hvpc = at(p.hvp_c, r0);
         } else {
             q.hupc = q.hvpc = 0.0;
         }
@@ -818,46 +757,26 @@ struct Loader {
         q.sy = tab(p.row_sy, n);
         q.wf = tab(p.row_wf, n + 1);
     }
-    // the prefetched values of iteration n, zeroed outside the array (in the
-    // fast modes the mask alone: FastStage selects by it)
+    // the prefetched values of iteration n
     __device__ __forceinline__ void take(int n, StageIn<R> &in) const
     {
-        if constexpr (!EXACT) {
-            in.s2 = q.s;
-            in.H2 = q.H;
-            in.mb2 = rowok(n + 2) ? q.mb : 0;
-            in.u1 = q.u;
-            in.v1 = q.v;
-            in.up1 = q.up;
-            in.vp1 = q.vp;
-            in.sp1 = q.sp;
-            in.rd1 = q.rd;
-            in.fx0 = q.fx;
-            in.fy0 = q.fy;
-            in.f0 = R(q.f);
-            in.sx0 = R(q.sx);
-            in.sy0 = R(q.sy);
-            in.wf1 = R(q.wf);
-            return;
-        }
-        const int k1 = n + 1;
-        in.s2 = rowok(n + 2) ? q.s : R(0);
-        in.H2 = rowok(n + 2) ? q.H : R(0);
-        in.mb2 = rowok(n + 2) ? q.mb : 0;
-        in.u1 = rowok(k1) ? q.u : R(0);
-        in.v1 = rowok(k1) ? q.v : R(0);
-        in.up1 = rowok(k1) ? q.up : 0.0;
-        in.vp1 = rowok(k1) ? q.vp : 0.0;
-        in.sp1 = rowok(k1) ? q.sp : 0.0;
-        in.rd1 = rowok(k1) ? q.rd : R(0);
+        in.s2 = q.s;
+        in.H2 = q.H;
+        in.mb2 = colok && n + 2 >= 1 && n + 2 <= p.ny ? q.mb : 0;
+        in.u1 = q.u;
+        in.v1 = q.v;
+        in.up1 = q.up;
+        in.vp1 = q.vp;
+        in.sp1 = q.sp;
+        in.rd1 = q.rd;
         in.fx0 = q.fx;
         in.fy0 = q.fy;
         in.hupc0 = q.hupc;
         in.hvpc0 = q.hvpc;
-        in.f0 = (n >= 1 && n <= p.ny) ? R(q.f) : R(0);
+        in.f0 = R(q.f);
         in.sx0 = R(q.sx);
         in.sy0 = R(q.sy);
-        in.wf1 = (k1 >= 1 && k1 <= p.ny) ? R(q.wf) : R(0);
+        in.wf1 = R(q.wf);
     }
 };
 
@@ -957,11 +876,8 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
         if (n + 1 < r1 + 2) ld.issue(n + 1);
         const bool keepA = n >= r0 - 2;
         A.row(n, ia, keepA, oa);
-        // A's row n as the 2-launch sequence would have stored it: zero
-        // outside the array, as B's loads would read it
-        const bool okn = !EXACT || (ld.rowok(n) && keepA);
         if (runB) {
-            ib.s2 = okn ? oa.s : R(0);
+            ib.s2 = oa.s;
             ib.H2 = H_d2;
             ib.mb2 = mb_d2;
             ib.u1 = u_prev;
@@ -974,10 +890,10 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
             ib.fy0 = fy_d2;
             ib.hupc0 = hu_d2;
             ib.hvpc0 = hv_d2;
-            ib.f0 = (nb >= 1 && nb <= p.ny) ? R(ld.tab(p.row_f, nb)) : R(0);
+            ib.f0 = R(ld.tab(p.row_f, nb));
             ib.sx0 = R(ld.tab(p.row_sx, nb));
             ib.sy0 = R(ld.tab(p.row_sy, nb));
-            ib.wf1 = (nb + 1 >= 1 && nb + 1 <= p.ny) ? R(ld.tab(p.row_wf, nb + 1)) : R(0);
+            ib.wf1 = R(ld.tab(p.row_wf, nb + 1));
             const bool produce = nb >= r0;
             B.row(nb, ib, produce, ob);
             if (produce && writer && nb <= p.ny) {
@@ -999,17 +915,17 @@ __device__ __forceinline__ void fused_chunk2(const FusedParams &p, int chunk_id,
         H_d2 = H_d1; H_d1 = ia.H2;
         mb_d2 = mb_d1; mb_d1 = ia.mb2;
         rd_d2 = rd_d1; rd_d1 = ia.rd1;
-        fx_d2 = fx_d1; fx_d1 = (!EXACT || keepA) ? oa.rhs_u : R(0);
-        fy_d2 = fy_d1; fy_d1 = (!EXACT || keepA) ? oa.rhs_v : R(0);
+        fx_d2 = fx_d1; fx_d1 = oa.rhs_u;
+        fy_d2 = fy_d1; fy_d1 = oa.rhs_v;
         if constexpr (EXACT) {
-            hu_d2 = hu_d1; hu_d1 = keepA ? oa.hu : 0.0;
-            hv_d2 = hv_d1; hv_d1 = keepA ? oa.hv : 0.0;
+            hu_d2 = hu_d1; hu_d1 = oa.hu;
+            hv_d2 = hv_d1; hv_d1 = oa.hv;
         }
-        u_prev = okn ? oa.u : R(0);
-        v_prev = okn ? oa.v : R(0);
-        up_prev = okn ? oa.up : 0.0;
-        vp_prev = okn ? oa.vp : 0.0;
-        sp_prev = okn ? oa.sp : 0.0;
+        u_prev = oa.u;
+        v_prev = oa.v;
+        up_prev = oa.up;
+        vp_prev = oa.vp;
+        sp_prev = oa.sp;
     }
 }
 

@@ -1,0 +1,60 @@
+"""FP64_EXACT's shared-divisor quotients against the oracle, bit for bit, where
+they could go wrong: states whose numerators lie at the format's limits
+(denormals, the smallest normals, products that underflow, huge values that
+overflow), waves that mix such cells with ordinary ones, divisors that are not
+powers of two (nstep 3, 5, 7), and divisors so small that the step takes IEEE
+divisions throughout."""
+import numpy as np
+import pytest
+
+import oracle
+from _util import STATE, assert_bitwise
+from inmsom_bt import BarotropicModel, make_basin, randomize_state
+from inmsom_bt.ensemble import Ensemble
+
+pytestmark = pytest.mark.gpu
+
+
+def _scaled(kind, shape, seed):
+    """A basin whose fields' magnitudes are drawn over the exponents of `kind`,
+    some cells staying ordinary."""
+    b = randomize_state(make_basin(*shape, seed=seed, sigma=5.0), seed + 1)
+    rng = np.random.default_rng(seed + 2)
+    lo, hi = {"denormal": (-1074, -1000), "tiny": (-1030, -200), "all": (-1074, 0), "huge": (300, 1000),
+              "zeros": (-1074, -1074)}[kind]
+    for f in ("u", "up", "v", "vp", "ssh", "sshp"):
+        a = np.array(getattr(b, f), dtype=np.float64)
+        e = rng.integers(lo, hi + 1, size=a.shape)
+        t = np.ldexp(1.0 + rng.random(a.shape), e) * np.where(rng.random(a.shape) < 0.5, -1.0, 1.0)
+        if kind == "zeros":
+            t = np.where(rng.random(a.shape) < 0.5, -0.0, 0.0)
+        pick = rng.random(a.shape) < (0.02 if kind == "huge" else 0.7)
+        if kind == "huge" and f in ("ssh", "sshp"):
+            continue
+        setattr(b, f, np.where((b.wet > 0) & pick, t, a))
+    return b
+
+
+CASES = [("denormal", (150, 40), 2, 40.0), ("tiny", (130, 37), 3, 40.0), ("all", (61, 50), 5, 40.0),
+         ("zeros", (70, 30), 7, 40.0), ("huge", (64, 30), 2, 40.0), ("tiny", (62, 33), 2, 1e-25)]
+
+
+@pytest.mark.parametrize("kind,shape,nstep,dt", CASES)
+def test_exact_step_at_the_format_limits(kind, shape, nstep, dt):
+    print(f"exact divisions {kind} {shape} nstep={nstep} dt={dt}", flush=True)
+    b = _scaled(kind, shape, seed=61)
+    b.dt = dt
+    with np.errstate(all="ignore"):
+        want = oracle.run(b, 2, nstep, out_steps=[2])[2]
+    with BarotropicModel(b) as m:
+        m.run(2, "fp64_exact", nstep=nstep)
+        got = m.get_state()
+    with Ensemble([b, b], mode="fp64_exact") as ens:
+        ens.run(2, nstep=nstep)
+        member = ens.get_state(1)
+    for f in STATE:  # a NaN's sign and payload are the processor's own
+        for g, what in ((got, "step"), (member, "member")):
+            w, a = np.asarray(want[f]), np.asarray(g[f])
+            assert np.array_equal(np.isnan(w), np.isnan(a)), (what, f)
+            assert_bitwise({f: np.where(np.isnan(a), 0.0, a)}, {f: np.where(np.isnan(w), 0.0, w)}, (f,),
+                           f"{kind} {what}")
