@@ -169,7 +169,7 @@ struct EnsMember {
     void *lvl[2][3] = {};
     double *flt[2][3] = {};
     void *frx = nullptr, *fry = nullptr;
-    double *hup_c = nullptr, *hvp_c = nullptr;
+    double *hup_c[2] = {}, *hvp_c[2] = {};
     double *row_f = nullptr, *row_sx = nullptr, *row_sy = nullptr, *row_wf = nullptr;
     double nu = 0.0;
     int items = 0;
@@ -447,8 +447,11 @@ int build_member(inmsom_bt_ens *e, const inmsom_bt_grid *gr, const inmsom_bt_for
         }
     EHC(hipMalloc(&mb.frx, n * es));
     EHC(hipMalloc(&mb.fry, n * es));
-    EHC(hipMalloc(&mb.hup_c, n * 8));
-    EHC(hipMalloc(&mb.hvp_c, n * 8));
+    if (e->mode == INMSOM_BT_FP64_EXACT)
+        for (int b = 0; b < 2; ++b) {
+            EHC(hipMalloc(&mb.hup_c[b], n * 8));
+            EHC(hipMalloc(&mb.hvp_c[b], n * 8));
+        }
     return INMSOM_BT_OK;
 }
 
@@ -495,8 +498,10 @@ FusedParams member_params(const inmsom_bt_ens *e, const EnsMember &mb, int phase
     p.fry = mb.fry;
     p.frx_in = mb.frx;
     p.fry_in = mb.fry;
-    p.hup_c = mb.hup_c;
-    p.hvp_c = mb.hvp_c;
+    p.hup_in = mb.hup_c[b];
+    p.hvp_in = mb.hvp_c[b];
+    p.hup_c = mb.hup_c[o];
+    p.hvp_c = mb.hvp_c[o];
     step_constants(p);
     return p;
 }
@@ -794,7 +799,8 @@ int inmsom_bt_ens_destroy(inmsom_bt_ens *e)
     if (e->stream) hipStreamSynchronize(e->stream);
     drop_graphs(e);
     for (auto &mb : e->mem) {
-        for (void *q : {(void *)mb.mb, mb.H, mb.rd, mb.frx, mb.fry, (void *)mb.hup_c, (void *)mb.hvp_c,
+        for (void *q : {(void *)mb.mb, mb.H, mb.rd, mb.frx, mb.fry, (void *)mb.hup_c[0], (void *)mb.hup_c[1],
+                        (void *)mb.hvp_c[0], (void *)mb.hvp_c[1],
                         (void *)mb.row_f, (void *)mb.row_sx, (void *)mb.row_sy, (void *)mb.row_wf})
             if (q) hipFree(q);
         for (int b = 0; b < 2; ++b)

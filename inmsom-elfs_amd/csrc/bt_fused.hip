@@ -311,7 +311,7 @@ struct FusedAlloc {
     // overwrite rows another still reads); frc_cur: the set holding it
     void *frx2 = nullptr, *fry2 = nullptr;
     int frc_cur = 0;
-    double *hup_c = nullptr, *hvp_c = nullptr;  // carried filtered depths
+    double *hup_c[2] = {}, *hvp_c[2] = {};  // carried filtered depths (FP64_EXACT), read and written in turn
     int mode = -1;
 };
 static FusedAlloc *falloc(inmsom_bt_ctx *c) { return c->fa; }
@@ -325,7 +325,8 @@ void fused_release(inmsom_bt_ctx *c)
                 if (a->lvl[b][k]) hipFree(a->lvl[b][k]);
                 if (a->flt[b][k]) hipFree(a->flt[b][k]);
             }
-        for (void *q : {a->H, a->rd, a->frx, a->fry, a->frx2, a->fry2, (void *)a->hup_c, (void *)a->hvp_c})
+        for (void *q : {a->H, a->rd, a->frx, a->fry, a->frx2, a->fry2, (void *)a->hup_c[0], (void *)a->hup_c[1],
+                        (void *)a->hvp_c[0], (void *)a->hvp_c[1]})
             if (q) hipFree(q);
         delete a;
         c->fa = nullptr;
@@ -370,8 +371,11 @@ static int fused_load(inmsom_bt_ctx *c, int mode)
         HC(hipMalloc(&a->fry, n * es));
         HC(hipMalloc(&a->frx2, n * es));
         HC(hipMalloc(&a->fry2, n * es));
-        HC(hipMalloc(&a->hup_c, n * 8));
-        HC(hipMalloc(&a->hvp_c, n * 8));
+        if (mode == INMSOM_BT_FP64_EXACT)
+            for (int b = 0; b < 2; ++b) {
+                HC(hipMalloc(&a->hup_c[b], n * 8));
+                HC(hipMalloc(&a->hvp_c[b], n * 8));
+            }
         if (es == 4) {
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->hr, (float *)a->H);
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->rdis, (float *)a->rd);
@@ -550,8 +554,10 @@ static FusedParams make_params(inmsom_bt_ctx *c, FusedAlloc *a, int b, double ta
     p.fry = a->frc_cur ? a->fry2 : a->fry;
     p.frx_in = p.frx;
     p.fry_in = p.fry;
-    p.hup_c = a->hup_c;
-    p.hvp_c = a->hvp_c;
+    p.hup_in = a->hup_c[b];
+    p.hvp_in = a->hvp_c[b];
+    p.hup_c = a->hup_c[1 - b];
+    p.hvp_c = a->hvp_c[1 - b];
     p.cb = c->cb_nl;
     p.eb = c->ebottom;
     p.nu = c->nu;

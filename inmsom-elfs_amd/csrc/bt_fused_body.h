@@ -40,7 +40,11 @@ struct FusedParams {
     int exp_lim;                           // and the limit of ExpCheck
     void *frx, *fry;       // forcing frozen over the substeps of one call (stencil type), written
     const void *frx_in, *fry_in;  // the same, read (a separate buffer when a launch forms new forcing)
-    double *hup_c, *hvp_c; // filtered U/V depths carried between substeps (FP64_EXACT only)
+    // filtered U/V depths carried between substeps (FP64_EXACT only): read, and
+    // written for the next launch (the other buffer: a pair's work items read
+    // them on the rows around their own)
+    const double *hup_in, *hvp_in;
+    double *hup_c, *hvp_c;
 };
 
 // the constants' quotients of the fast modes and FP64_EXACT's divisors, once on
@@ -747,8 +751,8 @@ struct Loader {
             q.fx = q.fy = R(0);
         }
         if constexpr (EXACT && FROZEN) {
-            q.hupc = at(p.hup_c, r0);
-            q.hvpc = at(p.hvp_c, r0);
+            q.hupc = at(p.hup_in, r0);
+            q.hvpc = at(p.hvp_in, r0);
         } else {
             q.hupc = q.hvpc = 0.0;
         }

@@ -58,3 +58,22 @@ def test_exact_step_at_the_format_limits(kind, shape, nstep, dt):
             assert np.array_equal(np.isnan(w), np.isnan(a)), (what, f)
             assert_bitwise({f: np.where(np.isnan(a), 0.0, a)}, {f: np.where(np.isnan(w), 0.0, w)}, (f,),
                            f"{kind} {what}")
+
+
+@pytest.mark.parametrize("shape,nstep,chunk", [((150, 110), 5, 4), ((61, 70), 6, 1), ((300, 64), 7, 3)])
+def test_exact_pairs_carry_depths(shape, nstep, chunk):
+    """Substep pairs past the first read the filtered depths of the rows
+    around their own while other work items write the next ones: two buffers,
+    the oracle's state bit for bit."""
+    print(f"exact pairs {shape} nstep={nstep} chunk={chunk}", flush=True)
+    b = randomize_state(make_basin(*shape, seed=36, sigma=5.0), 11)
+    want = oracle.run(b, 4, nstep, out_steps=[4])[4]
+    with BarotropicModel(b) as m:
+        m.set_launch(chunk)
+        m.set_substeps_per_launch(2)
+        m.run(4, "fp64_exact", nstep=nstep)
+        assert_bitwise(m.get_state(), want, STATE, "step")
+    with Ensemble([b, b], mode="fp64_exact") as ens:
+        ens.set_substeps_per_launch(2)
+        ens.run(4, nstep=nstep)
+        assert_bitwise(ens.get_state(1), want, STATE, "member")
