@@ -14,7 +14,10 @@
 // level it reads uu, vv, uup, vvp, amuv (and pgx, pgy) once, exchanges x
 // neighbours by DPP lane shifts and y neighbours through the thread's own
 // rows or a small LDS exchange between waves, and adds the level's terms
-// times dz to depth sums held in registers.  Every value is formed with the reference's expression and
+// times dz to depth sums held in registers.  A point's eight divisions per
+// level are by its four metrics, whose reciprocals and rests it keeps
+// (bt_exactdiv.h; 2048 x 1536 x 20 levels on MI355X: 1379 us with IEEE
+// divisions, 1249 with these; 7 fields read once take 720).  Every value is formed with the reference's expression and
 // operation order (this file is compiled with -ffp-contract=off), so the
 // result is the reference's bit for bit.  On periodic boundaries the
 // wrapped halo values of the stress, vorticity and bottom-friction arrays
@@ -22,6 +25,7 @@
 // pre-pass fills from their source points.
 #include <string>
 
+#include "bt_exactdiv.h"
 #include "bt_fused_body.h"
 #include "bt_internal.h"
 
@@ -160,7 +164,8 @@ __global__ void k_wrap_halo(F3Params p)
 // Level-independent values of one owned point held in registers; the
 // others (KS_*) live in LDS for the whole call.
 struct Pt {
-    double dxh, dyh, dxt, dyt, hu, hv, hh, hq;
+    Den dxh, dyh, dxt, dyt;
+    double hu, hv, hh, hq;
 };
 enum { KS_DYDX, KS_DXDY, KS_BXY, KS_BYX, KS_DY2, KS_DX2, KS_DXB, KS_DYB, KS_DXB2, KS_DYB2, KS_N };
 
@@ -175,6 +180,7 @@ struct Own {
     uint8_t mbit[R];
     Pt s[R];
     double dxb2_b, hh_b;  // of the point below row 0
+    int exp_lim;          // limit of the numerators' ExpCheck
 };
 
 template <int R, int NW>
@@ -245,14 +251,24 @@ __device__ __forceinline__ void level_terms(const F3Params &p, const Own<R> &o, 
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const Pt &s = o.s[j];
-        a[j] = in.up[j] / s.dyh;
-        b[j] = in.vp[j] / s.dxh;
-        c[j] = in.up[j] / s.dxt;
-        d[j] = in.vp[j] / s.dyt;
-        ev[j] = v[j] * s.dyt;
-        fu[j] = u[j] * s.dxt;
-        A[j] = u[j] * s.dyh * s.hu;  // the transport products u dyh hu, v dxh hv
-        B[j] = v[j] * s.dxh * s.hv;
+        ExpCheck ck;
+        ck.add(in.up[j]);
+        ck.add(in.vp[j]);
+        if (__builtin_expect(ck.any(o.exp_lim), 0)) {
+            a[j] = in.up[j] / s.dyh.b;
+            b[j] = in.vp[j] / s.dxh.b;
+            c[j] = in.up[j] / s.dxt.b;
+            d[j] = in.vp[j] / s.dyt.b;
+        } else {
+            a[j] = quot(in.up[j], s.dyh);
+            b[j] = quot(in.vp[j], s.dxh);
+            c[j] = quot(in.up[j], s.dxt);
+            d[j] = quot(in.vp[j], s.dyt);
+        }
+        ev[j] = v[j] * s.dyt.b;
+        fu[j] = u[j] * s.dxt.b;
+        A[j] = u[j] * s.dyh.b * s.hu;  // the transport products u dyh hu, v dxh hv
+        B[j] = v[j] * s.dxh.b * s.hv;
     }
     // first row: what the wave above needs at n + 1; last row: what the
     // wave below needs at n - 1
@@ -317,11 +333,21 @@ __device__ __forceinline__ void level_terms(const F3Params &p, const Own<R> &o, 
         TV[j] = T2 + xl(T2);
         const double muh_p = (mu[j] + mu_e + mu_n + mu_ne) / 4.0;
         MUM[j] = (mu[j] + mu_e + mu_s + mu_se) / 4.0;
-        PU[j] = (xr(D) - D) / s.dyh;
+        const double pu = xr(D) - D;
         QU[j] = L.ks[KS_DXB2][t] * muh_p * s.hh * ss[j];
         const double muh_mv = (mu[j] + mu_w + mu_n + mu_nw) / 4.0;
         const double dyb2 = L.ks[KS_DYB2][t];
-        QV[j] = (dyb2 * muh_p * s.hh * ss[j] - xl(dyb2) * muh_mv * xl(s.hh) * xl(ss[j])) / s.dyt;
+        const double qv = dyb2 * muh_p * s.hh * ss[j] - xl(dyb2) * muh_mv * xl(s.hh) * xl(ss[j]);
+        ExpCheck ck;
+        ck.add(pu);
+        ck.add(qv);
+        if (__builtin_expect(ck.any(o.exp_lim), 0)) {
+            PU[j] = pu / s.dyh.b;
+            QV[j] = qv / s.dyt.b;
+        } else {
+            PU[j] = quot(pu, s.dyh);
+            QV[j] = quot(qv, s.dyt);
+        }
     }
     L.e1[w][0][lane] = E[0];
     L.e1[w][1][lane] = FYU[R - 1];
@@ -341,11 +367,21 @@ __device__ __forceinline__ void level_terms(const F3Params &p, const Own<R> &o, 
         const double hh_s = j > 0 ? o.s[j - 1].hh : o.hh_b;
         const bool cu = o.in[j] && (o.mbit[j] & MB_LCU), cv = o.in[j] && (o.mbit[j] & MB_LCV);
         const double trU = -(XU[j] - fyU_s) + (T1[j] + T1_s) / 4.0;
-        const double qU = (QU[j] - dxb2_s * MUM[j] * hh_s * ss_s) / s.dxt;
+        const double qu = QU[j] - dxb2_s * MUM[j] * hh_s * ss_s, pv = E_n - E[j];
+        ExpCheck ck;
+        ck.add(qu);
+        ck.add(pv);
+        double qU, pV;
+        if (__builtin_expect(ck.any(o.exp_lim), 0)) {
+            qU = qu / s.dxt.b;
+            pV = pv / s.dxh.b;
+        } else {
+            qU = quot(qu, s.dxt);
+            pV = quot(pv, s.dxh);
+        }
         radv[j] = cu ? trU : 0.0;
         rdfx[j] = cu ? PU[j] + qU : 0.0;
         const double trV = -(XV[j] - fyV_s) - TV[j] / 4.0;
-        const double pV = (E_n - E[j]) / s.dxh;
         rady[j] = cv ? trV : 0.0;
         rdfy[j] = cv ? -pV + QV[j] : 0.0;
     }
@@ -388,6 +424,7 @@ __global__ __launch_bounds__(64 * NW) void k_forcing(F3Params p)
     const int m = 1 + bx * F3_COLS + lane;
     const int n0 = 1 + by * (R * NW - 2) + w * R;
     o.m = m;
+    o.exp_lim = ExpCheck::LIMIT;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const int n = n0 + j, e = w * R + j;  // e: tile row
@@ -413,10 +450,13 @@ __global__ __launch_bounds__(64 * NW) void k_forcing(F3Params p)
             L.ks[KS_DYB][t] = dyb;
             L.ks[KS_DXB2][t] = dxb * dxb;
             L.ks[KS_DYB2][t] = dyb * dyb;
-            s.dxh = g.dxh[i];
-            s.dyh = g.dyh[i];
-            s.dxt = g.dxt[i];
-            s.dyt = g.dyt[i];
+            s.dxh = make_den(g.dxh[i]);
+            s.dyh = make_den(g.dyh[i]);
+            s.dxt = make_den(g.dxt[i]);
+            s.dyt = make_den(g.dyt[i]);
+            bool wide = false;
+            for (const double d : {s.dxh.b, s.dyh.b, s.dxt.b, s.dyt.b}) wide = wide || !(d > DEN_MIN && d < DEN_MAX);
+            if (__any(wide)) o.exp_lim = -1;  // IEEE divisions throughout
             s.hu = p.hhu[i];
             s.hv = p.hhv[i];
             s.hh = p.hhh[i];
@@ -495,8 +535,8 @@ __global__ __launch_bounds__(64 * NW) void k_forcing(F3Params p)
         const double dx = g.dx[i], dy = g.dy[i];
         dxr[j] = dx;
         dyr[j] = dy;
-        G[j] = UB[i] * o.s[j].dxt * o.s[j].dyh * o.s[j].hu;
-        H[j] = VB[i] * o.s[j].dxh * o.s[j].dyt * o.s[j].hv;
+        G[j] = UB[i] * o.s[j].dxt.b * o.s[j].dyh.b * o.s[j].hu;
+        H[j] = VB[i] * o.s[j].dxh.b * o.s[j].dyt.b * o.s[j].hv;
         wx[j] = p.taux[i] * dx * dy;
         wy[j] = p.tauy[i] * dx * dy;
         sl[j] = p.slpr[i];
@@ -536,14 +576,14 @@ __global__ __launch_bounds__(64 * NW) void k_forcing(F3Params p)
         const double ty2 = (mbj & MB_LLV) ? aty[j] : 0.0;
         const double rho0 = g.rho0;
         if (o.in[j] && (mbj & MB_LCU)) {
-            const double sfx = (wx[j] + wx_e) / rho0 / 2.0 / s.dxt / s.dyh;
+            const double sfx = (wx[j] + wx_e) / rho0 / 2.0 / s.dxt.b / s.dyh.b;
             const double bfx = -(bf[j] + bf_e) / 2.0 * p.uup[bot + i];
-            X = X - dfx[j] + tx2 - txd[j] + (sfx + bfx) * s.dxt * s.dyh - (sl_e - sl[j]) * s.hu * s.dyh / rho0;
+            X = X - dfx[j] + tx2 - txd[j] + (sfx + bfx) * s.dxt.b * s.dyh.b - (sl_e - sl[j]) * s.hu * s.dyh.b / rho0;
         }
         if (o.in[j] && (mbj & MB_LCV)) {
-            const double sfy = (wy[j] + wy_n) / rho0 / 2.0 / s.dxh / s.dyt;
+            const double sfy = (wy[j] + wy_n) / rho0 / 2.0 / s.dxh.b / s.dyt.b;
             const double bfy = -(bf[j] + bf_n) / 2.0 * p.vvp[bot + i];
-            Y = Y - dfy[j] + ty2 - tyd[j] + (sfy + bfy) * s.dyt * s.dxh - (sl_n - sl[j]) * s.hv * s.dxh / rho0;
+            Y = Y - dfy[j] + ty2 - tyd[j] + (sfy + bfy) * s.dyt.b * s.dxh.b - (sl_n - sl[j]) * s.hv * s.dxh.b / rho0;
         }
         p.rhsx[i] = X;
         p.rhsy[i] = Y;

@@ -1,5 +1,5 @@
-"""FP64_EXACT's shared-divisor quotients against the oracle, bit for bit, where
-they could go wrong: states whose numerators lie at the format's limits
+"""Shared-divisor quotients (FP64_EXACT, the 3-D forcing) against the oracle, bit
+for bit, where they could go wrong: states whose numerators lie at the format's limits
 (denormals, the smallest normals, products that underflow, huge values that
 overflow), waves that mix such cells with ordinary ones, divisors that are not
 powers of two (nstep 3, 5, 7), and divisors so small that the step takes IEEE
@@ -77,3 +77,29 @@ def test_exact_pairs_carry_depths(shape, nstep, chunk):
         ens.set_substeps_per_launch(2)
         ens.run(4, nstep=nstep)
         assert_bitwise(ens.get_state(1), want, STATE, "member")
+
+
+@pytest.mark.parametrize("lo,hi,frac,scale", [(-1074, -950, 0.7, 1.0), (-600, -100, 0.05, 1.0), (450, 500, 0.01, 1.0),
+                                              (-20, 0, 1.0, 2.0 ** -70)])
+def test_forcing_at_the_format_limits(lo, hi, frac, scale):
+    """Velocities of level n-1 over the exponents lo .. hi at a fraction of the
+    points, and metrics outside the divisors' range."""
+    from test_gpu_forcing3d import _fields
+    print(f"forcing 2^{lo}..2^{hi} at {frac}, metrics x {scale}", flush=True)
+    b = randomize_state(make_basin(131, 45, seed=9, sigma=4.0, metrics="stretched"), 3)
+    f = _fields(b, 5, seed=4)
+    rng = np.random.default_rng(5)
+    for k in ("uup", "vvp", "uup2d", "vvp2d"):
+        t = np.ldexp(1.0 + rng.random(f[k].shape), rng.integers(lo, hi + 1, size=f[k].shape))
+        f[k] = np.where((f[k] != 0.0) & (rng.random(f[k].shape) < frac), np.copysign(t, f[k]), f[k])
+    for k in ("dx", "dy", "dxt", "dyt", "dxh", "dyh", "dxb", "dyb"):
+        setattr(b, k, np.ascontiguousarray(getattr(b, k)) * scale)
+    og = oracle.OracleGrid(b)
+    with np.errstate(all="ignore"):
+        want = oracle.forcing_3d(og, f, b.cb_nl, b.ebottom)
+    with BarotropicModel(b) as m:
+        got = m.forcing_3d(dict(f, taux=b.taux, tauy=b.tauy), f["dz"], f["rhsx2d"], f["rhsy2d"], f["pgx"], f["pgy"])
+    for k in ("rhsx2d", "rhsy2d"):  # a NaN's sign and payload are the processor's own
+        w, g = want[k], got[k]
+        assert np.array_equal(np.isnan(w), np.isnan(g)), k
+        assert_bitwise({k: np.where(np.isnan(g), 0.0, g)}, {k: np.where(np.isnan(w), 0.0, w)}, (k,), f"2^{lo}..2^{hi}")
