@@ -33,7 +33,8 @@
 // (ksw4 > 0, vel_ssh.f90:187-317), which it forms in the same launch.
 // Metrics: per cell (any grid), or per row when every metric and the
 // Coriolis parameter are uniform along x (Cartesian and longitude-latitude
-// grids): then they are read from row tables instead of 8 + 1 arrays.
+// grids): then they are read from row tables instead of 8 + 1 arrays; or one
+// number (uniform metrics), whose quotients the march shares (bt_exactdiv.h).
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -59,8 +60,15 @@ struct DropinParams {
     bool carry_out;                          // write the filtered U/V depths for the next substep
     double *acc[4];                          // ubrtr_i, vbrtr_i, ssh4gradx, ssh4grady, in place
     const double *mu4;                       // the biharmonic viscosity (ksw4 > 0)
-    double g, rho0, ts, tau, ffs, dn, d4n;
+    double g, rho0, ts, tau, ffs;
+    // divisors that every point shares (bt_exactdiv.h): rho0, tau, dfloat(nstep),
+    // 4 nstep and, on uniform metrics, d and d * d; the limit of ExpCheck
+    Den q_rho0, q_tau, q_dn, q_d4n, q_d, q_dd;
+    int exp_lim;
 };
+
+// how the metrics are read: per cell, per row, or one number for all
+enum { MET_CELL = 0, MET_ROW = 1, MET_ONE = 2 };
 
 // What iteration n consumes (outside the array the mask is 0 and the rest
 // whatever the clamped loads give: every use is selected by a mask, or
@@ -87,7 +95,7 @@ struct DOut {
 // One substep marching down the rows of one strip.  Suffixes: m1 = row
 // n-1, 0 = row n, p1 = row n+1, p2 = row n+2.  FIRST: the call's first
 // substep (filtered depths from hh_init, accumulators start at zero).
-template <bool FIRST>
+template <bool FIRST, bool ONE>
 struct DStage {
     const DropinParams &p;
     const bool inx, inx1;
@@ -114,16 +122,51 @@ struct DStage {
     double fv_0 = 0;               // v*hv*dxh on V points (continuity)
     double b_0 = 0, c_0 = 0, h_0 = 0;  // vp/dxh (V), up/dxt and u*dxt (U)
     double fyU_m1 = 0, fyV_m1 = 0;     // fy_p of row n-1 (zonal and meridional equations)
+    int slow = 0;                      // ONE: rows for which the depths take IEEE divisions
 
     __device__ DStage(const DropinParams &pp, int m)
         : p(pp), inx(m >= 3 && m <= pp.nx - 2), inx1(m >= 2 && m <= pp.nx - 1)
     {
     }
 
-    // hh_init / hh_update's average onto a U or V point of two T area
-    // weights, and onto an H point of four (Function/depth.f90:29-66):
-    // (w_a + w_b) / slu / metric_1 / metric_2, slu the number of wet T cells
-    __device__ static double avg(double wsum, double slu, double m1, double m2) { return wsum / slu / m1 / m2; }
+    // hh_init / hh_update's average onto a U or V point of two T area weights,
+    // and onto an H point of four (Function/depth.f90:29-66): (w_a + w_b) / slu /
+    // metric_1 / metric_2, slu the number of wet T cells; here what follows the
+    // first quotient, `mean`
+    __device__ __forceinline__ double avg(double mean, double m1, double m2) const
+    {
+        if constexpr (!ONE) return mean / m1 / m2;
+        double a[1] = {mean};
+        quots2(a, p.q_d, slow > 0);
+        return a[0];
+    }
+    // a[k] / m[k], metrics (ONE: all of them d)
+    template <int N>
+    __device__ __forceinline__ void by_metric(double (&a)[N], const double (&m)[N]) const
+    {
+        if constexpr (ONE) {
+            by(a, p.q_d);
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; ++k) a[k] = a[k] / m[k];
+        }
+    }
+    // a[k] / d, after a look at the numerators; with metrics per row or cell by
+    // IEEE divisions: there the quotients' operands spill (2048 x 1536, us per
+    // substep: rows 187 -> 221, cells 235 -> 633)
+    template <int N>
+    __device__ __forceinline__ void by(double (&a)[N], const Den &d) const
+    {
+        ExpCheck ck;
+        if constexpr (ONE) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) ck.add(a[k]);
+            quots(a, d, ck.any(p.exp_lim));
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; ++k) a[k] = a[k] / d.b;
+        }
+    }
 
     __device__ __forceinline__ void row(int n, const DIn &q, bool produce, DOut &o)
     {
@@ -147,31 +190,37 @@ struct DStage {
         dyt_p1 = q.dyt1;
         const double dxb_0 = q.dxb0, dyb_0 = q.dyb0;
 
-        const double lu_0 = bitf<double>(mb_0, MB_LU), lu_p1 = bitf<double>(mb_p1, MB_LU);
-        const double lu_p2 = bitf<double>(mb_p2, MB_LU);
-        const double lu_0r = xr(lu_0), lu_p1r = xr(lu_p1);
+        const int lu_0 = mb_0 & MB_LU ? 1 : 0, lu_p1 = mb_p1 & MB_LU ? 1 : 0, lu_p2 = mb_p2 & MB_LU ? 1 : 0;
+        const double lf_p1 = lu_p1, lf_p2 = lu_p2;
+        const int lus_0 = lu_0 + xr(lu_0), lus_p1 = lu_p1 + xr(lu_p1);
+        const double in_u = inv_cells(lus_p1), in_v0 = inv_cells(lu_0 + lu_p1);
         const bool iny1 = (k1 >= 3 && k1 <= p.ny - 2);
 
         // ---- depths at level n (hh_init at the first substep, hh_update's
         // results of the previous substep afterwards: both are these
         // averages of hq = H + ssh, depth.f90:21-66, 122-150)
         hq_p2 = H_p2 + s_p2;
-        w_p2 = hq_p2 * dx_p2 * dy_p2 * lu_p2;
+        w_p2 = hq_p2 * dx_p2 * dy_p2 * lf_p2;
+        if constexpr (FIRST) wp_p1 = (H_p1 + sp_p1) * dx_p1 * dy_p1 * lf_p1;  // hh_init's filtered level
+        if constexpr (ONE) {
+            ExpCheck ck;
+            ck.add(w_p2);
+            if (FIRST) ck.add(wp_p1);
+            slow = ck.any(p.exp_lim) ? 4 : slow - 1;
+        }
         {
             const double w1r = xr(w_p1);
-            hu_p1 = (mb_p1 & MB_LLU) ? avg(w_p1 + w1r, lu_p1 + lu_p1r, dxt_p1, dyh_p1) : 0.0;
-            hv_p1 = (mb_p1 & MB_LLV) ? avg(w_p1 + w_p2, lu_p1 + lu_p2, dxh_p1, dyt_p1) : 0.0;
-            const double w0r = xr(w_0);
-            hh_0 = (mb_0 & MB_LUH) ? avg(w_0 + w0r + w_p1 + w1r, lu_0 + lu_0r + lu_p1 + lu_p1r, dxb_0, dyb_0)
-                                   : 0.0;
+            hu_p1 = (mb_p1 & MB_LLU) ? avg((w_p1 + w1r) * in_u, dxt_p1, dyh_p1) : 0.0;
+            hv_p1 = (mb_p1 & MB_LLV) ? avg((w_p1 + w_p2) * inv_cells(lu_p1 + lu_p2), dxh_p1, dyt_p1) : 0.0;
+            const double w0r = xr(w_0), mean = mean_cells(w_0 + w0r + w_p1 + w1r, lus_0 + lus_p1);
+            hh_0 = (mb_0 & MB_LUH) ? avg(mean, dxb_0, dyb_0) : 0.0;
         }
         double hvp_0 = 0.0;
         if constexpr (FIRST) {
             // filtered-level depths of hh_init (depth.f90:22, :32-34, :41-43)
-            const double hqp_p1 = H_p1 + sp_p1;
-            wp_p1 = hqp_p1 * dx_p1 * dy_p1 * lu_p1;
-            hup_p1 = (mb_p1 & MB_LLU) ? avg(wp_p1 + xr(wp_p1), lu_p1 + lu_p1r, dxt_p1, dyh_p1) : 0.0;
-            hvp_0 = (mb_0 & MB_LLV) ? avg(wp_0 + wp_p1, lu_0 + lu_p1, dxh_0, dyt_0) : 0.0;
+            const double wp1r = xr(wp_p1);
+            hup_p1 = (mb_p1 & MB_LLU) ? avg((wp_p1 + wp1r) * in_u, dxt_p1, dyh_p1) : 0.0;
+            hvp_0 = (mb_0 & MB_LLV) ? avg((wp_0 + wp_p1) * in_v0, dxh_0, dyt_0) : 0.0;
         }
 
         // ---- T point of row n+1: continuity (vel_ssh.f90:487-499)
@@ -179,25 +228,40 @@ struct DStage {
         const double fv_p1 = v_p1 * hv_p1 * dxh_p1;
         {
             const bool tw = (mb_p1 & MB_LU) && inx && iny1;
-            const double sn = sp_p1 + 2.0 * tau *
-                                          (q.wf1 / p.rho0 * p.ffs -
-                                           (fu_p1 - xl(fu_p1) + fv_p1 - fv_0) / (dx_p1 * dy_p1));
+            double wf[1] = {q.wf1}, div[1] = {fu_p1 - xl(fu_p1) + fv_p1 - fv_0};
+            by(wf, p.q_rho0);
+            if constexpr (ONE)
+                by(div, p.q_dd);
+            else
+                div[0] = div[0] / (dx_p1 * dy_p1);
+            const double sn = sp_p1 + 2.0 * tau * (wf[0] * p.ffs - div[0]);
             sn_p1 = tw ? sn : 0.0;
         }
         // new-level depths (hh_update, depth.f90:122-150)
         const double hqn_p1 = H_p1 + sn_p1;
-        wn_p1 = hqn_p1 * dx_p1 * dy_p1 * lu_p1;
-        hun_p1 = (mb_p1 & MB_LLU) ? avg(wn_p1 + xr(wn_p1), lu_p1 + lu_p1r, dxt_p1, dyh_p1) : 0.0;
-        const double hvn_0 = (mb_0 & MB_LLV) ? avg(wn_0 + wn_p1, lu_0 + lu_p1, dxh_0, dyt_0) : 0.0;
+        wn_p1 = hqn_p1 * dx_p1 * dy_p1 * lf_p1;
+        if constexpr (ONE) {
+            ExpCheck ck;
+            ck.add(wn_p1);
+            if (ck.any(p.exp_lim)) slow = 4;
+        }
+        const double wn1r = xr(wn_p1);
+        hun_p1 = (mb_p1 & MB_LLU) ? avg((wn_p1 + wn1r) * in_u, dxt_p1, dyh_p1) : 0.0;
+        const double hvn_0 = (mb_0 & MB_LLV) ? avg((wn_0 + wn_p1) * in_v0, dxh_0, dyt_0) : 0.0;
 
         // tension of the filtered level on T points of row n+1 (mixing.f90:129-132)
         // and the two products uv_diff2 takes of it (vel_ssh.f90:146-148, 162-164)
         double P_p1, Px_p1;
+        double ab[2] = {up_p1, vp_p1};
+        by_metric(ab, {dyh_p1, dxh_p1});
+        const double e_0 = ONE ? b_0 : vp_0 / dyt_0, c_p1 = ONE ? ab[0] : up_p1 / dxt_p1;
         {
             const bool tw = (mb_p1 & MB_LU) && inx && iny1;
-            const double a_p1 = up_p1 / dyh_p1;
-            const double b_p1 = vp_p1 / dxh_p1;
-            const double st = dy_p1 / dx_p1 * (a_p1 - xl(a_p1)) - dx_p1 / dy_p1 * (b_p1 - b_0);
+            const double a_p1 = ab[0];
+            const double b_p1 = ab[1];
+            // d / d is 1 on uniform metrics
+            const double yx = ONE ? 1.0 : dy_p1 / dx_p1, xy = ONE ? 1.0 : dx_p1 / dy_p1;
+            const double st = yx * (a_p1 - xl(a_p1)) - xy * (b_p1 - b_0);
             const double stt_p1 = tw ? st : 0.0;
             P_p1 = dy_p1 * dy_p1 * mu_p1 * hq_p1 * stt_p1;
             Px_p1 = dx_p1 * dx_p1 * mu_p1 * hq_p1 * stt_p1;
@@ -212,9 +276,8 @@ struct DStage {
         double sts_0, vo_0;
         {
             const bool hw = (mb_0 & MB_LUU) && inx && (n >= 3 && n <= p.ny - 2);
-            const double c_p1 = up_p1 / dxt_p1;
-            const double e_0 = vp_0 / dyt_0;
-            const double ss = dxb_0 / dyb_0 * (c_p1 - c_0) + dyb_0 / dxb_0 * (xr(e_0) - e_0);
+            const double bxy = ONE ? 1.0 : dxb_0 / dyb_0, byx = ONE ? 1.0 : dyb_0 / dxb_0;
+            const double ss = bxy * (c_p1 - c_0) + byx * (xr(e_0) - e_0);
             const double h_p1 = u_p1 * dxt_p1;
             const double g_0 = v_0 * dyt_0;
             const double vo = (xr(g_0) - g_0) - (h_p1 - h_0) - ((xr(v_0) - v_0) * dyb_0 - (u_p1 - u_0) * dxb_0);
@@ -246,10 +309,34 @@ struct DStage {
             const double fx_m = xl(fx_p);
             const double radv = -(fx_p - fx_m + fyU_0 - fyU_m1) + (Cc_0 + Cc_m1) / 4.0;
             const double muh_m = (mu_0 + xr(mu_0) + mu_m1 + xr(mu_m1)) / 4.0;
-            const double rdfx = (xr(P_0) - P_0) / dyh_0 +
-                                (dxb_0 * dxb_0 * muh_p * hh_0 * sts_0 - dxb_m1 * dxb_m1 * muh_m * hh_m1 * sts_m1) / dxt_0;
-            const double bp = hun_0 * dxt_0 * dyh_0 / 2.0 / tau;
-            const double bp0 = hupc * dxt_0 * dyh_0 / 2.0 / tau;
+            const double muhv_m = (mu_0 + xl(mu_0) + mu_p1 + xl(mu_p1)) / 4.0;
+            const double dybl = xl(dyb_0), hhl = xl(hh_0), stsl = xl(sts_0), P0r = xr(P_0);
+            double rdfx, rdfy, bp, bp0, bq, bq0;
+            if constexpr (ONE) {
+                double df[4] = {P0r - P_0,
+                                dxb_0 * dxb_0 * muh_p * hh_0 * sts_0 - dxb_m1 * dxb_m1 * muh_m * hh_m1 * sts_m1,
+                                Px_p1 - Px_0,
+                                dyb_0 * dyb_0 * muh_p * hh_0 * sts_0 - dybl * dybl * muhv_m * hhl * stsl};
+                double b[4] = {hun_0 * dxt_0 * dyh_0 / 2.0, hupc * dxt_0 * dyh_0 / 2.0, hvn_0 * dyt_0 * dxh_0 / 2.0,
+                               hvpc * dyt_0 * dxh_0 / 2.0};
+                by(df, p.q_d);
+                by(b, p.q_tau);
+                rdfx = df[0] + df[1];
+                rdfy = -df[2] + df[3];
+                bp = b[0];
+                bp0 = b[1];
+                bq = b[2];
+                bq0 = b[3];
+            } else {
+                rdfx = (P0r - P_0) / dyh_0 +
+                       (dxb_0 * dxb_0 * muh_p * hh_0 * sts_0 - dxb_m1 * dxb_m1 * muh_m * hh_m1 * sts_m1) / dxt_0;
+                rdfy = -(Px_p1 - Px_0) / dxh_0 +
+                       (dyb_0 * dyb_0 * muh_p * hh_0 * sts_0 - dybl * dybl * muhv_m * hhl * stsl) / dyt_0;
+                bp = hun_0 * dxt_0 * dyh_0 / 2.0 / tau;
+                bp0 = hupc * dxt_0 * dyh_0 / 2.0 / tau;
+                bq = hvn_0 * dyt_0 * dxh_0 / 2.0 / tau;
+                bq0 = hvpc * dyt_0 * dxh_0 / 2.0 / tau;
+            }
             const double slx = -G * (xr(s_0) - s_0) * dyh_0 * hu_0;
             const double slxn = -G * (xr(sn_0) - sn_0) * dyh_0 * hun_0;
             const double grx = q.rx0 + slx + rdfx + radv - (rd_0 + xr(rd_0)) / 2.0 * up_0 * dxt_0 * dyh_0 * hu_0 +
@@ -261,12 +348,6 @@ struct DStage {
             const double fxV_m = xl(fxV_p);
             const double D = vh * (u_p1 + u_0);
             const double rady = -(fxV_p - fxV_m + fyV_0 - fyV_m1) - (D + xl(D)) / 4.0;
-            const double muhv_m = (mu_0 + xl(mu_0) + mu_p1 + xl(mu_p1)) / 4.0;
-            const double dybl = xl(dyb_0), hhl = xl(hh_0), stsl = xl(sts_0);
-            const double rdfy = -(Px_p1 - Px_0) / dxh_0 +
-                                (dyb_0 * dyb_0 * muh_p * hh_0 * sts_0 - dybl * dybl * muhv_m * hhl * stsl) / dyt_0;
-            const double bq = hvn_0 * dyt_0 * dxh_0 / 2.0 / tau;
-            const double bq0 = hvpc * dyt_0 * dxh_0 / 2.0 / tau;
             const double sly = -G * (s_p1 - s_0) * dxh_0 * hv_0;
             const double slyn = -G * (sn_p1 - sn_0) * dxh_0 * hvn_0;
             const double Gc = fhdd * (u_p1 + u_0);
@@ -282,41 +363,68 @@ struct DStage {
             // averages over the call's substeps (vel_ssh.f90:549-550, 567-568)
             const double a0 = FIRST ? 0.0 : q.a0, a1 = FIRST ? 0.0 : q.a1;
             const double a2 = FIRST ? 0.0 : q.a2, a3 = FIRST ? 0.0 : q.a3;
-            o.a0 = uw ? a0 + (u_0 * hu_0 + un * hun_0) / p.d4n : a0;
-            o.a2 = uw ? a2 + (slx + slxn) / p.d4n : a2;
-            o.a1 = vw ? a1 + (v_0 * hv_0 + vn * hvn_0) / p.d4n : a1;
-            o.a3 = vw ? a3 + (sly + slyn) / p.d4n : a3;
+            if constexpr (ONE) {
+                double t[4] = {u_0 * hu_0 + un * hun_0, v_0 * hv_0 + vn * hvn_0, slx + slxn, sly + slyn};
+                by(t, p.q_d4n);
+                o.a0 = uw ? a0 + t[0] : a0;
+                o.a1 = vw ? a1 + t[1] : a1;
+                o.a2 = uw ? a2 + t[2] : a2;
+                o.a3 = vw ? a3 + t[3] : a3;
+            } else {
+                o.a0 = uw ? a0 + (u_0 * hu_0 + un * hun_0) / p.q_d4n.b : a0;
+                o.a2 = uw ? a2 + (slx + slxn) / p.q_d4n.b : a2;
+                o.a1 = vw ? a1 + (v_0 * hv_0 + vn * hvn_0) / p.q_d4n.b : a1;
+                o.a3 = vw ? a3 + (sly + slyn) / p.q_d4n.b : a3;
+            }
 
             // time-level shift with the Robert-Asselin filter (vel_ssh.f90:588-612)
             // and hh_shift of the U/V depths (depth.f90:195-203)
-            double s_new = s_0, u_new = u_0, v_new = v_0;
-            double sp_new = sp_0, up_new = up_0, vp_new = vp_0;
-            double hu_new = hupc, hv_new = hvpc;
-            if (inx1 && n >= 2 && n <= p.ny - 1) {
-                const double ts = p.ts;
-                if (mb_0 & MB_LU) {
-                    sp_new = s_0 + ts * (sn_0 - 2.0 * s_0 + sp_0) / 2.0 / p.dn;
-                    s_new = sn_0;
+            const double ts = p.ts;
+            if constexpr (ONE) {
+                double e[5] = {ts * (sn_0 - 2.0 * s_0 + sp_0) / 2.0, ts * (un - 2.0 * u_0 + up_0) / 2.0,
+                               ts * (vn - 2.0 * v_0 + vp_0) / 2.0, ts * (hun_0 - 2.0 * hu_0 + hupc) / 2.0,
+                               ts * (hvn_0 - 2.0 * hv_0 + hvpc) / 2.0};
+                by(e, p.q_dn);
+                const bool sh = inx1 && n >= 2 && n <= p.ny - 1;
+                const bool bs = sh && (mb_0 & MB_LU), bu = sh && (mb_0 & MB_LCU), bv = sh && (mb_0 & MB_LCV);
+                o.s = bs ? sn_0 : s_0;
+                o.u = bu ? un : u_0;
+                o.v = bv ? vn : v_0;
+                o.sp = bs ? s_0 + e[0] : sp_0;
+                o.up = bu ? u_0 + e[1] : up_0;
+                o.vp = bv ? v_0 + e[2] : vp_0;
+                o.hu = sh && (mb_0 & MB_LLU) ? hu_0 + e[3] : hupc;
+                o.hv = sh && (mb_0 & MB_LLV) ? hv_0 + e[4] : hvpc;
+            } else {
+                double s_new = s_0, u_new = u_0, v_new = v_0;
+                double sp_new = sp_0, up_new = up_0, vp_new = vp_0;
+                double hu_new = hupc, hv_new = hvpc;
+                const double dn = p.q_dn.b;
+                if (inx1 && n >= 2 && n <= p.ny - 1) {
+                    if (mb_0 & MB_LU) {
+                        sp_new = s_0 + ts * (sn_0 - 2.0 * s_0 + sp_0) / 2.0 / dn;
+                        s_new = sn_0;
+                    }
+                    if (mb_0 & MB_LCU) {
+                        up_new = u_0 + ts * (un - 2.0 * u_0 + up_0) / 2.0 / dn;
+                        u_new = un;
+                    }
+                    if (mb_0 & MB_LCV) {
+                        vp_new = v_0 + ts * (vn - 2.0 * v_0 + vp_0) / 2.0 / dn;
+                        v_new = vn;
+                    }
+                    if (mb_0 & MB_LLU) hu_new = hu_0 + ts * (hun_0 - 2.0 * hu_0 + hupc) / 2.0 / dn;
+                    if (mb_0 & MB_LLV) hv_new = hv_0 + ts * (hvn_0 - 2.0 * hv_0 + hvpc) / 2.0 / dn;
                 }
-                if (mb_0 & MB_LCU) {
-                    up_new = u_0 + ts * (un - 2.0 * u_0 + up_0) / 2.0 / p.dn;
-                    u_new = un;
-                }
-                if (mb_0 & MB_LCV) {
-                    vp_new = v_0 + ts * (vn - 2.0 * v_0 + vp_0) / 2.0 / p.dn;
-                    v_new = vn;
-                }
-                if (mb_0 & MB_LLU) hu_new = hu_0 + ts * (hun_0 - 2.0 * hu_0 + hupc) / 2.0 / p.dn;
-                if (mb_0 & MB_LLV) hv_new = hv_0 + ts * (hvn_0 - 2.0 * hv_0 + hvpc) / 2.0 / p.dn;
+                o.s = s_new;
+                o.u = u_new;
+                o.v = v_new;
+                o.sp = sp_new;
+                o.up = up_new;
+                o.vp = vp_new;
+                o.hu = hu_new;
+                o.hv = hv_new;
             }
-            o.s = s_new;
-            o.u = u_new;
-            o.v = v_new;
-            o.sp = sp_new;
-            o.up = up_new;
-            o.vp = vp_new;
-            o.hu = hu_new;
-            o.hv = hv_new;
         }
 
         // ---- advance the window one row
@@ -366,11 +474,12 @@ struct DStage {
     }
 };
 
-// Loads of one iteration, issued one iteration ahead of their use.
-template <bool FIRST, bool ROWMET>
+// Loads of one iteration, issued one iteration ahead of their use.  As the fused step's Loader: a row's address by the scalar unit, a lane's
+// constant column added to it.
+template <bool FIRST, int MET>
 struct DLoader {
     const DropinParams &p;
-    const RowAddr ra;
+    const uint32_t col;  // the lane's column, clamped, from 0
     const bool colok;
     struct Pre {
         double s, H, dx, dy, u, v, up, vp, sp, rd, mu, wf, dxt, dyh, dxh, dyt, f, rx, ry, dxb, dyb, hupc, hvpc;
@@ -379,34 +488,49 @@ struct DLoader {
     } q;
 
     __device__ DLoader(const DropinParams &pp, int m)
-        : p(pp), ra{pp.nx, pp.ny, min(max(m, 1), pp.nx)}, colok(m >= 1 && m <= pp.nx)
+        : p(pp), col(min(max(m, 1), pp.nx) - 1), colok(m >= 1 && m <= pp.nx)
     {
     }
     __device__ __forceinline__ bool rowok(int row) const { return colok && row >= 1 && row <= p.ny; }
-    // metric k (0..7: dx dy dxt dyt dxh dyh dxb dyb; 8: rlh_s) at (this column, row)
+    // the lane's element of the row whose index row_of gave
+    template <class T>
+    __device__ __forceinline__ T at(const T *base, size_t row) const
+    {
+        if constexpr (MET == MET_CELL) return base[row];
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base + row) + (uint32_t)(col * sizeof(T)));
+    }
+    // metric k (0..7: dx dy dxt dyt dxh dyh dxb dyb; 8: rlh_s) at (this column,
+    // row), whose cells start at element i
     __device__ __forceinline__ double met(int k, int row, size_t i) const
     {
-        if constexpr (ROWMET)
+        if (MET == MET_ONE && k < 8) return p.q_d.b;
+        if constexpr (MET != MET_CELL)
             return scalar_load(p.met[k] + min(max(row, 1), p.ny) - 1);
         else
-            return p.met[k][i];
+            return at(p.met[k], i);
+    }
+    // first element of a row, or (MET_CELL) the lane's own element of it: there
+    // nine more arrays' scalar addresses spill (235 us a substep -> 547)
+    __device__ __forceinline__ size_t row_of(int r) const
+    {
+        return (size_t)(min(max(r, 1), p.ny) - 1) * (size_t)p.nx + (MET == MET_CELL ? col : 0u);
     }
     __device__ __forceinline__ void issue(int n)
     {
-        const size_t i2 = ra.at(n + 2), i1 = ra.at(n + 1), i0 = ra.at(n);
-        q.s = p.s[i2];
-        q.H = p.H[i2];
-        q.mb = p.mb[i2];
+        const size_t i2 = row_of(n + 2), i1 = row_of(n + 1), i0 = row_of(n);
+        q.s = at(p.s, i2);
+        q.H = at(p.H, i2);
+        q.mb = at(p.mb, i2);
         q.dx = met(0, n + 2, i2);
         q.dy = met(1, n + 2, i2);
-        q.u = p.u[i1];
-        q.v = p.v[i1];
-        q.up = p.up[i1];
-        q.vp = p.vp[i1];
-        q.sp = p.sp[i1];
-        q.rd = p.rd[i1];
-        q.mu = p.mu[i1];
-        q.wf = p.wf[i1];
+        q.u = at(p.u, i1);
+        q.v = at(p.v, i1);
+        q.up = at(p.up, i1);
+        q.vp = at(p.vp, i1);
+        q.sp = at(p.sp, i1);
+        q.rd = at(p.rd, i1);
+        q.mu = at(p.mu, i1);
+        q.wf = at(p.wf, i1);
         q.dxt = met(2, n + 1, i1);
         q.dyt = met(3, n + 1, i1);
         q.dxh = met(4, n + 1, i1);
@@ -414,12 +538,12 @@ struct DLoader {
         q.dxb = met(6, n, i0);
         q.dyb = met(7, n, i0);
         q.f = met(8, n, i0);
-        q.rx = p.rx[i0];
-        q.ry = p.ry[i0];
+        q.rx = at(p.rx, i0);
+        q.ry = at(p.ry, i0);
         if constexpr (!FIRST) {
-            q.hupc = p.hupc[i0];
-            q.hvpc = p.hvpc[i0];
-            for (int k = 0; k < 4; ++k) q.a[k] = p.acc[k][i0];
+            q.hupc = at((const double *)p.hupc, i0);
+            q.hvpc = at((const double *)p.hvpc, i0);
+            for (int k = 0; k < 4; ++k) q.a[k] = at((const double *)p.acc[k], i0);
         }
     }
     __device__ __forceinline__ void take(int n, DIn &in) const
@@ -459,11 +583,13 @@ struct DLoader {
     }
 };
 
-// Two waves per SIMD (with the row metrics by the scalar unit 211 VGPRs; from
-// vector loads, and zeroed by lane outside the array, they took 256 and spilled
-// 12 bytes per lane).  At 2048 x 1536 on MI355X a call of 4 launches takes
-// 0.768 ms (0.782); bound by FP64 issue, 44 IEEE divisions a point.
-template <bool FIRST, bool ROWMET>
+// Two waves per SIMD.  Measured on MI355X, us per substep before (metrics per row
+// or cell, 44 IEEE divisions a point) / now: one metric (MET_ONE: two IEEE
+// divisions, the others by d, tau, rho0 and the numbers of substeps from their
+// reciprocals) 700 x 600 37.6 / 29.4, 1300 x 1000 81 / 71, 2048 x 1536 187 / 177,
+// where its 224 bytes a cell take 144; per row (depth means by products, scalar row
+// addresses) 38.0 / 36.5, 81 / 78.6, 186 / 183; per cell unchanged.
+template <bool FIRST, int MET>
 __global__ void __launch_bounds__(WAVE, 2) k_dropin(DropinParams p)
 {
     const int w = blockIdx.x;
@@ -477,8 +603,8 @@ __global__ void __launch_bounds__(WAVE, 2) k_dropin(DropinParams p)
     const int r0 = chunk_id * p.chunk + 1;
     const int r1 = min(r0 + p.chunk, p.ny + 1);
 
-    DStage<FIRST> st(p, m);
-    DLoader<FIRST, ROWMET> ld(p, m);
+    DStage<FIRST, MET == MET_ONE> st(p, m);
+    DLoader<FIRST, MET> ld(p, m);
     DIn in;
     DOut o;
     ld.issue(r0 - 3);
@@ -763,18 +889,18 @@ __global__ void __launch_bounds__(WAVE * DT_MAX_ROWS) k_dropin_tile(DropinParams
         p.cvp[io] = vp;
         p.csp[io] = sp;
     }
-    p.acc[0][io] = uw ? a0 + (u * hu + un * hun) / p.d4n : a0;
-    p.acc[2][io] = uw ? a2 + (slx + slxn) / p.d4n : a2;
-    p.acc[1][io] = vw ? a1 + (v * hv + vn * hvn) / p.d4n : a1;
-    p.acc[3][io] = vw ? a3 + (sly + slyn) / p.d4n : a3;
+    p.acc[0][io] = uw ? a0 + (u * hu + un * hun) / p.q_d4n.b : a0;
+    p.acc[2][io] = uw ? a2 + (slx + slxn) / p.q_d4n.b : a2;
+    p.acc[1][io] = vw ? a1 + (v * hv + vn * hvn) / p.q_d4n.b : a1;
+    p.acc[3][io] = vw ? a3 + (sly + slyn) / p.q_d4n.b : a3;
     if (!p.uo) return;
     const double ts = p.ts;
     const bool sh_ = m >= 2 && m <= p.nx - 1 && n >= 2 && n <= p.ny - 1;
-    const double spn = s + ts * (sn - 2.0 * s + sp) / 2.0 / p.dn;
-    const double upn = u + ts * (un - 2.0 * u + up) / 2.0 / p.dn;
-    const double vpn = v + ts * (vn - 2.0 * v + vp) / 2.0 / p.dn;
-    const double hupn = hu + ts * (hun - 2.0 * hu + hupc) / 2.0 / p.dn;
-    const double hvpn = hv + ts * (hvn - 2.0 * hv + hvpc) / 2.0 / p.dn;
+    const double spn = s + ts * (sn - 2.0 * s + sp) / 2.0 / p.q_dn.b;
+    const double upn = u + ts * (un - 2.0 * u + up) / 2.0 / p.q_dn.b;
+    const double vpn = v + ts * (vn - 2.0 * v + vp) / 2.0 / p.q_dn.b;
+    const double hupn = hu + ts * (hun - 2.0 * hu + hupc) / 2.0 / p.q_dn.b;
+    const double hvpn = hv + ts * (hvn - 2.0 * hv + hvpc) / 2.0 / p.q_dn.b;
     const bool bs = sh_ && (mb & MB_LU), bu = sh_ && (mb & MB_LCU), bv = sh_ && (mb & MB_LCV);
     p.so[io] = bs ? sn : s;
     p.spo[io] = bs ? spn : sp;
@@ -930,7 +1056,7 @@ int check_grid(inmsom_bt_ctx *c, DropinAlloc *a)
     int dev = 0, cus = 0, per_cu = 0;
     DHC(hipGetDevice(&dev));
     DHC(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const void *kf = rows ? (const void *)k_dropin<false, true> : (const void *)k_dropin<false, false>;
+    const void *kf = rows ? (const void *)k_dropin<false, MET_ROW> : (const void *)k_dropin<false, MET_CELL>;
     DHC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kf, WAVE, 0));
     a->slots = (long long)cus * (per_cu > 0 ? per_cu : 1);
     const int strips = (nx + SW - 1) / SW;
@@ -955,10 +1081,12 @@ int ensure_buffers(inmsom_bt_ctx *c, DropinAlloc *a)
 }
 
 template <bool FIRST>
-void launch_dropin(inmsom_bt_ctx *c, const DropinParams &p, bool rowmet)
+void launch_dropin(inmsom_bt_ctx *c, const DropinParams &p, int met)
 {
     dim3 grid((unsigned)(p.per_xcd * NXCD)), blk(WAVE);
-    const void *k = rowmet ? (const void *)k_dropin<FIRST, true> : (const void *)k_dropin<FIRST, false>;
+    const void *k = met == MET_ONE   ? (const void *)k_dropin<FIRST, MET_ONE>
+                    : met == MET_ROW ? (const void *)k_dropin<FIRST, MET_ROW>
+                                     : (const void *)k_dropin<FIRST, MET_CELL>;
     void *args[] = {const_cast<DropinParams *>(&p)};
     (void)hipLaunchKernel(k, grid, blk, args, 0, c->stream);
 }
@@ -1042,8 +1170,19 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
     p.ts = c->g.ts;
     p.tau = tau / (double)nstep;  // tau_inner, vel_ssh.f90:465
     p.ffs = (double)c->g.ffs;
-    p.dn = (double)nstep;
-    p.d4n = (double)(4 * nstep);
+    const double dn = (double)nstep, d4n = (double)(4 * nstep);
+    p.q_rho0 = make_den(p.rho0);
+    p.q_tau = make_den(p.tau);
+    p.q_dn = make_den(dn);
+    p.q_d4n = make_den(d4n);
+    p.exp_lim = ExpCheck::LIMIT;
+    for (const double d : {p.rho0, p.tau, dn, d4n})
+        if (!(d > DEN_MIN && d < DEN_MAX)) p.exp_lim = -1;  // IEEE divisions throughout
+    const bool one = a->rowmet_ok && c->uniform_metrics && c->metric0 > DEN_MIN && c->metric0 < DEN_MAX;
+    if (one) {
+        p.q_d = make_den(c->metric0);
+        p.q_dd = make_den(c->metric0 * c->metric0);
+    }
     if (ksw4 > 0) {
         if (!mu4) {
             set_error("mu4 is required when ksw4 > 0");
@@ -1057,6 +1196,7 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
         p.total = p.strips * p.nchunks;
         p.per_xcd = (p.total + NXCD - 1) / NXCD;
     }
+    const int met = one ? MET_ONE : a->rowmet_ok ? MET_ROW : MET_CELL;
     const int last = 2 * nstep;
     for (int k = 1; k <= last; ++k) {
         // substep k reads the caller's state (k = 1) or the buffer substep
@@ -1092,9 +1232,9 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
             (void)hipLaunchKernel(tile_kernel(a->rowmet_ok, ksw4 > 0), dim3((unsigned)(p.per_xcd * NXCD)),
                                   dim3((unsigned)(WAVE * tile_nr)), args, dropin_tile_lds(tile_nr), c->stream);
         } else if (k == 1)
-            launch_dropin<true>(c, p, a->rowmet_ok);
+            launch_dropin<true>(c, p, met);
         else
-            launch_dropin<false>(c, p, a->rowmet_ok);
+            launch_dropin<false>(c, p, met);
     }
     DHC(hipGetLastError());
     return INMSOM_BT_OK;

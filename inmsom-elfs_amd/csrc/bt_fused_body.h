@@ -204,6 +204,20 @@ struct StageOut {
     double hu, hv;
 };
 
+// 1 / n of a depth average over n = 1, 2 or 4 cells, whose product is the
+// quotient (n = 0: not a number, as 0 / 0)
+__device__ __forceinline__ double inv_cells(int n)
+{
+    return n == 4 ? 0.25 : n == 2 ? 0.5 : n == 0 ? __builtin_inf() : 1.0;
+}
+// sum / n for n of 4 cells; the division by 3 only in a wave that has one
+__device__ __forceinline__ double mean_cells(double sum, int n)
+{
+    double mean = sum * inv_cells(n);
+    if (__any(n == 3)) mean = n == 3 ? sum / 3.0 : mean;
+    return mean;
+}
+
 // One leap-frog substep of FP64_EXACT marching down the rows of one strip: the
 // rolling register window (suffix m1 = row n-1, 0 = row n, p1 = n+1, p2 = n+2)
 // of input rows and of T-, U-, V- and H-point terms.  row(n) takes the inputs
@@ -256,13 +270,6 @@ struct ExactStage {
     {
     }
 
-    // 1 / n of a depth average over n = 1, 2 or 4 cells (n = 3: the quotient,
-    // n = 0: not a number, as 0 / 0)
-    static __device__ __forceinline__ double inv_cells(int n)
-    {
-        return n == 4 ? 0.25 : n == 2 ? 0.5 : n == 0 ? __builtin_inf() : 1.0;
-    }
-
     __device__ __forceinline__ void row(int n, const StageIn<double> &q, bool produce, StageOut<double> &o)
     {
         const double d = p.d, tau = p.tau, nu = p.nu;
@@ -296,9 +303,7 @@ struct ExactStage {
             if (FORM) ck.add(wp_p1);
             slow = ck.any(p.exp_lim) ? 4 : slow - 1;
             const int nh = lus_0 + lus_p1;
-            const double sum4 = (su_0 + w_p1) + xr(w_p1);
-            double mean4 = sum4 * inv_cells(nh);
-            if (__any(nh == 3)) mean4 = nh == 3 ? sum4 / 3.0 : mean4;
+            const double mean4 = mean_cells((su_0 + w_p1) + xr(w_p1), nh);
             double a[3] = {su_p1 * inv_cells(lus_p1), (w_p1 + w_p2) * inv_cells(lu_p1 + lu_p2), mean4};
             quots2(a, p.q_d, slow > 0);
             hu_p1 = (mb_p1 & MB_LLU) ? a[0] : 0.0;

@@ -1,4 +1,4 @@
-"""Shared-divisor quotients (FP64_EXACT, the 3-D forcing) against the oracle, bit
+"""Shared-divisor quotients (FP64_EXACT, the drop-in, the 3-D forcing) against the oracle, bit
 for bit, where they could go wrong: states whose numerators lie at the format's limits
 (denormals, the smallest normals, products that underflow, huge values that
 overflow), waves that mix such cells with ordinary ones, divisors that are not
@@ -103,3 +103,30 @@ def test_forcing_at_the_format_limits(lo, hi, frac, scale):
         w, g = want[k], got[k]
         assert np.array_equal(np.isnan(w), np.isnan(g)), k
         assert_bitwise({k: np.where(np.isnan(g), 0.0, g)}, {k: np.where(np.isnan(w), 0.0, w)}, (k,), f"2^{lo}..2^{hi}")
+
+
+@pytest.mark.parametrize("kind,nstep,dt", [("all", 3, 40.0), ("zeros", 2, 40.0), ("tiny", 1, 1e-25)])
+def test_dropin_march_at_the_format_limits(kind, nstep, dt):
+    """barotropic_dynamics on uniform metrics, a grid of the march's size."""
+    print(f"drop-in march {kind} nstep={nstep} dt={dt}", flush=True)
+    b = _scaled(kind, (700, 590), seed=71)
+    og = oracle.OracleGrid(b)
+    rd = og.rayleigh()
+    rng = np.random.default_rng(6)
+    rx, ry = rng.standard_normal((2, b.ny, b.nx)) * 1e3
+    wf = rng.standard_normal((b.ny, b.nx)) * 1e-5
+    acc = ("ubrtr_i", "vbrtr_i", "ssh4gradx", "ssh4grady")
+    st = {k: np.ascontiguousarray(getattr(b, k)).copy() for k in ("u", "up", "v", "vp", "ssh", "sshp")}
+    want, wacc = {k: v.copy() for k, v in st.items()}, {k: np.zeros_like(rx) for k in acc}
+    with np.errstate(all="ignore"):
+        oracle.barotropic_dynamics(og, dt, nstep, 0, want, wacc, rx, ry, wf, b.mu, b.mu4, rd)
+    gacc = {k: np.zeros_like(rx) for k in acc}
+    with BarotropicModel(b, rdis=rd) as m:
+        m.barotropic_dynamics(dt, nstep, 0, *(st[k] for k in st), *(gacc[k] for k in acc), rx, ry, wf,
+                              np.ascontiguousarray(b.mu), np.ascontiguousarray(b.mu4), rd)
+    want.update(wacc)
+    st.update(gacc)
+    for k in want:  # a NaN's sign and payload are the processor's own
+        w, g = want[k], st[k]
+        assert np.array_equal(np.isnan(w), np.isnan(g)), k
+        assert_bitwise({k: np.where(np.isnan(g), 0.0, g)}, {k: np.where(np.isnan(w), 0.0, w)}, (k,), kind)
