@@ -317,6 +317,7 @@ int inmsom_bt_finalize(inmsom_bt_ctx *c)
     if (!c) return INMSOM_BT_OK;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
+    host_copy_release(c->hc);
     fused_release(c);
     dropin_release(c);
     auto fr = [](void *p) {
@@ -424,13 +425,11 @@ int inmsom_bt_barotropic_dynamics(inmsom_bt_ctx *c, double tau, int nstep, int k
     TRY(upload(c, c->bot_y, rdis, bd));
     TRY(dynamics_on_context(c, tau, nstep, ksw4, c->rhsx, c->rhsy, c->surf_x, c->surf_y, c->bot_x, c->bot_y));
     double *st_out[6] = {ubrtr_e, ubrtrp_e, vbrtr_e, vbrtrp_e, ssh_e, sshp_e};
-    for (int k = 0; k < 6; ++k)
-        HIPCHECK(hipMemcpyAsync(st_out[k], c->st[k], bd, hipMemcpyDeviceToHost, c->stream));
     double *acc_out[4] = {ubrtr_i, vbrtr_i, ssh4gradx, ssh4grady};
-    for (int k = 0; k < 4; ++k)
-        HIPCHECK(hipMemcpyAsync(acc_out[k], c->acc[k], bd, hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    return INMSOM_BT_OK;
+    HostPart parts[10];
+    for (int k = 0; k < 6; ++k) parts[k] = {st_out[k], c->st[k], c->n, false};
+    for (int k = 0; k < 4; ++k) parts[6 + k] = {acc_out[k], c->acc[k], c->n, false};
+    return host_copy(c->device, c->stream, c->hc, parts, 10);
 }
 
 int inmsom_bt_barotropic_dynamics_dev(inmsom_bt_ctx *c, double tau, int nstep, int ksw4,
@@ -661,11 +660,9 @@ int inmsom_bt_get_state(inmsom_bt_ctx *c, double *u, double *up, double *v, doub
     HIPCHECK(hipSetDevice(c->device));
     TRY(fused_flush(c));
     double *out[6] = {u, up, v, vp, ssh, sshp};
-    for (int k = 0; k < 6; ++k)
-        HIPCHECK(hipMemcpyAsync(out[k], c->st[k], c->n * sizeof(double), hipMemcpyDeviceToHost,
-                                c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    return INMSOM_BT_OK;
+    HostPart parts[6];
+    for (int k = 0; k < 6; ++k) parts[k] = {out[k], c->st[k], c->n, false};
+    return host_copy(c->device, c->stream, c->hc, parts, 6);
 }
 
 int inmsom_bt_get_means(inmsom_bt_ctx *c, double *ubrtr_i, double *vbrtr_i, double *ssh4gradx,
@@ -674,11 +671,9 @@ int inmsom_bt_get_means(inmsom_bt_ctx *c, double *ubrtr_i, double *vbrtr_i, doub
     REQUIRE(c && ubrtr_i && vbrtr_i && ssh4gradx && ssh4grady, "null pointer");
     HIPCHECK(hipSetDevice(c->device));
     double *out[4] = {ubrtr_i, vbrtr_i, ssh4gradx, ssh4grady};
-    for (int k = 0; k < 4; ++k)
-        HIPCHECK(hipMemcpyAsync(out[k], c->acc[k], c->n * sizeof(double), hipMemcpyDeviceToHost,
-                                c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    return INMSOM_BT_OK;
+    HostPart parts[4];
+    for (int k = 0; k < 4; ++k) parts[k] = {out[k], c->acc[k], c->n, false};
+    return host_copy(c->device, c->stream, c->hc, parts, 4);
 }
 
 int inmsom_bt_model_steps(inmsom_bt_ctx *c, double tau, int nstep, int ksw4, int nsteps)

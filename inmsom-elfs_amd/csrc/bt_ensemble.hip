@@ -178,6 +178,7 @@ struct EnsMember {
 struct inmsom_bt_ens {
     int device = 0;
     hipStream_t stream = nullptr;
+    ibt::HostCopy hc;  // pinned slots of large copies to the host
     int mode = INMSOM_BT_FP32;
     double g = 9.81, rho0 = 1025.0, ts = 0.05, cb = 2.5e-3, eb = 25e-4, ffs = 1.0;
     std::vector<EnsMember> mem;
@@ -798,6 +799,7 @@ int inmsom_bt_ens_destroy(inmsom_bt_ens *e)
     hipSetDevice(e->device);
     if (e->stream) hipStreamSynchronize(e->stream);
     drop_graphs(e);
+    host_copy_release(e->hc);
     for (auto &mb : e->mem) {
         for (void *q : {(void *)mb.mb, mb.H, mb.rd, mb.frx, mb.fry, (void *)mb.hup_c[0], (void *)mb.hup_c[1],
                         (void *)mb.hvp_c[0], (void *)mb.hvp_c[1],
@@ -875,17 +877,12 @@ int inmsom_bt_ens_get_state(inmsom_bt_ens *e, int k, double *u, double *up, doub
     EnsMember &mb = e->mem[k];
     double *lv[3] = {u, v, ssh}, *fl[3] = {up, vp, sshp};
     const int b = e->phase;
+    HostPart parts[6];
     for (int q = 0; q < 3; ++q) {
-        if (e->mode == INMSOM_BT_FP32) {
-            std::vector<float> t(mb.n);
-            EHC(hipMemcpy(t.data(), mb.lvl[b][q], mb.n * 4, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < mb.n; ++i) lv[q][i] = (double)t[i];
-        } else {
-            EHC(hipMemcpy(lv[q], mb.lvl[b][q], mb.n * 8, hipMemcpyDeviceToHost));
-        }
-        EHC(hipMemcpy(fl[q], mb.flt[b][q], mb.n * 8, hipMemcpyDeviceToHost));
+        parts[2 * q] = {lv[q], mb.lvl[b][q], mb.n, e->mode == INMSOM_BT_FP32};
+        parts[2 * q + 1] = {fl[q], mb.flt[b][q], mb.n, false};
     }
-    return INMSOM_BT_OK;
+    return host_copy(e->device, e->stream, e->hc, parts, 6);
 }
 
 int inmsom_bt_ens_set_launch(inmsom_bt_ens *e, int rows_per_wave, int waves_per_xcd)

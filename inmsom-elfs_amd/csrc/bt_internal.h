@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <string>
 
+#include "bt_hostcopy.h"
 #include "inmsom_bt.h"
 
 namespace ibt {
@@ -96,6 +97,7 @@ struct inmsom_bt_ctx {
     double *row_wy = nullptr;      // wind stress on V faces per row
     double nu = 0.0;               // constant viscosity on wet cells
     double *row_wf = nullptr;      // surface water flux per T row
+    ibt::HostCopy hc;               // pinned slots of large copies to the host
     ibt::FusedAlloc *fa = nullptr;  // ping-pong state buffers of the fused step
     int fz_cur = 0;
     int chunk = 0;                 // output rows per wave of the fused step (0 = per-mode default)
