@@ -684,7 +684,7 @@ __device__ __forceinline__ bf16x8 tr_operand(const bf16 *p, int step4)
 // (pixel-major, 16-byte loads and stores) and transposed on the way into
 // the operands by the LDS (tr_read: 8 reads of 8 bytes per 16 pixels and wave
 // where 2-byte reads took 32 and packed them; 32 x 388 x 516 on MI355X: 282 ->
-// 242 us, 8 input channels 167 -> 139).
+// 231 us; 8 input channels, read once per tap row, 167 -> 168).
 // A block of three waves walks work items of WG_R rows x WG_TW columns of
 // one image; wave ky multiplies the row's dy (A = dy[px][co]) by row
 // y + ky - 1 of x at the three column shifts kx (B = x[px + kx - 1][ci]):

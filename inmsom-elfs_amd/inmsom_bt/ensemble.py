@@ -106,7 +106,7 @@ class Ensemble:
 
     def set_pipeline(self, stages: int):
         """2 = substep pairs as a two-wave pipeline, 1 = off, 0 = by mode
-        (default); results agree to rounding."""
+        (default); results do not depend on it."""
         check(lib().inmsom_bt_ens_set_pipeline(self._h, int(stages)), "inmsom_bt_ens_set_pipeline")
 
     def pipeline(self) -> int:

@@ -253,8 +253,8 @@ class BarotropicModel:
 
     def set_pipeline(self, stages: int):
         """FP64 / FP32 fused step: stages = K in 2..4 runs K substeps per
-        launch as a K-wave pipeline, 1 = off, 0 = automatic; results agree
-        to rounding."""
+        launch as a K-wave pipeline, 1 = off, 0 = automatic; results do not
+        depend on it."""
         check(lib().inmsom_bt_set_pipeline(self._h, int(stages)), "inmsom_bt_set_pipeline")
 
     def pipeline(self, mode: str) -> int:
