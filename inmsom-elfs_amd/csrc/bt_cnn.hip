@@ -214,7 +214,8 @@ __global__ void __launch_bounds__(256)
 
 // The output layer and its loss in training (outputs OUT_UV): dL/d(outputs) of
 // the masked mean-square error over U (channel 0) and V (channel 1) points,
-// two BF16 per pixel, and each block's sum of squared errors.  With two output
+// two BF16 per pixel, and each block's sum of squared errors (FP64 from the
+// pixel on: a block sums thousands of pixels over its tiles).  With two output
 // channels the layer is one product per 32 input pixels, all 18 (tap, channel)
 // rows of W against the pixel's 32 channels straight from memory,
 //   Y[(t, co)][q] = sum_ci W[co][t][ci] a[q, ci],
@@ -226,7 +227,7 @@ struct LossArgs {
     const float *tgt;
     const uint8_t *mask;
     float inv_count;
-    float *part;
+    double *part;
 };
 
 __global__ void __launch_bounds__(256)
@@ -236,7 +237,7 @@ __global__ void __launch_bounds__(256)
 {
     constexpr int AW = TW + 2, NP = (TR + 2) * AW, NB = (NP + 31) / 32, ROWS = 18;
     __shared__ float Y[ROWS][NB * 32];
-    __shared__ float red[4];
+    __shared__ double red[4];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 31, half = lane >> 5;
     // A = weights: row i = 2 t + co, k = input channel; w is W[co][t * 32 + ci]
     bf16x8 a[2];
@@ -246,7 +247,7 @@ __global__ void __launch_bounds__(256)
         if (i < ROWS) a[s] = *reinterpret_cast<const bf16x8 *>(w + (size_t)(i & 1) * (9 * CH) + (i >> 1) * CH + 16 * s + 8 * half);
     }
     const float b0 = bias[0], b1 = bias[1];
-    float e2 = 0.0f;
+    double e2 = 0.0;
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const int ti = tile_img[tile], tl = tile_local[tile];
         const Img im = imgs[ti];
@@ -297,13 +298,15 @@ __global__ void __launch_bounds__(256)
                 z[1] += Y[2 * t + 1][q];
             }
             bf16x2 g;
+            float d2 = 0.0f;
 #pragma unroll
             for (int c = 0; c < NOUT; ++c) {
                 const float on = (mk >> c) & 1 ? 1.0f : 0.0f;
                 const float d = (z[c] - tg[c]) * on;
-                e2 += d * d;
+                d2 += d * d;
                 g[c] = (bf16)(2.0f * d * la.inv_count);
             }
+            e2 += d2;
             *reinterpret_cast<bf16x2 *>(out + (im.pix + (long long)y * im.W + x) * NOUT) = g;
         }
         __syncthreads();
@@ -978,13 +981,13 @@ __global__ void k_reduce_wgrad(int ngroups, int nco, int ncol, int kvalid, int k
 // a batch of H x W images: writes dL/dpred into dpred (the two output
 // channels) and per-block partial sums of the squared error; the target and
 // mask of image b start at pixel src[b] (null: in the batch's own order).
-// Training with outputs OUT_UV has it in the output layer (EPI_LOSS); this
+// Training with outputs OUT_UV has it in the output layer (k_conv_loss); this
 // one serves OUT_PSI, whose residuals reach the neighbours.  OUT_PSI: the tendencies are the stream-function differences (psi_uv) and
 // dL/dpsi is their adjoint: psi(x, y) enters du(x, y), du(x, y+1),
 // dv(x, y) and dv(x+1, y).
 __global__ void k_loss(long long n, int H, int W, const float *__restrict__ pred, const float *__restrict__ tgt,
                        const uint8_t *__restrict__ mask, const long long *__restrict__ src, float inv_count,
-                       bf16 *__restrict__ dpred, float *__restrict__ part)
+                       bf16 *__restrict__ dpred, double *__restrict__ part)
 {
     __shared__ float red[256];
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1210,7 +1213,8 @@ struct inmsom_bt_cnn {
     // (otherwise the backward pass ping-pongs dy / dx)
     bf16 *gz[NL] = {};
     uint32_t *bits[3] = {};  // signs of the hidden activations (out > 0), one word per pixel
-    float *pred = nullptr, *tgt = nullptr, *loss_part = nullptr;
+    float *pred = nullptr, *tgt = nullptr;
+    double *loss_part = nullptr;
     int nloss = 0;           // partial sums the last loss wrote
     // the batch: the x, tgt and mask buffers, or (from_ds) samples of the
     // training set in place, image b at pixel src[b]
@@ -1402,11 +1406,11 @@ void forward_loss(inmsom_bt_cnn *c, long long count, bf16 *g3)
 // the loss of the partial sums on the device (waits for them)
 int read_loss(inmsom_bt_cnn *c, long long count, double *loss)
 {
-    std::vector<float> part(c->nloss);
-    CHC(hipMemcpyAsync(part.data(), c->loss_part, (size_t)c->nloss * 4, hipMemcpyDeviceToHost, c->stream));
+    std::vector<double> part(c->nloss);
+    CHC(hipMemcpyAsync(part.data(), c->loss_part, (size_t)c->nloss * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     CHC(hipStreamSynchronize(c->stream));
     double s = 0.0;
-    for (float v : part) s += v;
+    for (double v : part) s += v;
     *loss = count > 0 ? s / (double)count : 0.0;
     return INMSOM_BT_OK;
 }

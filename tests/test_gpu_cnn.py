@@ -522,3 +522,17 @@ def test_training_batch_in_place(kind, b, h, w):
         ref.set_batch(y, ty, my)
         assert net.loss_grad() == ref.loss_grad()
         assert np.array_equal(net.grad(), ref.grad())
+
+
+def test_loss_sums_many_tiles():
+    """The loss of a batch of many tiles per block: zero outputs against
+    targets of 1 in the first two images and 2^-13 in the other six, so that
+    every partial sum of one tile is exact in FP32 and the sum of a block's
+    tiles (the four of a block lie in different images) only in FP64."""
+    print("loss over many tiles, 8x512x512", flush=True)
+    tgt = np.full((8, 512, 512, 2), 2.0 ** -13, dtype=np.float32)
+    tgt[:2] = 1.0
+    with ClosureNet(8, 512, 512) as net:
+        net.set_params(np.zeros_like(_params(1)))
+        net.set_batch(np.zeros((8, 512, 512, 8), dtype=np.float32), tgt, np.full((8, 512, 512), 3, dtype=np.uint8))
+        assert net.loss_grad() == (2.0 + 6.0 * 2.0 ** -26) / 8.0
