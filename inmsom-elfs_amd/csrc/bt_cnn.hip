@@ -696,16 +696,27 @@ __device__ __forceinline__ bf16x8 tr_operand(const bf16 *p, int step4)
 // 8 kx + ci).  x rows are kept in a ring of four LDS slots (rows y - 1 ..
 // y + 1 in use while row y + 2 is staged).  The next row's global loads are
 // issued before the current row's matrix products and written to LDS after
-// them; one barrier per row.  Blocks take consecutive runs of work items (a
-// fixed assignment: the record of block k is always the same sum, so the
-// gradient is deterministic).
+// them; one barrier per row.  Blocks take consecutive runs of work items and
+// leave a record of every `per_rec` of them: a fixed assignment (record k is
+// always the same sum, so the gradient is deterministic), and an accumulator
+// sums the items of one record in FP32 (about wg_chunk pixels), however many
+// a block takes.
 constexpr int WG_TW = 64;            // columns of a work item
 constexpr int WG_R = 16;             // rows of a work item
 constexpr int WG_SLOTS = 4;          // x rows in the ring
-// Blocks (records) of a weight gradient: one round of the five 32-channel
-// blocks a CU holds (four training steps of 32 x 388 x 516: 1024 blocks 9.52
-// ms, 1280 9.05, 2048 9.20, 4096 9.70).
-constexpr size_t WG_BLOCKS = 1280;
+// Blocks of a weight gradient: one round of the five 32-channel blocks a CU
+// holds (four training steps of 32 x 388 x 516 with a record per block: 1024
+// blocks 9.52 ms, 1280 9.05, 2048 9.20, 4096 9.70).
+constexpr int WG_BLOCKS = 1280;
+
+// A value that the compiler takes for a new one at this place, so that what is
+// formed from it (a record's addresses) does not wait in registers through the
+// loop before it.
+__device__ __forceinline__ int late(int x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 template <int CIN>
 struct WgradLds {
@@ -714,8 +725,8 @@ struct WgradLds {
 };
 
 template <int CIN>
-__global__ void __launch_bounds__(3 * 64)
-    k_wgrad(int H, int W, int nitems, int per, const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
+__global__ void __launch_bounds__(3 * 64, CIN == CH ? 4 : 7)
+    k_wgrad(int H, int W, int nitems, int per, int per_rec, const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
             const long long *__restrict__ src, float *__restrict__ part)
 {
     constexpr int NACC = CIN == CH ? 3 : 1;
@@ -815,26 +826,31 @@ __global__ void __launch_bounds__(3 * 64)
             if (more) commit((y + 2) % WG_SLOTS, (y + 1) & 1);
             __syncthreads();
         }
-    }
-    // record of this block: W partials [32][ncol] (column t CIN + ci), then
-    // the 32 bias partials
-    constexpr int ncol = CIN == CH ? 9 * CH : 96;
-    float *rec = part + (size_t)blockIdx.x * (32 * ncol + 32);
+        if ((it + 1) % per_rec != 0 && it + 1 < it1) continue;
+        // the record of these items: W partials [32][ncol] (column t CIN + ci), then
+        // the 32 bias partials
+        constexpr int ncol = CIN == CH ? 9 * CH : 96;
+        float *rec = part + (size_t)(it / per_rec) * (32 * ncol + 32);
+        const int i = late(lane) & 31, half = late(lane) >> 5;
 #pragma unroll
-    for (int a = 0; a < NACC; ++a)
+        for (int a = 0; a < NACC; ++a)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int co = 8 * (r >> 2) + 4 * half + (r & 3);
-            if constexpr (CIN == CH) {
-                rec[co * ncol + (3 * wv + a) * CH + i] = acc[a][r];
-            } else if (i < 24) {
-                rec[co * ncol + 24 * wv + i] = acc[a][r];
-                if (wv == 2) rec[co * ncol + 72 + i] = 0.0f;  // padding columns 72..95
+            for (int r = 0; r < 16; ++r) {
+                const int co = 8 * (r >> 2) + 4 * half + (r & 3);
+                if constexpr (CIN == CH) {
+                    rec[co * ncol + (3 * wv + a) * CH + i] = acc[a][r];
+                } else if (i < 24) {
+                    rec[co * ncol + 24 * wv + i] = acc[a][r];
+                    if (wv == 2) rec[co * ncol + 72 + i] = 0.0f;  // padding columns 72..95
+                }
             }
+        if (wv == 0) {
+            const float b = bsum + __shfl_xor(bsum, 32);
+            if (half == 0) rec[32 * ncol + i] = b;
         }
-    if (wv == 0) {
-        bsum += __shfl_xor(bsum, 32);
-        if (half == 0) rec[32 * ncol + i] = bsum;
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) acc[a] = f32x16{};
+        bsum = 0.0f;
     }
 }
 
@@ -843,11 +859,11 @@ __global__ void __launch_bounds__(3 * 64)
 // one side of a single 32 x 32 product and the input channels as the other:
 // one product per 16 pixels where the 32-channel form took nine, and 68 bytes
 // read per pixel instead of 128.  Wave w of four takes pixels 16 w .. 16 w + 15
-// of the staged row; dy rows y - 1 .. y + 1 sit in a ring of four.  A block's
-// record is W[2][288] then b[2], its waves summed in order.
+// of the staged row; dy rows y - 1 .. y + 1 sit in a ring of four.  A record (of
+// per_rec items, as above) is W[2][288] then b[2], the waves summed in order.
 constexpr int REC_OUT = NOUT * 9 * CH + NOUT;
-__global__ void __launch_bounds__(256)
-    k_wgrad_out(int H, int W, int nitems, int per, const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
+__global__ void __launch_bounds__(256, 8)
+    k_wgrad_out(int H, int W, int nitems, int per, int per_rec, const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
                 float *__restrict__ part)
 {
     struct Lds {
@@ -920,39 +936,57 @@ __global__ void __launch_bounds__(256)
             }
             __syncthreads();
         }
-    }
-    __syncthreads();
+        if ((it + 1) % per_rec != 0 && it + 1 < it1) continue;
+        const int i = late(lane) & 31, half = late(lane) >> 5;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * half + (r & 3);
-        if (row < 18) L.red[wv][row][i] = acc[r];
+        for (int r = 0; r < 16; ++r) {
+            const int row = 8 * (r >> 2) + 4 * half + (r & 3);
+            if (row < 18) L.red[wv][row][i] = acc[r];
+        }
+        const float b2 = bsum + __shfl_xor(bsum, 32);
+        if (t == 4 && half == 0) bred[wv][co] = b2;
+        __syncthreads();
+        float *rec = part + (size_t)(it / per_rec) * REC_OUT;
+        for (int k = threadIdx.x; k < 18 * CH; k += 256) {
+            const int row = k / CH, ci = k - row * CH;
+            const float v = ((L.red[0][row][ci] + L.red[1][row][ci]) + L.red[2][row][ci]) + L.red[3][row][ci];
+            rec[(row & 1) * 9 * CH + (row >> 1) * CH + ci] = v;
+        }
+        if (threadIdx.x < NOUT)
+            rec[NOUT * 9 * CH + threadIdx.x] =
+                ((bred[0][threadIdx.x] + bred[1][threadIdx.x]) + bred[2][threadIdx.x]) + bred[3][threadIdx.x];
+        acc = f32x16{};
+        bsum = 0.0f;
+        __syncthreads();  // the sums are read: the next items' rows take their place
     }
-    bsum += __shfl_xor(bsum, 32);
-    if (t == 4 && half == 0) bred[wv][co] = bsum;
-    __syncthreads();
-    float *rec = part + (size_t)blockIdx.x * REC_OUT;
-    for (int k = threadIdx.x; k < 18 * CH; k += 256) {
-        const int row = k / CH, ci = k - row * CH;
-        const float v = ((L.red[0][row][ci] + L.red[1][row][ci]) + L.red[2][row][ci]) + L.red[3][row][ci];
-        rec[(row & 1) * 9 * CH + (row >> 1) * CH + ci] = v;
-    }
-    if (threadIdx.x < NOUT)
-        rec[NOUT * 9 * CH + threadIdx.x] =
-            ((bred[0][threadIdx.x] + bred[1][threadIdx.x]) + bred[2][threadIdx.x]) + bred[3][threadIdx.x];
 }
 
 // Fixed-order reduction of the chunk records (rec floats each) in two
 // passes: groups of RG consecutive chunks in parallel, then the groups.
 constexpr int RG = 64;
 
+// p[0] + p[step] + .. in this order, n terms, eight loads under way
+__device__ __forceinline__ float strided_sum(const float *__restrict__ p, size_t step, int n)
+{
+    float s = 0.0f;
+    int k = 0;
+    for (; k + 8 <= n; k += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = p[(size_t)(k + j) * step];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += v[j];
+    }
+    for (; k < n; ++k) s += p[(size_t)k * step];
+    return s;
+}
+
 __global__ void k_reduce_groups(int nchunks, int rec, const float *__restrict__ part, float *__restrict__ part2)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= rec) return;
     const int c0 = blockIdx.y * RG, c1 = min(c0 + RG, nchunks);
-    float s = 0.0f;
-    for (int c = c0; c < c1; ++c) s += part[(size_t)c * rec + e];
-    part2[(size_t)blockIdx.y * rec + e] = s;
+    part2[(size_t)blockIdx.y * rec + e] = strided_sum(part + (size_t)c0 * rec + e, rec, c1 - c0);
 }
 
 // groups -> gradient: W in [32][kpad] (zero past kvalid), bias [32], from
@@ -964,17 +998,9 @@ __global__ void k_reduce_wgrad(int ngroups, int nco, int ncol, int kvalid, int k
     const size_t rec = (size_t)nco * ncol + nco;
     if (idx < 32 * kpad) {
         const int co = idx / kpad, k = idx - co * kpad;
-        float s = 0.0f;
-        if (k < kvalid && co < nco)
-            for (int g = 0; g < ngroups; ++g) s += part2[g * rec + (size_t)co * ncol + k];
-        gw[idx] = s;
+        gw[idx] = k < kvalid && co < nco ? strided_sum(part2 + (size_t)co * ncol + k, rec, ngroups) : 0.0f;
     }
-    if (idx < 32) {
-        float s = 0.0f;
-        if (idx < nco)
-            for (int g = 0; g < ngroups; ++g) s += part2[g * rec + (size_t)nco * ncol + idx];
-        gb[idx] = s;
-    }
+    if (idx < 32) gb[idx] = idx < nco ? strided_sum(part2 + (size_t)nco * ncol + idx, rec, ngroups) : 0.0f;
 }
 
 // Masked mean-square loss over U (channel 0) and V (channel 1) points of
@@ -1331,20 +1357,23 @@ void conv_launch(const inmsom_bt_cnn *c, hipStream_t st, int l, bool bwd, const 
 
 void wgrad_launch(inmsom_bt_cnn *c, int l, const bf16 *dy, const bf16 *x, const long long *src = nullptr)
 {
-    // work items (image, 16-row band, 64-column strip) in runs of `per`
-    // per block, at most one record per block of the record buffer
+    // work items (image, 16-row band, 64-column strip): a record per `per_rec`
+    // of them, as many records per block as WG_BLOCKS blocks need
     const int nitems = c->B * ((c->H + WG_R - 1) / WG_R) * ((c->W + WG_TW - 1) / WG_TW);
-    const int per = (nitems + c->wg_nchunks - 1) / c->wg_nchunks;
-    const int nch = (nitems + per - 1) / per;
+    const int per_rec = (nitems + c->wg_nchunks - 1) / c->wg_nchunks;
+    const int nch = (nitems + per_rec - 1) / per_rec;  // records
+    const int per = per_rec * ((nch + WG_BLOCKS - 1) / WG_BLOCKS);
+    const dim3 grid((unsigned)((nitems + per - 1) / per));
     const Layer &Ly = c->L[l];
     if (l == 0)
-        hipLaunchKernelGGL(k_wgrad<CIN0>, dim3(nch), dim3(3 * 64), 0, c->stream, c->H, c->W, nitems, per, dy, x, src,
-                           c->part_w);
+        hipLaunchKernelGGL(k_wgrad<CIN0>, grid, dim3(3 * 64), 0, c->stream, c->H, c->W, nitems, per, per_rec, dy, x,
+                           src, c->part_w);
     else if (l < NL - 1)
-        hipLaunchKernelGGL(k_wgrad<CH>, dim3(nch), dim3(3 * 64), 0, c->stream, c->H, c->W, nitems, per, dy, x, src,
-                           c->part_w);
+        hipLaunchKernelGGL(k_wgrad<CH>, grid, dim3(3 * 64), 0, c->stream, c->H, c->W, nitems, per, per_rec, dy, x,
+                           src, c->part_w);
     else
-        hipLaunchKernelGGL(k_wgrad_out, dim3(nch), dim3(256), 0, c->stream, c->H, c->W, nitems, per, dy, x, c->part_w);
+        hipLaunchKernelGGL(k_wgrad_out, grid, dim3(256), 0, c->stream, c->H, c->W, nitems, per, per_rec, dy, x,
+                           c->part_w);
     const int ncol = l == 0 ? 96 : 288, nco = l < NL - 1 ? CH : NOUT;
     const int rec = nco * ncol + nco;
     const int ngroups = (nch + RG - 1) / RG;
@@ -1623,8 +1652,7 @@ int inmsom_bt_cnn_create(int batch, int ny, int nx, int device, inmsom_bt_cnn **
         CTRY(dmalloc(&c->tgt, np * NOUT));
         CTRY(dmalloc(&c->mask, np));
         CTRY(dmalloc(&c->loss_part, std::max<size_t>((np + 255) / 256, LOSS_BLOCKS)));
-        // records: one per wg_chunk pixels, at most WG_BLOCKS
-        c->wg_nchunks = (int)std::min<size_t>((np + c->wg_chunk - 1) / c->wg_chunk, WG_BLOCKS);
+        c->wg_nchunks = (int)((np + c->wg_chunk - 1) / c->wg_chunk);
         // chunk records, then group records (32 x 288 weights + 32 biases each)
         CTRY(dmalloc(&c->part_w, (size_t)c->wg_nchunks * (32 * 9 * CH + 32)));
         CTRY(dmalloc(&c->part_b, (size_t)((c->wg_nchunks + RG - 1) / RG) * (32 * 9 * CH + 32)));

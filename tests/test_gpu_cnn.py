@@ -536,3 +536,39 @@ def test_loss_sums_many_tiles():
         net.set_params(np.zeros_like(_params(1)))
         net.set_batch(np.zeros((8, 512, 512, 8), dtype=np.float32), tgt, np.full((8, 512, 512), 3, dtype=np.uint8))
         assert net.loss_grad() == (2.0 + 6.0 * 2.0 ** -26) / 8.0
+
+
+def _pass_through_net(p):
+    """Biases of 1 in channel 0 of the hidden layers, the output 0 that
+    channel less 1: activations 1, outputs 0, and dL/dz_2 = dL/dz_3 in channel 0."""
+    p = np.zeros_like(p)
+    for l, (woff, boff, kp) in enumerate(co.layout()):
+        p[boff] = 1.0 if l < 3 else -1.0
+        if l == 3:
+            p[woff + 4 * co.CH] = 1.0
+    return p
+
+
+def test_gradient_of_a_large_batch():
+    """Weight and bias gradients of a batch with more records than blocks:
+    every second pair of work items (16 rows x 64 columns) has targets 2^-18
+    and the others 1, so that a sum over one record of two items is exact in
+    FP32, as are the sums of the records, and a sum that runs on over the next
+    items in one accumulator loses theirs."""
+    print("gradient of a large batch, 16x512x512", flush=True)
+    item = np.arange(16 * 32 * 8).reshape(16, 32, 8)
+    val = np.where(item // 2 % 2 == 0, 1.0, 2.0 ** -18).astype(np.float32)
+    tgt = np.zeros((16, 512, 512, 2), dtype=np.float32)
+    tgt[..., 0] = np.repeat(np.repeat(val, 16, 1), 64, 2)
+    with ClosureNet(16, 512, 512) as net:
+        net.set_params(_pass_through_net(_params(1)))
+        net.set_batch(np.zeros((16, 512, 512, 8), dtype=np.float32), tgt, np.ones((16, 512, 512), dtype=np.uint8))
+        assert not net.forward().any()
+        net.loss_grad()
+        g = net.grad()
+    # sum of -2 tgt / 2^22
+    want = -(1.0 + 2.0 ** -18)
+    for l in (2, 3):
+        woff, boff, kp = co.layout()[l]
+        assert g[boff] == want, (l, "b", g[boff])
+        assert g[woff + 4 * co.CH] == want, (l, "W", g[woff + 4 * co.CH])  # the centre tap of channel 0
