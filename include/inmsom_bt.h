@@ -254,7 +254,9 @@ int inmsom_bt_synchronize(inmsom_bt_ctx *ctx);
  * (uniform metrics, forcing uniform along x, mu = constant * lu) and must
  * share g, rho0, time_smooth and the drag parameters.  grids[k] and
  * forcing[k] describe member k (forcing[k].rdis must be set).  State per
- * member follows inmsom_bt_set_state/get_state. */
+ * member follows inmsom_bt_set_state/get_state.  Calls on one ensemble must
+ * come from one host thread at a time, except that several threads may read
+ * members (inmsom_bt_ens_get_state) at once. */
 typedef struct inmsom_bt_ens inmsom_bt_ens;
 
 int inmsom_bt_ens_create(int nmembers, const inmsom_bt_grid *grids,

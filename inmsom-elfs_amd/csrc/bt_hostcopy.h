@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstddef>
+#include <mutex>
 
 #include <hip/hip_runtime.h>
 
@@ -14,8 +15,9 @@ constexpr size_t HC_SLOT = (size_t)2 << 20;     // bytes of a pinned slot, two p
 constexpr size_t HC_STAGED = (size_t)8 << 20;
 
 // The pinned slots of one context or ensemble (16 MB, allocated by its first
-// large copy, freed with it).
+// large copy, freed with it); one copy at a time uses them.
 struct HostCopy {
+    std::mutex use;
     char *pin = nullptr;
     hipEvent_t ev[2 * HC_THREADS] = {};
 };
@@ -29,7 +31,8 @@ struct HostPart {
 };
 
 // Copies all parts behind the stream's work and waits for them; on return the
-// host arrays hold the values.  Errors leave a message and return its code.
+// host arrays hold the values.  Several threads may copy from one object at a
+// time.  Errors leave a message and return its code; nothing is thrown.
 int host_copy(int device, hipStream_t stream, HostCopy &h, const HostPart *parts, int nparts);
 void host_copy_release(HostCopy &h);
 

@@ -10,8 +10,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
+#include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -36,7 +37,14 @@ int copy_direct(hipStream_t stream, const HostPart *parts, int nparts)
     std::vector<float> t;
     for (int k = 0; k < nparts; ++k) {
         const HostPart &q = parts[k];
-        if (q.f32 && t.size() < q.n) t.resize(q.n);
+        if (q.f32 && t.size() < q.n) {
+            try {
+                t.resize(q.n);
+            } catch (const std::bad_alloc &) {
+                set_error("copy to the host: out of memory");
+                return INMSOM_BT_ENOMEM;
+            }
+        }
         hipError_t e = hipMemcpyAsync(q.f32 ? (void *)t.data() : q.dst, q.src, q.n * elem(q), hipMemcpyDeviceToHost,
                                       stream);
         if (e == hipSuccess && (q.f32 || k == nparts - 1)) e = hipStreamSynchronize(stream);
@@ -46,13 +54,25 @@ int copy_direct(hipStream_t stream, const HostPart *parts, int nparts)
     return INMSOM_BT_OK;
 }
 
+// Chunk c of the parts, each of which is cut into whole slots and a rest.
 struct Chunk {
     const HostPart *part;
     size_t first, n;
 };
+size_t chunks_of(const HostPart &q)
+{
+    const size_t per = HC_SLOT / elem(q);
+    return (q.n + per - 1) / per;
+}
+Chunk chunk_at(const HostPart *part, size_t c)
+{
+    for (; c >= chunks_of(*part); ++part) c -= chunks_of(*part);
+    const size_t per = HC_SLOT / elem(*part);
+    return Chunk{part, c * per, std::min(per, part->n - c * per)};
+}
 
-// chunks t, t + step, .. through two slots
-void copy_chunks(int device, hipStream_t stream, HostCopy &h, const std::vector<Chunk> &chunks, int t, int step,
+// chunks t, t + step, .. of `total` through two slots
+void copy_chunks(int device, hipStream_t stream, HostCopy &h, const HostPart *parts, size_t total, int t, int step,
                  std::atomic<int> &err)
 {
     auto failed = [&](hipError_t e) {
@@ -61,20 +81,20 @@ void copy_chunks(int device, hipStream_t stream, HostCopy &h, const std::vector<
     };
     if (failed(hipSetDevice(device))) return;
     auto issue = [&](size_t c, int slot) {
-        const Chunk &q = chunks[c];
+        const Chunk q = chunk_at(parts, c);
         const size_t es = elem(*q.part);
         const hipError_t e = hipMemcpyAsync(h.pin + (size_t)slot * HC_SLOT, (const char *)q.part->src + q.first * es,
                                             q.n * es, hipMemcpyDeviceToHost, stream);
         return e != hipSuccess ? e : hipEventRecord(h.ev[slot], stream);
     };
     int cur = 2 * t;
-    if ((size_t)t < chunks.size() && failed(issue((size_t)t, cur))) return;
-    for (size_t c = (size_t)t; c < chunks.size(); c += (size_t)step) {
+    if ((size_t)t < total && failed(issue((size_t)t, cur))) return;
+    for (size_t c = (size_t)t; c < total; c += (size_t)step) {
         const int nxt = cur ^ 1;
         // the other slot was copied out in the round before
-        if (c + (size_t)step < chunks.size() && failed(issue(c + (size_t)step, nxt))) break;
+        if (c + (size_t)step < total && failed(issue(c + (size_t)step, nxt))) break;
         if (failed(hipEventSynchronize(h.ev[cur]))) break;
-        const Chunk &q = chunks[c];
+        const Chunk q = chunk_at(parts, c);
         const char *from = h.pin + (size_t)cur * HC_SLOT;
         double *to = q.part->dst + q.first;
         if (q.part->f32)
@@ -123,24 +143,24 @@ int host_copy(int device, hipStream_t stream, HostCopy &h, const HostPart *parts
     for (int k = 0; k < nparts; ++k) bytes += parts[k].n * elem(parts[k]);
     bool staged = bytes >= HC_STAGED;
     for (int k = 0; k < nparts && staged; ++k) staged = pageable(parts[k].dst);
-    if (!staged || !ensure_slots(h)) return copy_direct(stream, parts, nparts);
-    std::vector<Chunk> chunks;
-    for (int k = 0; k < nparts; ++k) {
-        const size_t per = HC_SLOT / elem(parts[k]);
-        for (size_t i = 0; i < parts[k].n; i += per) chunks.push_back({parts + k, i, std::min(per, parts[k].n - i)});
-    }
+    if (!staged) return copy_direct(stream, parts, nparts);
+    const std::lock_guard<std::mutex> one_at_a_time(h.use);
+    if (!ensure_slots(h)) return copy_direct(stream, parts, nparts);
+    size_t total = 0;
+    for (int k = 0; k < nparts; ++k) total += chunks_of(parts[k]);
     std::atomic<int> err{0};
     // a thread that cannot be started leaves its chunks to this one
     std::thread th[HC_THREADS];
-    std::vector<int> mine{0};
+    bool mine[HC_THREADS] = {true};
     for (int t = 1; t < HC_THREADS; ++t) {
         try {
-            th[t] = std::thread([&, t] { copy_chunks(device, stream, h, chunks, t, HC_THREADS, err); });
-        } catch (const std::system_error &) {
-            mine.push_back(t);
+            th[t] = std::thread([&, t] { copy_chunks(device, stream, h, parts, total, t, HC_THREADS, err); });
+        } catch (const std::exception &) {
+            mine[t] = true;
         }
     }
-    for (int t : mine) copy_chunks(device, stream, h, chunks, t, HC_THREADS, err);
+    for (int t = 0; t < HC_THREADS; ++t)
+        if (mine[t]) copy_chunks(device, stream, h, parts, total, t, HC_THREADS, err);
     for (std::thread &t : th)
         if (t.joinable()) t.join();
     // nothing of this copy may still be under way when the slots are used again

@@ -1,7 +1,8 @@
 """State to host arrays through pinned slots: every element of every array, over
 the sizes where it could go wrong (below and above the limit of the staged
 copy, whole slots, a last chunk of one element), FP64 and widened FP32, into
-pageable and pinned arrays, from two contexts at once."""
+pageable and pinned arrays, from two contexts at once, and two members of one
+ensemble at once."""
 import ctypes as C
 import threading
 
@@ -65,3 +66,28 @@ def test_two_contexts_at_once():
     for k, b in enumerate(basins):
         for g in got[k]:
             assert_bitwise(g, {f: np.asarray(getattr(b, f)) for f in STATE}, STATE, f"context {k}")
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32"])
+def test_two_members_at_once(mode):
+    """Threads that each read a member of one ensemble get that member's
+    state, whole, every time."""
+    print(f"host copy, members of one ensemble at once, {mode}", flush=True)
+    basins = [_basin(700, 600, seed=s) for s in (3, 4, 5)]
+    want = []
+    for b in basins:
+        want.append({f: np.asarray(getattr(b, f)) for f in STATE})
+        if mode == "fp32":
+            want[-1].update({f: want[-1][f].astype(np.float32).astype(np.float64) for f in ("u", "v", "ssh")})
+    got = [None] * len(basins)
+    with Ensemble(basins, mode=mode) as ens:
+        def read(k):
+            got[k] = [ens.get_state(k) for _ in range(6)]
+        th = [threading.Thread(target=read, args=(k,)) for k in range(len(basins))]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    for k, w in enumerate(want):
+        for rep, g in enumerate(got[k]):
+            assert_bitwise(g, w, STATE, f"member {k}, read {rep}")
