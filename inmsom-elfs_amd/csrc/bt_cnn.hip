@@ -738,7 +738,7 @@ __global__ void __launch_bounds__(3 * 64, CIN == CH ? 4 : 7)
     __shared__ __attribute__((aligned(16))) WgradLds<CIN> L;
 
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // ky
-    const int lane = threadIdx.x & 63, i = lane & 31, half = lane >> 5;
+    const int lane = threadIdx.x & 63, half = lane >> 5;
     const int nsx = (W + WG_TW - 1) / WG_TW, nry = (H + WG_R - 1) / WG_R;
     f32x16 acc[NACC];
 #pragma unroll
