@@ -342,6 +342,16 @@ void fused_release(inmsom_bt_ctx *c)
     c->state_on_fused = false;
 }
 
+static const void *tile_kernel(int mode)
+{
+    return mode == INMSOM_BT_FP64 ? (const void *)&k_fused_tile<double> : (const void *)&k_fused_tile<float>;
+}
+
+static size_t tile_lds_bytes(int mode, int nr)
+{
+    return mode == INMSOM_BT_FP64 ? tile_lds<double>(nr) : tile_lds<float>(nr);
+}
+
 // Moves the canonical FP64 state into the fused buffers of `mode`.
 static int fused_load(inmsom_bt_ctx *c, int mode)
 {
@@ -376,6 +386,9 @@ static int fused_load(inmsom_bt_ctx *c, int mode)
                 HC(hipMalloc(&a->hup_c[b], n * 8));
                 HC(hipMalloc(&a->hvp_c[b], n * 8));
             }
+        else  // the limit belongs to the kernel, so every context sets the same: the largest tile's
+            HC(hipFuncSetAttribute(tile_kernel(mode), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)tile_lds_bytes(mode, TILE_MAX_ROWS)));
         if (es == 4) {
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->hr, (float *)a->H);
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->rdis, (float *)a->rd);
@@ -588,27 +601,14 @@ static void launch_pipe(inmsom_bt_ctx *c, const FusedParams &p, int mode, int K,
     (void)hipLaunchKernel(pipe_kernel(mode, K), grid, blk, args, 0, c->stream);
 }
 
-static const void *tile_kernel(int mode)
-{
-    return mode == INMSOM_BT_FP64 ? (const void *)&k_fused_tile<double> : (const void *)&k_fused_tile<float>;
-}
-
-static size_t tile_lds_bytes(int mode, int nr)
-{
-    return mode == INMSOM_BT_FP64 ? tile_lds<double>(nr) : tile_lds<float>(nr);
-}
-
-// rows per tile of a grid; the kernel's LDS limit raised to what they need
-static int tile_shape(inmsom_bt_ctx *c, int mode)
+// rows per tile of a grid
+static int tile_shape(inmsom_bt_ctx *c)
 {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1)
         cus = 256;
     const long long strips = (c->nx + pipe_width(TILE_K) - 1) / pipe_width(TILE_K);
-    const int nr = tile_rows(cus, [&](int rows) { return strips * ((c->ny + rows - 1) / rows); });
-    (void)hipFuncSetAttribute(tile_kernel(mode), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)tile_lds_bytes(mode, nr));
-    return nr;
+    return tile_rows(cus, [&](int rows) { return strips * ((c->ny + rows - 1) / rows); });
 }
 
 static void launch_tile(inmsom_bt_ctx *c, FusedParams &p, int mode, int nr, int ksub, int form_mask, int save_forcing)
@@ -671,7 +671,7 @@ int fused_run(inmsom_bt_ctx *c, double tau, int nstep, int nsteps, int mode, dou
     // one- and two-substep launches stay within one.
     const int K = pipe_stages(c, mode);
     const bool tiles = tile_path(c, mode);
-    const int tile_nr = tiles ? tile_shape(c, mode) : 0;
+    const int tile_nr = tiles ? tile_shape(c) : 0;
     const long long total = (long long)nsteps * nstep;
     for (long long g = 0; g < total;) {
         const int sub = (int)(g % nstep) + 1;

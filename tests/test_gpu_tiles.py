@@ -1,7 +1,10 @@
 """The tiles of the fast modes on small grids: bit for bit what the march
 gives (a launch shape of the caller's, here one row chunk, selects the march),
 over tile edges in both directions, odd substep counts and calls that span
-launches, for one basin and for an ensemble."""
+launches, for one basin and for an ensemble; and basins of different tile
+sizes run by several threads at once."""
+import threading
+
 import pytest
 
 from _util import STATE, assert_bitwise
@@ -46,3 +49,29 @@ def test_ensemble_tiles_equal_march(mode, nstep):
     for o in out[1:]:
         for k in range(len(basins)):
             assert_bitwise(o[k], out[0][k], STATE, f"member {k} {mode} nstep={nstep}")
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32"])
+def test_tile_sizes_in_several_threads(mode):
+    """Basins whose tiles differ in rows (and in LDS), each run by a thread of
+    its own at once, give what each gives alone."""
+    print(f"tiles of several sizes in threads, {mode}", flush=True)
+    basins = [_basin(*shape, seed=21) for shape in ((64, 64), (256, 256), (512, 384))]
+    out = [None] * len(basins)
+
+    def run(k, reps):
+        with BarotropicModel(basins[k]) as m:
+            for _ in range(reps):
+                m.run(3, mode, nstep=2)
+            out[k] = m.get_state()
+
+    for k in range(len(basins)):
+        run(k, 20)
+    alone = list(out)
+    th = [threading.Thread(target=run, args=(k, 20)) for k in range(len(basins))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for k, b in enumerate(basins):
+        assert_bitwise(out[k], alone[k], STATE, f"{b.nx}x{b.ny} {mode}")
