@@ -882,7 +882,8 @@ int inmsom_bt_ens_get_state(inmsom_bt_ens *e, int k, double *u, double *up, doub
         parts[2 * q] = {lv[q], mb.lvl[b][q], mb.n, e->mode == INMSOM_BT_FP32};
         parts[2 * q + 1] = {fl[q], mb.flt[b][q], mb.n, false};
     }
-    return host_copy(e->device, e->stream, e->hc, parts, 6);
+    const size_t cell = 3 * sizeof(double) + 3 * esz(e->mode);
+    return host_copy(e->device, e->stream, e->hc, parts, 6, (size_t)all_cells(e) * cell);
 }
 
 int inmsom_bt_ens_set_launch(inmsom_bt_ens *e, int rows_per_wave, int waves_per_xcd)

@@ -6,7 +6,8 @@
 // c % HC_THREADS) through two pinned slots: the next chunk is under way while
 // the last one is copied out, or widened.  Measured on MI355X (six arrays, ms
 // before / now): 1021 x 763 2.1 / 1.07, 2048 x 1536 8.7 / 3.9 (38 GB/s: the link;
-// 2 or 8 threads the same), FP32 widened 9.3 / 3.1.
+// 2 or 8 threads the same, slots of 1 MB 4.9), FP32 widened 9.3 / 3.1; the copy
+// that makes the slots takes up to 2 ms longer (HC_FIRST).
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -137,14 +138,19 @@ bool ensure_slots(HostCopy &h)
 
 }  // namespace
 
-int host_copy(int device, hipStream_t stream, HostCopy &h, const HostPart *parts, int nparts)
+int host_copy(int device, hipStream_t stream, HostCopy &h, const HostPart *parts, int nparts, size_t whole)
 {
     size_t bytes = 0;
     for (int k = 0; k < nparts; ++k) bytes += parts[k].n * elem(parts[k]);
     bool staged = bytes >= HC_STAGED;
     for (int k = 0; k < nparts && staged; ++k) staged = pageable(parts[k].dst);
     if (!staged) return copy_direct(stream, parts, nparts);
-    const std::lock_guard<std::mutex> one_at_a_time(h.use);
+    std::unique_lock<std::mutex> one_at_a_time(h.use);
+    if (!h.pin && h.direct + std::max(bytes, whole) < HC_FIRST) {
+        h.direct += bytes;
+        one_at_a_time.unlock();
+        return copy_direct(stream, parts, nparts);
+    }
     if (!ensure_slots(h)) return copy_direct(stream, parts, nparts);
     size_t total = 0;
     for (int k = 0; k < nparts; ++k) total += chunks_of(parts[k]);
