@@ -23,6 +23,7 @@ from .model import STATE, _d, _grid_struct, rayleigh
 
 DEFAULT_ROWS = (0, 12, 16, 24, 32, 40, 48, 64)
 DEFAULT_WAVES = (0, 256, 384, 512)
+KERNELS = "march, pairs, pipeline, tiles"
 # two-wave workgroups per XCD when substep pairs run as a pipeline
 DEFAULT_GROUPS = (0, 96, 128, 160, 192)
 
@@ -182,8 +183,12 @@ class Ensemble:
 
     # ------------------------------------------------------------ autotuner
     def signature(self) -> str:
+        """Key of the ensemble's entry in an autotune cache.  KERNELS goes with
+        the kernels that a launch shape chooses between: a shape found with
+        others (before small ensembles ran on tiles, which any shape of the
+        caller's turns off) is not taken but tuned again."""
         shapes = ",".join(f"{b.nx}x{b.ny}" for b in self.basins)
-        return hashlib.sha1(f"{self.mode}|pipeline {self.pipeline()}|{shapes}".encode()).hexdigest()[:16]
+        return hashlib.sha1(f"{KERNELS}|{self.mode}|pipeline {self.pipeline()}|{shapes}".encode()).hexdigest()[:16]
 
     def autotune(self, nstep: int = 2, trial_steps: int = 20,
                  rows: Sequence[int] = DEFAULT_ROWS, waves: Optional[Sequence[int]] = None,

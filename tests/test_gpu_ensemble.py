@@ -3,6 +3,9 @@ fused step bit for bit (same arithmetic, different work mapping), the
 FP64_EXACT members equal the oracle, graph replays equal direct launches,
 the launch shape never changes results, and the autotuner restores the
 state it times from."""
+import hashlib
+import json
+
 import numpy as np
 import pytest
 
@@ -123,6 +126,22 @@ def test_autotune_restores_state_and_conserves_volume(tmp_path):
         again = ens.autotune(nstep=2, trial_steps=3, rows=(12, 24), waves=(128, 384),
                              cache=str(tmp_path / "tune.json"))
         assert again["cached"]
+
+
+def test_autotune_leaves_shapes_of_other_kernels(tmp_path):
+    """A cache entry under the key of the library before small ensembles ran
+    on tiles (mode, pipeline, sizes) is not taken: any launch shape of the
+    caller's would turn the tiles off."""
+    basins = _members(3, seed=12)
+    print("autotune with an entry of other kernels", flush=True)
+    cache = tmp_path / "tune.json"
+    with Ensemble(basins, mode="fp32") as ens:
+        old = "fp32|pipeline %d|" % ens.pipeline() + ",".join(f"{b.nx}x{b.ny}" for b in basins)
+        key = hashlib.sha1(old.encode()).hexdigest()[:16]
+        cache.write_text(json.dumps({key: {"rows_per_wave": 16, "waves_per_xcd": 256, "ms_per_step": 0.01}}))
+        res = ens.autotune(nstep=2, trial_steps=2, rows=(0,), waves=(0,), cache=str(cache))
+        assert not res["cached"] and ens.launch == (0, 0)
+        assert set(json.loads(cache.read_text())) == {key, ens.signature()}  # the other entry stays
 
 
 def test_graphs_follow_table_rebuilds():
