@@ -657,10 +657,10 @@ __global__ void __launch_bounds__(WAVE, 2) k_dropin(DropinParams p)
 // the stage-by-stage path's (uv_diff4), operand for operand: the same bits.
 // FIRST of DStage is the launch argument here (it is uniform).
 // Measured on MI355X, us per substep on a longitude-latitude grid, march /
-// tiles: 285 x 159 14.5 / 7.7, 512 x 384 24.3 / 19.1, 640 x 512 31.3 / 29.4,
-// 900 x 700 48.7 / 54; with the biharmonic term (its march took two more
-// launches) 285 x 159 42 / 10.3, 2048 x 1536 408 / 369, and with metrics per
-// cell 657 / 434.  Bound by FP64 issue (about 30 IEEE divisions a point, 50
+// tiles: 285 x 159 14.5 / 7.7, 512 x 384 24.3 / 19.1 (take_march has the sizes
+// where the march is the faster); with the biharmonic term (its march took two
+// more launches) 285 x 159 42 / 10.3, 2048 x 1536 408 / 369, and with metrics
+// per cell 657 / 434.  Bound by FP64 issue (about 30 IEEE divisions a point, 50
 // with the term) and, below 300 x 200, by the launch and the phases' latency.
 constexpr int DT_MAX_ROWS = 12;
 constexpr int DT_RIM = 4;  // rows of a tile that it does not write
@@ -922,6 +922,7 @@ struct DropinAlloc {
     int eligible = -1;  // grid part of the eligibility: -1 not checked, 0 no, 1 yes
     std::string why;
     bool rowmet_ok = false;
+    int met = MET_CELL;  // how the march reads the metrics
     int chunk = 0;
     long long slots = 0;
     int tile_nr[2] = {};  // rows per tile without and with the biharmonic term (0: the march)
@@ -957,31 +958,51 @@ __global__ void k_dropin_masks(size_t n, const float *lu, const float *luu, cons
     mb[i] = b;
 }
 
+template <bool FIRST>
+const void *march_kernel(int met)
+{
+    return met == MET_ONE   ? (const void *)k_dropin<FIRST, MET_ONE>
+           : met == MET_ROW ? (const void *)k_dropin<FIRST, MET_ROW>
+                            : (const void *)k_dropin<FIRST, MET_CELL>;
+}
+
 const void *tile_kernel(bool rowmet, bool d4)
 {
     return rowmet ? (d4 ? (const void *)k_dropin_tile<true, true> : (const void *)k_dropin_tile<true, false>)
                   : (d4 ? (const void *)k_dropin_tile<false, true> : (const void *)k_dropin_tile<false, false>);
 }
 
-// Whether this grid's calls run on tiles (below DT_CELLS cells, where they
-// are measured faster than the march; with the biharmonic term always), and
-// their rows: 8 or 12, which give the busiest CU the fewest to work through.
-constexpr size_t DT_CELLS = 400000;
+// Whether a call without the biharmonic term takes the march, by the rounds in
+// which the CUs, one block each, work through the t tiles of 12 rows (with the
+// term: the tiles always).  A tile's time goes in such steps, the march's with the
+// cells.  Measured on MI355X (256 CUs), us per substep, march / the better tiles,
+// with t: metrics per row 340 x 260 (198) 17.3 / 11.3, 380 x 300 (266) 21.8 / 18.3,
+// 512 x 384 (441) 24.6 / 20.0, 540 x 420 (530) 29.2 / 29.8, 600 x 440 (616) 30.3 /
+// 28.6, 640 x 512 (715) 32.0 / 30.7, 620 x 580 (803) 35.7 / 37.3; per cell 340 x 260
+// 17.5 / 12.1, 380 x 300 21.9 / 19.7, 540 x 420 30.5 / 34.0, 600 x 440 34.1 / 32.8,
+// 640 x 512 37.6 / 35.2, 620 x 580 39.9 / 42.8; one metric, whose quotients only
+// the march shares, 340 x 260 13.6 / 11.3, 380 x 300 16.3 / 18.1, 512 x 384 18.7 /
+// 20.5, 640 x 512 26.7 / 30.7.
+bool take_march(int met, long long t, long long cus)
+{
+    if (met == MET_ONE) return t > cus;
+    return t > 3 * cus || (t > 2 * cus && 3 * t < 7 * cus);
+}
+
+// Whether this grid's calls run on tiles, and their rows, 8 or 12: the fewer us
+// by the rounds r of each, 9.0 r + 1.3 with 12 rows and 5.2 r + 3.1 with 8 (with
+// the biharmonic term 1.3 times as long; us with 12 / 8 rows without and with it:
+// 285 x 159, r = 1 and 1, 10.6 / 8.7, 13.8 / 11.2; 340 x 260, 1 and 2, 11.3 / 13.5,
+// 15.0 / 17.9; 400 x 360, 2 and 3, 19.0 / 18.7, 25.7 / 25.0; 512 x 384, 2 and 4,
+// 20.0 / 23.8, 27.2 / 31.3; 1021 x 763 with it 83 / 93).
 int choose_tiles(inmsom_bt_ctx *c, DropinAlloc *a, int cus)
 {
     const long long strips = (c->nx + SW - 1) / SW;
+    auto tiles = [&](int nr) { return strips * ((c->ny + nr - DT_RIM - 1) / (nr - DT_RIM)); };
+    auto rounds = [&](int nr) { return (double)((tiles(nr) + cus - 1) / cus); };
+    const int nr = 9.0 * rounds(12) + 1.3 < 5.2 * rounds(8) + 3.1 ? 12 : 8;
     for (int d4 = 0; d4 < 2; ++d4) {
-        a->tile_nr[d4] = 0;
-        if (!d4 && c->n >= DT_CELLS) continue;
-        long long best = -1;
-        for (int nr : {12, 8}) {
-            const int rows = nr - DT_RIM;
-            const long long cost = (strips * ((c->ny + rows - 1) / rows) + cus - 1) / cus * (nr + 4);
-            if (best < 0 || cost < best) {
-                best = cost;
-                a->tile_nr[d4] = nr;
-            }
-        }
+        a->tile_nr[d4] = d4 || !take_march(a->met, tiles(12), cus) ? nr : 0;
         DHC(hipFuncSetAttribute(tile_kernel(a->rowmet_ok, d4), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)dropin_tile_lds(DT_MAX_ROWS)));
     }
@@ -1056,8 +1077,10 @@ int check_grid(inmsom_bt_ctx *c, DropinAlloc *a)
     int dev = 0, cus = 0, per_cu = 0;
     DHC(hipGetDevice(&dev));
     DHC(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const void *kf = rows ? (const void *)k_dropin<false, MET_ROW> : (const void *)k_dropin<false, MET_CELL>;
-    DHC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kf, WAVE, 0));
+    a->met = !rows ? MET_CELL
+             : c->uniform_metrics && c->metric0 > DEN_MIN && c->metric0 < DEN_MAX ? MET_ONE
+                                                                                 : MET_ROW;
+    DHC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, march_kernel<false>(a->met), WAVE, 0));
     a->slots = (long long)cus * (per_cu > 0 ? per_cu : 1);
     const int strips = (nx + SW - 1) / SW;
     a->chunk = fit_chunk(ny, strips, a->slots, 3, 2);
@@ -1084,11 +1107,8 @@ template <bool FIRST>
 void launch_dropin(inmsom_bt_ctx *c, const DropinParams &p, int met)
 {
     dim3 grid((unsigned)(p.per_xcd * NXCD)), blk(WAVE);
-    const void *k = met == MET_ONE   ? (const void *)k_dropin<FIRST, MET_ONE>
-                    : met == MET_ROW ? (const void *)k_dropin<FIRST, MET_ROW>
-                                     : (const void *)k_dropin<FIRST, MET_CELL>;
     void *args[] = {const_cast<DropinParams *>(&p)};
-    (void)hipLaunchKernel(k, grid, blk, args, 0, c->stream);
+    (void)hipLaunchKernel(march_kernel<FIRST>(met), grid, blk, args, 0, c->stream);
 }
 
 }  // namespace
@@ -1178,8 +1198,7 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
     p.exp_lim = ExpCheck::LIMIT;
     for (const double d : {p.rho0, p.tau, dn, d4n})
         if (!(d > DEN_MIN && d < DEN_MAX)) p.exp_lim = -1;  // IEEE divisions throughout
-    const bool one = a->rowmet_ok && c->uniform_metrics && c->metric0 > DEN_MIN && c->metric0 < DEN_MAX;
-    if (one) {
+    if (a->met == MET_ONE) {
         p.q_d = make_den(c->metric0);
         p.q_dd = make_den(c->metric0 * c->metric0);
     }
@@ -1196,7 +1215,6 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
         p.total = p.strips * p.nchunks;
         p.per_xcd = (p.total + NXCD - 1) / NXCD;
     }
-    const int met = one ? MET_ONE : a->rowmet_ok ? MET_ROW : MET_CELL;
     const int last = 2 * nstep;
     for (int k = 1; k <= last; ++k) {
         // substep k reads the caller's state (k = 1) or the buffer substep
@@ -1232,9 +1250,9 @@ int dropin_call(inmsom_bt_ctx *c, double tau, int nstep, double *const st[6], do
             (void)hipLaunchKernel(tile_kernel(a->rowmet_ok, ksw4 > 0), dim3((unsigned)(p.per_xcd * NXCD)),
                                   dim3((unsigned)(WAVE * tile_nr)), args, dropin_tile_lds(tile_nr), c->stream);
         } else if (k == 1)
-            launch_dropin<true>(c, p, met);
+            launch_dropin<true>(c, p, a->met);
         else
-            launch_dropin<false>(c, p, met);
+            launch_dropin<false>(c, p, a->met);
     }
     DHC(hipGetLastError());
     return INMSOM_BT_OK;

@@ -52,11 +52,14 @@ def _rows_basin(b):
 
 
 # the march with its three kinds of metrics, where it takes over from the tiles
-# (360,000 and 100,000 cells): columns and rows that fill no strip and no
-# chunk, wet cells next to the halo
+# (more than three rounds of 12-row tiles over 256 CUs, a third round less than a
+# third full; one metric: more than one round) and the tiles just below: columns
+# and rows that fill no strip, tile or chunk, wet cells next to the halo
 @pytest.mark.parametrize("shape,metrics,nstep", [((691, 593), "stretched", 1), ((1013, 419), "stretched", 3),
                                                  ((691, 593), "rows", 1), ((1013, 419), "rows", 3),
-                                                 ((691, 593), "uniform", 3), ((333, 301), "uniform", 1)])
+                                                 ((691, 593), "uniform", 3), ((361, 299), "uniform", 1),
+                                                 ((333, 301), "uniform", 2), ((541, 419), "rows", 2),
+                                                 ((541, 419), "stretched", 1), ((601, 439), "rows", 1)])
 def test_march_equals_stage_by_stage(shape, metrics, nstep):
     print(f"drop-in march {shape} {metrics} nstep={nstep}", flush=True)
     b = make_basin(*shape, seed=17, sigma=6.0, hland=1.0, metrics="stretched" if metrics == "stretched" else "uniform")
