@@ -191,6 +191,7 @@ struct inmsom_bt_ens {
     int pipe = 0;           // substep pairs as a two-wave pipeline: 0 = by mode, 1 = off, 2 = on
     int built_chunk = -1;
     bool built_two = false, built_tile = false;
+    int tile_out = 0;       // rows that a tile writes (choose_tiles), 0: no tiles
     unsigned table_gen = 0;  // bumped whenever build_tables replaces table[] / item_*
     int phase = 0;          // buffer set holding the current state
     // graph of one outer step for (tau, nstep, start phase)
@@ -244,12 +245,11 @@ long long all_cells(const inmsom_bt_ens *e)
     return cells;
 }
 
-// the tiles: the fast modes below TWO_SUBSTEP_CELLS cells in all, unless the
-// caller chose a launch shape
+// the tiles: the fast modes below TWO_SUBSTEP_CELLS cells in all, while they
+// fit the rounds of choose_tiles, unless the caller chose a launch shape
 bool tile_path(const inmsom_bt_ens *e)
 {
-    return e->mode != INMSOM_BT_FP64_EXACT && e->subs == 0 && e->pipe == 0 && e->chunk == 0 && e->waves_per_xcd == 0 &&
-           all_cells(e) < TWO_SUBSTEP_CELLS;
+    return e->tile_out > 0 && e->subs == 0 && e->pipe == 0 && e->chunk == 0 && e->waves_per_xcd == 0;
 }
 
 // two substeps per launch: as set, or by mode and size as for one basin
@@ -278,17 +278,29 @@ size_t tile_lds_bytes(const inmsom_bt_ens *e, int nr)
     return e->mode == INMSOM_BT_FP64 ? tile_lds<double>(nr) : tile_lds<float>(nr);
 }
 
-// rows a tile writes, of the tile_rows rule over all members
-int tile_chunk(const inmsom_bt_ens *e)
+// Rows a tile writes, of the tile_rows rule over all members, or 0: the march.
+// A round of tiles over the CUs takes longer here than on one basin (a tile first
+// reads which member's it is), so the march wins from three rounds of 16 rows on
+// in FP64 and four in FP32.  Measured on MI355X, us per substep, march / tiles,
+// rounds: FP64 four of 256 x 256 11.5 / 14.6, 3; 128 of 44 x 40 11.8 / 14.3, 3; 400 of
+// 22 x 20 15.9 / 22.1, 5; ten of 150 x 140 10.8 / 10.5, 2; FP32 four of 256 x 256 9.4 /
+// 9.7, 60 of 60 x 56 10.9 / 9.9, 3; 400 of 22 x 20 12.9 / 14.9, 5; ten of 150 x 140
+// 9.3 / 7.3, 2.
+void choose_tiles(inmsom_bt_ens *e)
 {
+    e->tile_out = 0;
+    if (e->mode == INMSOM_BT_FP64_EXACT || all_cells(e) >= TWO_SUBSTEP_CELLS) return;
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device) != hipSuccess || cus < 1)
         cus = 256;
-    return tile_out_rows(tile_rows(cus, [&](int rows) {
+    auto tiles = [&](int rows) {
         long long t = 0;
         for (const EnsMember &m : e->mem) t += (long long)((m.nx + SW2 - 1) / SW2) * ((m.ny + rows - 1) / rows);
         return t;
-    }));
+    };
+    const int nr = tile_rows(cus, tiles), out = tile_out_rows(nr);
+    const long long rounds = (tiles(out) + cus - 1) / cus;
+    if (rounds * (nr + 4) <= (e->mode == INMSOM_BT_FP64 ? 2 : 3) * (TILE_MAX_ROWS + 4)) e->tile_out = out;
 }
 
 // the batch kernel for (mode, two substeps, forming substep)
@@ -698,7 +710,7 @@ void launch_shape(const inmsom_bt_ens *e, bool *two, int *wpx, int *chunk)
     *two = two_per_launch(e);
     if (tile_path(e)) {
         *wpx = 0;
-        *chunk = tile_chunk(e);
+        *chunk = e->tile_out;
         return;
     }
     *wpx = e->waves_per_xcd > 0 ? e->waves_per_xcd : default_waves(e, *two);
@@ -789,6 +801,7 @@ int inmsom_bt_ens_create(int nmembers, const inmsom_bt_grid *grids, const inmsom
         inmsom_bt_ens_destroy(e);
         return rc;
     }
+    choose_tiles(e);
     *out = e;
     return INMSOM_BT_OK;
 }

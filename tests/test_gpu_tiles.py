@@ -36,9 +36,12 @@ def test_tiles_equal_march(mode, shape, nstep, steps):
     assert_bitwise(out[0], out[1], STATE, f"tiles vs march {mode} {shape} nstep={nstep}")
 
 
-@pytest.mark.parametrize("mode,nstep", [("fp32", 2), ("fp64", 3), ("fp32", 1)])
-def test_ensemble_tiles_equal_march(mode, nstep):
+# the last with more tiles than two rounds of the CUs: the march in FP64
+@pytest.mark.parametrize("mode,nstep,many", [("fp32", 2, 1), ("fp64", 3, 1), ("fp32", 1, 1), ("fp64", 2, 30),
+                                             ("fp32", 2, 30)])
+def test_ensemble_tiles_equal_march(mode, nstep, many):
     basins = [_basin(x, y, seed=9 + k) for k, (x, y) in enumerate(((40, 90), (130, 33), (61, 62), (9, 7)))]
+    basins = [b for b in basins for _ in range(many)]
     print(f"ensemble tiles {mode} nstep={nstep}", flush=True)
     out = []
     for rows, graph in ((0, True), (0, False), (7, False)):
