@@ -123,19 +123,13 @@ def test_ensemble_64_members_5000_steps():
     assert max(drift) <= 1e-5, max(drift)
     for k in sample:
         b = basins[k]
-        # the single basin runs the same kernel body (the two-wave pipeline
-        # when the ensemble uses it); the two kernels may contract
-        # multiply-adds differently, so the members agree to FP32 rounding
-        # grown over 5000 steps, not bit for bit
+        # the same bits as the single basin, whichever way each runs
         print(f"member {k}: {b.nx}x{b.ny} single-basin run, pipeline {stages}", flush=True)
         with BarotropicModel(b) as m:
             m.set_pipeline(stages if stages else 1)
             m.run(steps, "fp32", nstep=NSTEP_BAROTROP)
             want = m.get_state()
-        for f in STATE:
-            e = rel_l2(got[k][f], want[f])
-            print(f"  {f}: rel L2 {e:.2e}")
-            assert e <= 1e-5, (k, f, e)
+        assert_bitwise(got[k], want, STATE, f"member {k}")
 
 
 CLOSURE_PARAMS = os.path.join(ROOT, "inmsom-elfs_amd", "inmsom_bt", "data", "closure_cfg1.npz")

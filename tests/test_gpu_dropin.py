@@ -150,7 +150,7 @@ def test_routing():
     b = make_basin(40, 30, seed=5, sigma=3.0)
     with BarotropicModel(b) as m:
         assert m.dropin_path(0) == "fused"
-        assert m.dropin_path(1) == "fused"  # biharmonic viscosity: pre-pass per substep
+        assert m.dropin_path(1) == "fused"  # the biharmonic viscosity in the same launch
         m.set_dropin_path("literal")
         assert m.dropin_path(0) == "literal"
     pb, _, _ = periodic_pair((1, 0))

@@ -112,9 +112,7 @@ def test_pipeline_matches_one_launch_per_substep(mode, stages, shape, nstep, ste
     """K substeps per launch as a K-wave pipeline (across outer steps, with
     one- and two-substep launches for the remainder) give what one launch
     per substep gives, over strip and chunk edges, odd nstep and a ragged
-    last chunk: to rounding (FP64 relative L2 <= 1e-14, FP32 <= 1e-6; the
-    modes contract multiply-adds as the compiler finds them, which the
-    pipeline's code may do differently)."""
+    last chunk, bit for bit (the modes' multiply-adds are explicit)."""
     b = randomize_state(make_basin(*shape, seed=34, sigma=5.0), 10)
     print(f"pipeline {stages} {mode} {shape} nstep={nstep} steps={steps} chunk={chunk}", flush=True)
     out = {}
@@ -125,11 +123,7 @@ def test_pipeline_matches_one_launch_per_substep(mode, stages, shape, nstep, ste
             m.set_pipeline(k)
             m.run(steps, mode, nstep=nstep)
             out[k] = m.get_state()
-    tol = 1e-14 if mode == "fp64" else 1e-6
-    for k in STATE:
-        e = rel_l2(out[stages][k], out[1][k])
-        print(f"  {k}: rel L2 {e:.2e}")
-        assert e <= tol, (k, e)
+    assert_bitwise(out[stages], out[1], STATE, f"pipeline of {stages}, {mode} {shape} nstep={nstep}")
 
 
 def test_fused_fp64_within_1e12():
