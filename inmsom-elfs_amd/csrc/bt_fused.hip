@@ -393,12 +393,10 @@ static int fused_load(inmsom_bt_ctx *c, int mode)
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->hr, (float *)a->H);
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->rdis, (float *)a->rd);
         } else {
-#pragma clang fp contract(fast)
             hipLaunchKernelGGL(k_copy_d, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->hr, (double *)a->H);
             hipLaunchKernelGGL(k_copy_d, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->rdis, (double *)a->rd);
         }
     } else {
-#pragma clang fp contract(fast)
         // forcing may have changed: refresh the static copies
         if (es == 4)
             hipLaunchKernelGGL(k_to_f32, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->rdis, (float *)a->rd);
@@ -455,14 +453,11 @@ static bool tile_path(const inmsom_bt_ctx *c, int mode)
     return mode != INMSOM_BT_FP64_EXACT && c->n < TWO_SUBSTEP_CELLS && c->subs_per_launch == 0 && c->pipe_k == 0 && c->chunk == 0;
 }
 
-// Parameters of a launch that reads buffer set b and writes 1 - b: substep
-// `sub`, or substeps sub and sub + 1 when `two`.
-// Substeps per launch: as set, or automatically two in FP64 and FP32 on
-// grids large enough to be bandwidth-bound and one otherwise.  Measured on
-// MI355X (us per substep, one / two per launch): 2048 x 1536 FP64 91.3 /
-// 81.5, FP32 66.1 / 53.9, FP64_EXACT 118 / 138 (two windows in one wave's
-// registers leave one wave per SIMD); 512 x 384 (latency-bound, rows per wave 2) FP32
-// 8.7 / 9.5 per substep.
+// Substeps per launch: as set, or automatically two in FP64 and FP32 (on tiles,
+// or as a pipeline from TWO_SUBSTEP_CELLS cells on; one on a small grid with a
+// launch shape of the caller's) and one in FP64_EXACT, where two windows in one
+// wave's registers leave one wave per SIMD (2048 x 1536 on MI355X, us per
+// substep, one / two per launch: 118 / 138).
 int subs_per_launch(const inmsom_bt_ctx *c, int mode)
 {
     if (c->subs_per_launch > 0) return c->subs_per_launch;
@@ -525,6 +520,8 @@ static long long wave_slots(inmsom_bt_ctx *c, int mode, bool two)
     return c->slots[idx];
 }
 
+// Parameters of a launch that reads buffer set b and writes 1 - b: substep
+// `sub`, or substeps sub and sub + 1 when `two`.
 static FusedParams make_params(inmsom_bt_ctx *c, FusedAlloc *a, int b, double tau, int nstep,
                                int sub, int mode, bool two)
 {
@@ -740,7 +737,6 @@ int fused_range_check(inmsom_bt_ctx *c, long long *bad)
                                c->mask[0], c->mask[3], c->mask[4], (const double *)a->lvl[b][2],
                                (const double *)a->lvl[b][0], (const double *)a->lvl[b][1], cnt);
     } else {
-#pragma clang fp contract(fast)
         hipLaunchKernelGGL(k_range<double>, dim3(nblk(n)), dim3(256), 0, c->stream, c->nx, c->ny,
                            c->mask[0], c->mask[3], c->mask[4], c->st[4], c->st[0], c->st[2], cnt);
     }
