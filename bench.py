@@ -47,11 +47,6 @@ BYTES_PER_CELL = {
     "fp64_exact": 12 * 8 + 8 + 8,          # 112
     "fp32": 6 * 4 + 6 * 8 + 4 + 4,         # 80
 }
-# The same count with the two RHS components frozen over a call, which a
-# substep of the reference reads (written by the first substep of a call,
-# read by the second: one access per component per substep on average with
-# nstep_barotrop = 2); reported beside the minimal count, never as it.
-BYTES_PER_CELL_WITH_RHS = {"fp64": 128, "fp64_exact": 128, "fp32": 88}
 # Warm-up before a timed region: at least the requested warm-up steps and
 # at least this many seconds of them, so that the clocks have settled.
 WARMUP_SECONDS = 2.0
@@ -179,6 +174,11 @@ def traffic_from_profiles(mode):
         return None
 
 
+def measured_frac(traffic, launch_s):
+    """Share of HBM peak of the bytes a launch was measured to move."""
+    return None if traffic is None else traffic / launch_s / 1e9 / PEAK_HBM_GBS
+
+
 def warm_up(run, sync, steps, seconds=WARMUP_SECONDS):
     """Runs at least ``steps`` warm-up steps and keeps running them, in
     doubling batches, until ``seconds`` have passed; returns (steps run,
@@ -226,8 +226,7 @@ def timed_mode(m, b, mode, steps, warmup, ncell):
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS, "traffic": traffic,
                      "bytes_per_cell_substep": bpc, "cells_per_launch": ncell, "substeps_per_launch": subs,
-                     "frac_with_frozen_rhs": BYTES_PER_CELL_WITH_RHS[mode] * subs * ncell / avg_launch_s / 1e9
-                     / PEAK_HBM_GBS},
+                     "frac_measured": measured_frac(traffic, avg_launch_s)},
         "range_check_bad_cells": bad,
         "volume_rel_drift": abs(vol1 - vol0) / max(abs(vol0), 1e-300),
     }
@@ -316,16 +315,16 @@ def ensemble_leg(steps, warmup, nmembers):
     avg = ms * 1e-3 / launches
     bpc = BYTES_PER_CELL["fp32"]
     achieved = bpc * subs * cells / avg / 1e9
+    traffic = traffic_from_profiles("ensemble_fp32")
     res = {"value": wet * substeps / (ms * 1e-3), "unit": "wet-cell steps/s",
            "members": nmem, "wet_cells": wet, "array_cells": cells, "steps": steps,
            "ms_per_step": ms / steps, "avg_launch_us": avg * 1e6, "substeps_per_launch": subs,
            "launch": {"rows_per_wave": tune["rows_per_wave"], "waves_per_xcd": tune["waves_per_xcd"]},
            "warmup_steps_run": warm_steps, "warmup_s": warm_s,
            "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                        "frac": achieved / PEAK_HBM_GBS, "traffic": traffic_from_profiles("ensemble_fp32"),
+                        "frac": achieved / PEAK_HBM_GBS, "traffic": traffic,
                         "bytes_per_cell_substep": bpc, "cells_per_launch": cells, "substeps_per_launch": subs,
-                        "frac_with_frozen_rhs": BYTES_PER_CELL_WITH_RHS["fp32"] * subs * cells / avg / 1e9
-                        / PEAK_HBM_GBS},
+                        "frac_measured": measured_frac(traffic, avg)},
            "range_check_bad_cells": bad, "max_volume_rel_drift": drift}
     log(f"ensemble fp32: {ms:.1f} ms for {steps} steps ({avg * 1e6:.1f} us/launch), "
         f"{res['value']:.3e} wet-cell steps/s, {achieved:.0f} GB/s")

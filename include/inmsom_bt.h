@@ -271,7 +271,8 @@ int inmsom_bt_ens_set_state(inmsom_bt_ens *ens, int member, const double *u, con
 int inmsom_bt_ens_get_state(inmsom_bt_ens *ens, int member, double *u, double *up, double *v,
                             double *vp, double *ssh, double *sshp);
 /* launch shape: output rows per wave (0 = default) and waves per XCD of
- * the persistent grid (0 = default); results do not depend on it */
+ * the persistent grid (0 = default; both 0: tiles where a small ensemble
+ * takes them); results do not depend on it */
 int inmsom_bt_ens_set_launch(inmsom_bt_ens *ens, int rows_per_wave, int waves_per_xcd);
 /* substeps per launch, as inmsom_bt_set_substeps_per_launch (0 = by mode) */
 int inmsom_bt_ens_set_substeps_per_launch(inmsom_bt_ens *ens, int substeps);
