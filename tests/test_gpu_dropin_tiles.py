@@ -14,12 +14,14 @@ pytestmark = pytest.mark.gpu
 ACC = ("ubrtr_i", "vbrtr_i", "ssh4gradx", "ssh4grady")
 
 
-# columns around the 60-column tiles, rows around the 4- and 8-row ones; the
-# smallest basin; 660 x 640 is the march's without the biharmonic term
+# columns around the 60-column tiles, rows around those of 4 and 8 rows written;
+# the smallest basin; 333 x 301 has tiles of 12 rows, the smaller ones of 8; 660 x
+# 640 is the march's without the biharmonic term
 @pytest.mark.parametrize("ksw4", [0, 1])
 @pytest.mark.parametrize("shape,metrics,nstep", [((7, 5), "uniform", 2), ((56, 28), "uniform", 1),
                                                  ((57, 29), "stretched", 3), ((117, 61), "stretched", 2),
-                                                 ((285, 159), "uniform", 2), ((660, 640), "uniform", 1)])
+                                                 ((285, 159), "uniform", 2), ((333, 301), "stretched", 1),
+                                                 ((660, 640), "uniform", 1)])
 def test_tiles_equal_stage_by_stage(shape, metrics, nstep, ksw4):
     print(f"drop-in tiles {shape} {metrics} nstep={nstep} ksw4={ksw4}", flush=True)
     b = randomize_state(make_basin(*shape, seed=31, sigma=min(5.0, 0.2 * min(shape)), metrics=metrics, lvisc_4=1e-3,
